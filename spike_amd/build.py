@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import os
 import subprocess
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -28,12 +29,29 @@ def run(cmd, cwd=None):
     return r
 
 
+# Translation units: (source, extra flags).  The persistent kernels' many instances make up
+# most of the compile time, so they are split over parts that compile side by side.
+FUSED_PARTS = 7
+UNITS = ([("fused_part.hip", [f"-DSPK_FUSED_PART={k}"]) for k in range(FUSED_PARTS)]
+         + [("spike_hip.hip", []), ("mlp.hip", [])])
+
+
 def build_hip_library() -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
-    srcs = [os.path.join(HERE, "csrc", f) for f in ("spike_hip.hip", "mlp.hip")]
+    obj_dir = os.path.join(LIB_DIR, "obj")
+    os.makedirs(obj_dir, exist_ok=True)
+
+    def unit(k):
+        src, flags = UNITS[k]
+        obj = os.path.join(obj_dir, f"{k}_{src.split('.')[0]}.o")
+        run([HIPCC, *HIP_FLAGS, *flags, "-c", os.path.join(HERE, "csrc", src), "-o", obj])
+        return obj
+
+    with ThreadPoolExecutor(max(1, min(8, os.cpu_count() or 1))) as pool:
+        objs = list(pool.map(unit, range(len(UNITS))))
     out = os.path.join(LIB_DIR, "libspike_hip.so")
     tmp = out + ".tmp"
-    run([HIPCC, *HIP_FLAGS, "-shared", "-o", tmp, *srcs])
+    run([HIPCC, *HIP_FLAGS, "-shared", "-o", tmp, *objs])
     os.replace(tmp, out)
     return out
 

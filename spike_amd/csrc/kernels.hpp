@@ -212,7 +212,7 @@ __device__ __forceinline__ void wave_append(bool pred, uint32_t id, uint32_t* __
 // ---------------------------------------------------------------------------------
 // group bookkeeping: clear the G per-sub-step counts of a list slot, record its time
 
-__global__ void k_begin_group(int* __restrict__ counts, int G, float* __restrict__ slot_time,
+static __global__ void k_begin_group(int* __restrict__ counts, int G, float* __restrict__ slot_time,
                               int* __restrict__ slot_tidx, int slot, float t, int tidx) {
   const int i = threadIdx.x;
   for (int g = i; g < G; g += blockDim.x) counts[g] = 0;
@@ -476,7 +476,7 @@ __device__ __forceinline__ float poisson_unit(const PoissonArgs& a, int i) {
   return last;
 }
 
-__global__ __launch_bounds__(256) void k_poisson(PoissonArgs a) {
+static __global__ __launch_bounds__(256) void k_poisson(PoissonArgs a) {
   poisson_unit(a, (int)(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
@@ -504,7 +504,7 @@ struct GeneratorArgs {
   uint32_t* rate;          // [Nin] spike counts of a rate monitor, or nullptr
 };
 
-__global__ __launch_bounds__(256) void k_generator(GeneratorArgs a) {
+static __global__ __launch_bounds__(256) void k_generator(GeneratorArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool active = i < a.Nin;
   if (active) {
@@ -566,7 +566,7 @@ struct PropArgs {
 // loads in flight: each lane's iterations are chains of dependent loads.
 constexpr int kRowWaves = 8;
 
-__global__ __launch_bounds__(256) void k_propagate(PropArgs a) {
+static __global__ __launch_bounds__(256) void k_propagate(PropArgs a) {
   const int lane = (int)__lane_id();
   const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
   const int nwaves = (int)((gridDim.x * blockDim.x) / kWave);
@@ -693,7 +693,7 @@ __device__ __forceinline__ void stdp_wd_one(const StdpArgs& a, int64_t j) {
   tstore(a.tr, 1, j, xpost);
 }
 
-__global__ __launch_bounds__(256) void k_stdp_wd(StdpArgs a) {
+static __global__ __launch_bounds__(256) void k_stdp_wd(StdpArgs a) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j < a.P) stdp_wd_one(a, j);
 }
@@ -777,7 +777,7 @@ __device__ __forceinline__ void wd_post_unit(const WdEventArgs& a, int v, bool a
   wave_push(listed, (uint32_t)v, a.act + a.N + a.Nin, a.cnt + 2 * a.par + 1, a.N);
 }
 
-__global__ __launch_bounds__(256) void k_wd_neurons(WdEventArgs a) {
+static __global__ __launch_bounds__(256) void k_wd_neurons(WdEventArgs a) {
   const int U = a.N + a.Nin;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool pre = i < U;
@@ -787,7 +787,7 @@ __global__ __launch_bounds__(256) void k_wd_neurons(WdEventArgs a) {
   wd_post_unit(a, v, post, post ? a.last_n[v] : 0.0f);
 }
 
-__global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
+static __global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
   const int lane = (int)__lane_id();
   const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
   const int nwaves = (int)((gridDim.x * blockDim.x) / kWave);
@@ -963,7 +963,7 @@ __global__ __launch_bounds__(256) void k_deliver(DeliverArgs a) {
 }
 
 // Marks the rule's synapses in a bitmask over CSR positions (k_deliver's source side).
-__global__ __launch_bounds__(256) void k_mark_rule(const int64_t* __restrict__ pos, int64_t P,
+static __global__ __launch_bounds__(256) void k_mark_rule(const int64_t* __restrict__ pos, int64_t P,
                                                    uint32_t* __restrict__ mask) {
   for (int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; j < P; j += (int64_t)gridDim.x * blockDim.x) {
     const int64_t s = pos[j];
@@ -983,7 +983,7 @@ struct TraceCopyArgs {
   int to_neurons;
 };
 
-__global__ __launch_bounds__(256) void k_trace_copy(TraceCopyArgs a) {
+static __global__ __launch_bounds__(256) void k_trace_copy(TraceCopyArgs a) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= a.P) return;
   const int u = a.pre[j];
@@ -1034,7 +1034,7 @@ __device__ __forceinline__ void stdp_vogels_one(const StdpArgs& a, int64_t j) {
   tstore(a.tr, 1, j, xpost);
 }
 
-__global__ __launch_bounds__(256) void k_stdp_vogels(StdpArgs a) {
+static __global__ __launch_bounds__(256) void k_stdp_vogels(StdpArgs a) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j < a.P) stdp_vogels_one(a, j);
 }
@@ -1070,7 +1070,7 @@ __device__ __forceinline__ void stdp_evans_one(const StdpArgs& a, int64_t j) {
   tstore(a.tr, 1, j, D);
 }
 
-__global__ __launch_bounds__(256) void k_stdp_evans(StdpArgs a) {
+static __global__ __launch_bounds__(256) void k_stdp_evans(StdpArgs a) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j < a.P) stdp_evans_one(a, j);
 }
@@ -1108,7 +1108,7 @@ __device__ __forceinline__ void stdp_custom_one(const StdpArgs& a, int64_t j) {
   tstore(a.tr, 1, j, xpost);
 }
 
-__global__ __launch_bounds__(256) void k_stdp_custom(StdpArgs a) {
+static __global__ __launch_bounds__(256) void k_stdp_custom(StdpArgs a) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j < a.P) stdp_custom_one(a, j);
 }
@@ -1128,7 +1128,7 @@ struct WeightNormArgs {
   int N;
 };
 
-__global__ __launch_bounds__(256) void k_weightnorm(WeightNormArgs a) {
+static __global__ __launch_bounds__(256) void k_weightnorm(WeightNormArgs a) {
   const int v = blockIdx.x * blockDim.x + threadIdx.x;
   if (v >= a.N || !a.in_set[v]) return;
   const int64_t e0 = a.ptr[v], e1 = a.ptr[v + 1];
@@ -1165,7 +1165,7 @@ struct CollectArgs {
   float dt;
 };
 
-__global__ __launch_bounds__(256) void k_collect(CollectArgs a) {
+static __global__ __launch_bounds__(256) void k_collect(CollectArgs a) {
   // blockIdx.y = slot offset * G + g; blockIdx.x strides over the list entries
   const int sg = blockIdx.y;
   const int s = a.slot0 + sg / a.G;
@@ -1211,7 +1211,7 @@ struct StatsOut {
 
 constexpr int kStatsBlock = 1024;
 
-__device__ double block_sum_f64(double v, double* sh) {
+static __device__ double block_sum_f64(double v, double* sh) {
   sh[threadIdx.x] = v;
   __syncthreads();
   for (int off = kStatsBlock / 2; off > 0; off >>= 1) {
@@ -1223,7 +1223,7 @@ __device__ double block_sum_f64(double v, double* sh) {
   return r;
 }
 
-__global__ __launch_bounds__(kStatsBlock) void k_stats_reduce(StatsArgs st, int N, int64_t steps, float dt,
+static __global__ __launch_bounds__(kStatsBlock) void k_stats_reduce(StatsArgs st, int N, int64_t steps, float dt,
                                                               StatsOut* out) {
   __shared__ double sh[kStatsBlock];
   double spikes = 0.0, cv = 0.0, ncv = 0.0;

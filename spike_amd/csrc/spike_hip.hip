@@ -17,6 +17,7 @@
 #include "../../include/spike_hip.h"
 #include "kernels.hpp"
 #include "fused.hpp"
+#include "fused_table.hpp"
 #include "gen.hpp"
 
 #pragma clang fp contract(off)
@@ -972,15 +973,9 @@ const void* fused_kernel(const spk_network* n, bool plastic) {
   // Brunel-type networks (voltage synapses, compact records): kernels holding only their
   // delivery form
   if (!plastic && n->kind == SPK_SYN_VOLTAGE && l1 && n->compact && n->rules.empty())
-    return n->lseg_U > 0 ? (const void*)spk::k_fused<0, true, false, spk::kDeliverLdsTable>
-                         : (const void*)spk::k_fused<0, true, false, spk::kDeliverCompact>;
-#define SPK_FUSED_PICK(K)                                                                  \
-  (plastic ? (l1 ? (const void*)spk::k_fused<K, true, true> : (const void*)spk::k_fused<K, false, true>) \
-           : (l1 ? (const void*)spk::k_fused<K, true, false> : (const void*)spk::k_fused<K, false, false>))
-  if (n->kind == SPK_SYN_VOLTAGE) return SPK_FUSED_PICK(0);
-  if (n->kind == SPK_SYN_CONDUCTANCE) return SPK_FUSED_PICK(1);
-  return SPK_FUSED_PICK(2);
-#undef SPK_FUSED_PICK
+    return n->lseg_U > 0 ? spk::fused_kernel_lds_table() : spk::fused_kernel_compact();
+  const spk::FusedKernels k = spk::fused_kernels(n->kind, l1);
+  return plastic ? k.run_plastic : k.run;
 }
 
 // Dynamic LDS a persistent workgroup may take: the per-workgroup limit less the static LDS
@@ -2931,35 +2926,20 @@ void batch_drop_graph(spk_batch* b) {
   b->g_fn = nullptr;
 }
 
-template <int BS>
-const void* batch_kernel_bs(const spk_batch* b) {
-  if (b->kind == SPK_SYN_VOLTAGE)
-    return b->l1 ? (const void*)spk::k_fused_batch<0, true, false, BS> : (const void*)spk::k_fused_batch<0, false, false, BS>;
-  if (b->kind == SPK_SYN_CONDUCTANCE)
-    return b->l1 ? (const void*)spk::k_fused_batch<1, true, false, BS> : (const void*)spk::k_fused_batch<1, false, false, BS>;
-  return b->l1 ? (const void*)spk::k_fused_batch<2, true, false, BS> : (const void*)spk::k_fused_batch<2, false, false, BS>;
-}
-
 // Batches of Brunel-type networks (voltage synapses, one label, compact records) run
 // kernels without the full-record delivery: compact only when no network keeps its table in
 // LDS, else both compact forms.
-template <int BS>
-const void* batch_kernel_compact(const spk_batch* b, bool tables) {
-  return tables ? (const void*)spk::k_fused_batch<0, true, false, BS, spk::kDeliverCompactAny>
-                : (const void*)spk::k_fused_batch<0, true, false, BS, spk::kDeliverCompact>;
-}
-
 const void* batch_kernel(const spk_batch* b, int bs) {
+  const bool small = bs == spk::kBatchSmallBlock;
   bool compact = b->kind == SPK_SYN_VOLTAGE && b->l1, tables = false;
   for (auto* n : b->nets) {
     compact = compact && n->compact && n->rules.empty();
     tables = tables || n->lseg_U > 0;
   }
-  tables = tables && bs != spk::kBatchSmallBlock && b->lds_tables;
-  if (compact)
-    return bs == spk::kBatchSmallBlock ? batch_kernel_compact<spk::kBatchSmallBlock>(b, false)
-                                       : batch_kernel_compact<spk::kFusedBlock>(b, tables);
-  return bs == spk::kBatchSmallBlock ? batch_kernel_bs<spk::kBatchSmallBlock>(b) : batch_kernel_bs<spk::kFusedBlock>(b);
+  tables = tables && !small && b->lds_tables;
+  if (compact) return spk::batch_kernel_compact(small, tables);
+  const spk::FusedKernels k = spk::fused_kernels(b->kind, b->l1);
+  return small ? k.batch_small : k.batch;
 }
 
 }  // namespace
