@@ -179,6 +179,7 @@ struct FusedLayout {
 constexpr int kHeadWords = 12;         // words of a source block fetched in the first trip
 constexpr int kEntCap = 4096;          // spike entries staged in LDS per delivery round
 constexpr int kQuad = 4;               // lanes cooperating on one spike's row segment
+constexpr int kStatBins = 64;          // histogram bins of a group (G <= 64, bins of >= 1 step) and more; a wavefront
 constexpr int kSpikesPerQuad = 4;      // spikes a quad handles with its loads in flight together
 
 __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~(size_t)15; }
@@ -203,13 +204,13 @@ __host__ __device__ inline FusedLayout fused_layout(int BL, int L, int W, int G,
   f.scan = o;    o = align16(o + (size_t)(P + 1) * 4);
   f.ent = o;     o = align16(o + (size_t)kEntCap * 4);
   f.counter = o; o = align16(o + 4 * 4);
-  // window statistics of the owned neurons, and spikes per sub-step of the group
+  // window statistics of the owned neurons, and the population histogram's open bins
   f.st_cnt = o;  o = align16(o + (size_t)nown * 4);
   f.st_nisi = o; o = align16(o + (size_t)nown * 4);
   f.st_prev = o; o = align16(o + (size_t)nown * 4);
   f.st_s1 = o;   o = align16(o + (size_t)nown * 8);
   f.st_s2 = o;   o = align16(o + (size_t)nown * 8);
-  f.st_g = o;    o = align16(o + 64 * 4);
+  f.st_g = o;    o = align16(o + kStatBins * 4);
   f.cdf = o;     o = align16(o + (size_t)kMaxExtTable * 4);   // external count thresholds
   f.guide = o;   o = align16(o + 256);                          // guide table of the thresholds
   f.lseg = o;    o = align16(o + (segU ? (size_t)(segU + 1) * 2 : 0));   // local starts
@@ -1095,7 +1096,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
       sst_s1[i] = a.st.s1[nlo + i];
       sst_s2[i] = a.st.s2[nlo + i];
     }
-    if (tid < 64) sst_g[tid] = 0u;
+    if (tid < kStatBins) sst_g[tid] = 0u;
   }
   // LDS-resident delivery table: this partition's segment of every source row, concatenated
   // in source order (so start[u + 1] ends segment u).  Thread t takes a run of consecutive
@@ -1167,6 +1168,19 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   const bool in_ring = DM != kDeliverLdsTable && a.cring && a.nown_max > kWave && a.lseg_U == 0;
   // one wavefront holds every unit of the partition (nown_waves <= kWave)
   const bool early = !PLASTIC && a.xquad && a.early && BS > kWave;
+  // population histogram of the window statistics: kStatBins consecutive bins, bin b in slot
+  // b % kStatBins, collected in LDS and added to the global histogram when the next group's
+  // bins would not fit (Brunel10K at 10-step bins: every 42 groups).  Adding every group's
+  // counts at once puts 256 workgroups' atomics on the same two words in front of each
+  // workgroup's polling loads, which wait for them: 2.8 us per group, 5.8 instead of 4.0 ms
+  // per simulated second.
+  int hbase = 0;
+  if (a.st.on) {
+    float t0;
+    int ti;
+    group_time(a, 0, t0, ti);
+    hbase = max(0, ti - (int)a.st.t0) / a.st.bin;
+  }
   // spike counters of the exchange list, one per group parity (the other parity's is
   // cleared while the group runs)
   if (tid < 2) scounter[tid] = 0;
@@ -1285,6 +1299,23 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     __syncthreads();
     clk.lap(a, 0);
     // -- B2. LIF recurrence, one lane per neuron (LIFSpikingNeurons.cu:115-190) -------
+    // window statistics of this lane's spikes of the group, in time order (LDS only)
+    auto window_stats = [&](unsigned long long mm) {
+      unsigned int c0 = sst_cnt[tid], c1 = sst_nisi[tid];
+      float pv = sst_prev[tid];
+      double d1 = sst_s1[tid], d2 = sst_s2[tid];
+      while (mm) {
+        const int g = __ffsll((unsigned long long)mm) - 1;
+        mm &= mm - 1ull;
+        const int64_t step = (int64_t)tidx + g;
+        stats_spike(a.st, step, t + (float)g * a.dt, c0, c1, pv, d1, d2);
+        if (step >= a.st.t0 && step < a.st.t0 + a.st.nsteps)
+          atomicAdd(&sst_g[((tidx + g - (int)a.st.t0) / a.st.bin) & (kStatBins - 1)], 1u);
+      }
+      sst_cnt[tid] = c0; sst_nisi[tid] = c1; sst_prev[tid] = pv;
+      sst_s1[tid] = d1; sst_s2[tid] = d2;
+    };
+    unsigned long long smask_w = 0ull;
     if (early && tid >= kWave) {
       // the next group's random draws on the other wavefronts while wavefront 0 integrates
       if ((s + 1) % a.dahead == 0 && s + 1 < a.ngroups)
@@ -1401,21 +1432,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
           }
         }
         if (a.rate_n != nullptr && smask) a.rate_n[gi] += (uint32_t)__popcll(smask);
-        if (a.st.on && smask) {
-          // window statistics of this neuron's spikes, in time order
-          unsigned int c0 = sst_cnt[tid], c1 = sst_nisi[tid];
-          float pv = sst_prev[tid];
-          double d1 = sst_s1[tid], d2 = sst_s2[tid];
-          unsigned long long mm = smask;
-          while (mm) {
-            const int g = __ffsll((unsigned long long)mm) - 1;
-            mm &= mm - 1ull;
-            stats_spike(a.st, (int64_t)tidx + g, t + (float)g * a.dt, c0, c1, pv, d1, d2);
-            atomicAdd(&sst_g[g], 1u);
-          }
-          sst_cnt[tid] = c0; sst_nisi[tid] = c1; sst_prev[tid] = pv;
-          sst_s1[tid] = d1; sst_s2[tid] = d2;
-        }
+        if (!early && a.st.on && smask) window_stats(smask);
       }
       if (early) {
         // wavefront 0 holds the partition: its spikes' list positions by a wavefront prefix
@@ -1430,6 +1447,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         unsigned long long* xl = a.xlist64 + ((size_t)par * a.P + p) * a.xstride;
         const uint32_t tag = a.xtag_base + (uint32_t)s + 1u;
         st_spk += (unsigned long long)c;
+        smask_w = smask;
         unsigned long long mm = smask;
         while (mm) {
           const int g = __ffsll((unsigned long long)mm) - 1;
@@ -1462,13 +1480,19 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
       }
     }
     __syncthreads();
-    if (a.st.on && tid < G) {
-      // population spikes of this partition per sub-step into the window's bins
-      const unsigned int c = sst_g[tid];
-      const int64_t step = (int64_t)tidx + tid;
-      if (c && step >= a.st.t0 && step < a.st.t0 + a.st.nsteps)
-        atomicAdd(a.st.hist + (step - a.st.t0) / a.st.bin, c);
-      sst_g[tid] = 0u;
+    if (a.st.on && tid < kWave) {
+      // (early form: after the publication, while the lists travel; smask_w is wavefront 0's)
+      if (early && smask_w) window_stats(smask_w);
+      float tn;
+      int tin;
+      group_time(a, s + 1, tn, tin);
+      const int rel = tin - (int)a.st.t0;
+      if (s + 1 == a.ngroups || max(0, rel + G - 1) / a.st.bin - hbase >= kStatBins) {
+        const unsigned int c = sst_g[tid];
+        if (c) atomicAdd(a.st.hist + hbase + ((tid - hbase) & (kStatBins - 1)), c);
+        sst_g[tid] = 0u;
+        hbase = max(0, rel) / a.st.bin;
+      }
     }
     clk.lap(a, 1);
     // -- C. publish: {count, entries} block, and state other workgroups may read ------

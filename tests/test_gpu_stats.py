@@ -135,3 +135,26 @@ def test_fp32_plastic_weight_histogram_within_2pc_of_fp64():
     assert abs(wg.mean() - wo.mean()) <= 0.02 * wo.mean()
     assert abs(wg.std() - wo.std()) <= 0.02 * wo.std()
     assert l1 <= 0.02
+
+
+@pytest.mark.parametrize("partitions", [0, 4])
+@pytest.mark.parametrize("delay,bin_steps,window", [(64, 1, 1500), (15, 1, 3000), (15, 3, 997), (1, 7, 3000),
+                                                    (20, 100, 3000), (15, 4000, 3000)])
+def test_population_bins_at_the_edges_of_the_lds_histogram(partitions, delay, bin_steps, window):
+    """The open bins of the population histogram are kept in 64 LDS slots: bins of one step
+    with 64-step groups (every slot used by one group), bins that no group ends on, one bin
+    for the whole window; one and several wavefronts of neurons per partition; two runs."""
+    d = builders.brunel(n_exc=320, n_inh=80, seed=21, delay_steps=delay, monitors=(0,))
+    G = d.timestep_grouping()
+    n1, n2 = 700 // G, 2300 // G
+    net = abi.Network(d, partitions=partitions)
+    net.stats_begin(bin_steps, window)
+    net.run(0.0, n1)
+    net.run(float(d.group_time(0.0, n1)), n2)
+    s = net.stats()
+    ids, times = net.take_spikes(0)
+    steps = min((n1 + n2) * G, window)
+    e = expected_stats(ids, times, d.n_neurons, d.dt, 0, steps, bin_steps)
+    assert s.steps == steps and s.bins == e["bins"] and s.spikes == e["spikes"] > 0
+    assert abs(s.synchrony - e["sync"]) <= 1e-9 * max(e["sync"], 1e-3)
+    assert abs(s.isi_cv - e["cv"]) <= 1e-9 * e["cv"]
