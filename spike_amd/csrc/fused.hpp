@@ -1223,6 +1223,11 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     unsigned long long* imask = simask + (size_t)dslot * a.iown_max;
     const int b0 = tidx % bits;
     const int slot0 = tidx % BL;
+    // the lane's LDS addresses are computed in every group: hoisted out of the group loop they
+    // would stay live across the delivery, which has no registers to spare (an empty asm, no
+    // instruction)
+    int lt = tid;
+    asm volatile("" : "+v"(lt));
     // -- A. Poisson inputs: append this group's spikes, update histories ------------
     for (int i = tid; i < iown; i += BS) {
       const unsigned long long m = imask[i];
@@ -1301,9 +1306,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     // -- B2. LIF recurrence, one lane per neuron (LIFSpikingNeurons.cu:115-190) -------
     // window statistics of this lane's spikes of the group, in time order (LDS only)
     auto window_stats = [&](unsigned long long mm) {
-      unsigned int c0 = sst_cnt[tid], c1 = sst_nisi[tid];
-      float pv = sst_prev[tid];
-      double d1 = sst_s1[tid], d2 = sst_s2[tid];
+      unsigned int c0 = sst_cnt[lt], c1 = sst_nisi[lt];
+      float pv = sst_prev[lt];
+      double d1 = sst_s1[lt], d2 = sst_s2[lt];
       while (mm) {
         const int g = __ffsll((unsigned long long)mm) - 1;
         mm &= mm - 1ull;
@@ -1312,8 +1317,8 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         if (step >= a.st.t0 && step < a.st.t0 + a.st.nsteps)
           atomicAdd(&sst_g[((tidx + g - (int)a.st.t0) / a.st.bin) & (kStatBins - 1)], 1u);
       }
-      sst_cnt[tid] = c0; sst_nisi[tid] = c1; sst_prev[tid] = pv;
-      sst_s1[tid] = d1; sst_s2[tid] = d2;
+      sst_cnt[lt] = c0; sst_nisi[lt] = c1; sst_prev[lt] = pv;
+      sst_s1[lt] = d1; sst_s2[lt] = d2;
     };
     unsigned long long smask_w = 0ull;
     if (early && tid >= kWave) {
@@ -1332,7 +1337,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         auto take = [&](int g) -> float {
           int sl = slot0 + g;
           if (sl >= BL) sl -= BL;
-          uint32_t* w = scring + (size_t)sl * nown + tid;
+          uint32_t* w = scring + (size_t)sl * nown + lt;
           const float v = __uint_as_float(*w);
           *w = 0u;
           return v;
@@ -1357,7 +1362,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
             for (int x = 0; x < kPrefetch; ++x) cin[x] = (x < G) ? take(x) : 0.0f;
             SPK_LIF_SWITCH(cin)
           } else {
-            const float* in = sinp + tid * G;
+            const float* in = sinp + lt * G;
             SPK_LIF_SWITCH(in)
           }
 #undef SPK_LIF_SWITCH
@@ -1370,7 +1375,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
             float dvs[kPrefetch];
 #pragma unroll
             for (int x = 0; x < kPrefetch; ++x)
-              dvs[x] = (x < gn) ? (in_ring ? take(g0 + x) : sinp[tid * G + g0 + x]) : 0.0f;
+              dvs[x] = (x < gn) ? (in_ring ? take(g0 + x) : sinp[lt * G + g0 + x]) : 0.0f;
             const float tref = a.tref, dt = a.dt, tg0 = t;
             unsigned long long mk = 0ull;
 #pragma unroll
@@ -1394,7 +1399,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
 #pragma unroll
               for (int l = 0; l < kMaxLabels; ++l) {
                 if (l < L) {
-                  const float in = sinp[((size_t)tid * G + g) * L + l];
+                  const float in = sinp[((size_t)lt * G + g) * L + l];
                   gl[l] = a.decay_g[l] * gl[l] + in;
                   total += (KIND == 1) ? gl[l] * (a.erev[l] - V) : gl[l];
                 }
@@ -1424,7 +1429,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
             const int n = min(min(32 - off, G - done), bits - pos);
             const uint32_t ones = n == 32 ? 0xFFFFFFFFu : ((1u << n) - 1u);
             const uint32_t sp = (uint32_t)(smask >> done) & ones;
-            uint32_t* wp = shist + (pos >> 5) * nown + tid;
+            uint32_t* wp = shist + (pos >> 5) * nown + lt;
             *wp = (*wp & ~(ones << off)) | (sp << off);
             done += n;
             pos += n;
@@ -1453,7 +1458,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
           const int g = __ffsll((unsigned long long)mm) - 1;
           mm &= mm - 1ull;
           if (pos < a.xcap) {
-            const uint32_t e = ((uint32_t)g << 24) | (uint32_t)(nlo + tid);
+            const uint32_t e = ((uint32_t)g << 24) | (uint32_t)(nlo + lt);
             sxbuf[pos] = e;
             xstore64(xl + 1 + pos, e, tag);
           }
@@ -1474,7 +1479,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         while (mm) {
           const int g = __ffsll((unsigned long long)mm) - 1;
           mm &= mm - 1ull;
-          if (pos < a.xcap) sxbuf[pos] = ((uint32_t)g << 24) | (uint32_t)(nlo + tid);
+          if (pos < a.xcap) sxbuf[pos] = ((uint32_t)g << 24) | (uint32_t)(nlo + lt);
           ++pos;
         }
       }
