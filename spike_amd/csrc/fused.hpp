@@ -11,8 +11,8 @@
 //      spikes are compacted into the workgroup's exchange list (id | g << 24);
 //   2. the list is published as tagged 64-bit words in the workgroup's exchange block --
 //      by the LIF wavefront itself when one wavefront holds the partition -- and every
-//      workgroup polls the blocks it needs (no grid barrier); with plasticity a grid
-//      barrier orders the phases instead;
+//      workgroup polls the blocks it needs (no grid barrier); with plasticity per synapse a
+//      grid barrier orders the phases instead;
 //   3. plasticity of the plastic synapses whose postsynaptic neuron the workgroup owns
 //      (they are the only weights its own delivery reads);
 //   4. delivery: every spike's row segment that targets this partition
@@ -59,7 +59,32 @@ struct FusedRule {
   int kind;
 };
 
+// How a persistent kernel applies plasticity: not at all, per synapse behind a grid barrier
+// (any rules), or driven by spikes (one weight-dependent rule; no grid barrier).
+enum { kRulesOff = 0, kRulesDense = 1, kRulesEvents = 2 };
+
+// The weight-dependent rule driven by spikes (kRulesEvents; the per-phase form of kernels.hpp,
+// k_wd_neurons and k_wd_events, inside the group loop).  Every workgroup keeps the presynaptic
+// trace of every source the rule may have in LDS and advances all of them each group: a
+// source's trace depends only on its own spikes, which every workgroup receives through the
+// exchange, so no workgroup reads another's state and no grid barrier is needed.  Weights are
+// touched only by the workgroup that owns their target.  Bound by the exchange's latency: 6000
+// neurons x 500 synapses (3.1e6, delays from one step) take 5.1 us per group; per synapse, with
+// the barrier's cache write-backs, 51 us.
+struct EventRule {
+  Traces tr;               // stored traces per neuron: a [sources], b [N]
+  Weights wts;
+  const float* tab;        // wd_weight's table, `ntab` floats
+  const uint32_t* mask;    // bit k: CSR position k belongs to the rule
+  const int64_t* post_ptr; // the rule's synapses onto neuron v: positions and sources
+  const uint32_t* post_pos;
+  const int32_t* post_pre;
+  int sources;             // N, or N + Nin when inputs have rule synapses
+  int ntab, nearest;
+};
+
 struct FusedArgs {
+  EventRule ev;            // kRulesEvents only
   // partitions: neurons [nlo[p], nlo[p+1]), inputs [ilo[p], ilo[p+1])
   const int* nlo;
   const int* ilo;
@@ -173,7 +198,7 @@ struct PhaseClock {
 // spike masks take 64-bit LDS atomics, which need 8-byte aligned addresses).
 struct FusedLayout {
   size_t ring, hist, ext, imask, inp, xbuf, head, scan, ent, counter, st_cnt, st_nisi, st_prev, st_s1,
-      st_s2, st_g, cdf, guide, lseg, lrec, total;
+      st_s2, st_g, cdf, guide, lseg, lrec, ev_x, ev_bits, ev_xq, ev_qg, ev_list, ev_tab, total;
 };
 
 constexpr int kHeadWords = 12;         // words of a source block fetched in the first trip
@@ -189,7 +214,7 @@ __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~(size_t
 // table is read from global memory).
 __host__ __device__ inline FusedLayout fused_layout(int BL, int L, int W, int G, int nown, int iown,
                                                     int xcap, int P, int segU = 0, int lrec = 0, int cring = 0,
-                                                    int dahead = 1) {
+                                                    int dahead = 1, int ev_src = 0) {
   FusedLayout f;
   size_t o = 0;
   f.ring = o;    o = align16(o + (size_t)BL * nown * L * (cring ? 4 : 8));
@@ -215,14 +240,22 @@ __host__ __device__ inline FusedLayout fused_layout(int BL, int L, int W, int G,
   f.guide = o;   o = align16(o + 256);                          // guide table of the thresholds
   f.lseg = o;    o = align16(o + (segU ? (size_t)(segU + 1) * 2 : 0));   // local starts
   f.lrec = o;    o = align16(o + (size_t)lrec * 2);             // this partition's targets
+  // kRulesEvents: presynaptic traces of `ev_src` sources and a bit per source that spiked in
+  // the group, traces and spike steps of the owned neurons, the spiking ones, the rule's table
+  f.ev_x = o;    o = align16(o + (size_t)ev_src * 4);
+  f.ev_bits = o; o = align16(o + (size_t)(ev_src + 31) / 32 * 4);
+  f.ev_xq = o;   o = align16(o + (ev_src ? (size_t)nown * 4 : 0));
+  f.ev_qg = o;   o = align16(o + (ev_src ? (size_t)nown * 4 : 0));
+  f.ev_list = o; o = align16(o + (ev_src ? (size_t)nown * 4 : 0));
+  f.ev_tab = o;  o = align16(o + (ev_src ? (size_t)(5 + 4 * (G + 1)) * 4 : 0));
   f.total = o;
   return f;
 }
 
 __host__ __device__ inline size_t fused_lds_bytes(int BL, int L, int W, int G, int nown, int iown,
                                                   int xcap, int P, int segU = 0, int lrec = 0, int cring = 0,
-                                                  int dahead = 1) {
-  return fused_layout(BL, L, W, G, nown, iown, xcap, P, segU, lrec, cring, dahead).total;
+                                                  int dahead = 1, int ev_src = 0) {
+  return fused_layout(BL, L, W, G, nown, iown, xcap, P, segU, lrec, cring, dahead, ev_src).total;
 }
 
 __host__ __device__ inline int fused_xstride(int xcap) { return ((1 + xcap + 7) / 8) * 8; }
@@ -713,13 +746,119 @@ constexpr int kQuadEnt = 8;   // entries of one source a quad stages in LDS at a
 // memory (a kernel holding only the form it runs keeps its registers for it).
 enum { kDeliverAny = 0, kDeliverLdsTable = 1, kDeliverCompact = 2, kDeliverCompactAny = 3 };
 
+// LDS state of the spike-driven rule (kRulesEvents) and the group's start time.
+struct EventLds {
+  float* x;              // presynaptic traces, decayed for this group
+  uint32_t* bits;        // sources that spiked in the group
+  float* xq;             // postsynaptic traces of the owned neurons
+  int* qg;               // steps of their last spikes within the group (negative: before it)
+  int* list;             // owned neurons that spiked
+  float* tab;
+  float t;
+};
+
+// A source's spike at sub-step g: its step in the group as the rule reads it (wd_pre_step of
+// its last spike time), or -1 for sources outside the rule.  Lane q = 0 of the quad raises the
+// source's trace and marks it; every lane returns the raised trace.
+__device__ __forceinline__ int event_source(const FusedArgs& a, const EventLds& ev, uint32_t id, int g, int q,
+                                            float& x) {
+  x = 0.0f;
+  if ((int)id >= a.ev.sources) return -1;
+  const int pg = wd_pre_step(ev.t + (float)g * a.dt, ev.t, a.dt, a.G);
+  if (pg < 0) return -1;
+  const float* Ep = ev.tab + 5 + (a.G + 1);
+  const float add = ev.tab[1] * Ep[a.G - pg];
+  x = a.ev.nearest ? add : ev.x[id] + add;
+  if (q == 0) {
+    ev.x[id] = x;
+    atomicOr(&ev.bits[id >> 5], 1u << (id & 31));
+  }
+  return pg;
+}
+
+// deliver_quad with the rule's source side folded in: a synapse of the rule (a bit of the
+// mask) is updated and delivered with its new weight (the reference applies plasticity before
+// propagation, SpikingModel.cpp:228-233).  A source spikes at most once per group here, so
+// its row is walked once.
+template <bool PER_SYN_SCALE>
+__device__ __forceinline__ void deliver_quad_events(const FusedArgs& a, const EventLds& ev, const uint32_t* ents,
+                                                    int n, int q, int p, int slot0, int B, int nownL, int L,
+                                                    int64_t* sring, unsigned long long& st_del) {
+  const uint32_t* synw = (const uint32_t*)a.syn;
+  for (int r = 0; r < n; ++r) {
+    const uint32_t e = ents[r];
+    const uint32_t id = e & kIdMask;
+    const int g = (int)(e >> 24);
+    const size_t sb = (size_t)id * (a.P + 1) + p;
+    const uint32_t s0 = a.seg[sb], s1 = a.seg[sb + 1];
+    float xpre;
+    const int pg = event_source(a, ev, id, g, q, xpre);
+    if (q == 0) st_del += (unsigned long long)(s1 - s0);
+    // four synapses per lane and step, their loads in flight together
+    for (uint32_t k0 = s0 + (uint32_t)q; k0 < s1; k0 += 4 * kQuad) {
+      uint32_t pk[4], wb[4], mk[4];
+      float sc[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t k = k0 + (uint32_t)(u * kQuad);
+        if (k < s1) {
+          pk[u] = synw[(size_t)k * 2];
+          wb[u] = a.wfmt ? a.wc[k] : synw[(size_t)k * 2 + 1];
+          mk[u] = a.ev.mask[k >> 5];
+          sc[u] = PER_SYN_SCALE ? a.scale[k] : a.scale0;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t k = k0 + (uint32_t)(u * kQuad);
+        if (k >= s1) continue;
+        float w = a.wfmt ? dec16((uint16_t)(wb[u] & 0xFFFFu), a.wfmt) : __uint_as_float(wb[u]);
+        const uint32_t loc = pk[u] & 0xFFFFFu;
+        if (pg >= 0 && ((mk[u] >> (k & 31)) & 1u))
+          w = wupdate_c(a.ev.wts, (int64_t)k, w, (uint16_t)(wb[u] >> 16),
+                        wd_weight(w, xpre, ev.xq[loc], pg, ev.qg[loc], ev.tab, a.G), 0.0f, __builtin_inff());
+        const long long qv = __float2ll_rn((w * sc[u]) * a.two_k);
+        int slot = slot0 + g + (int)((pk[u] >> 20) & 0xFFu);
+        while (slot >= B) slot -= B;
+        atomicAdd((unsigned long long*)&sring[(size_t)slot * nownL + (size_t)loc * L + (pk[u] >> 28)],
+                  (unsigned long long)qv);
+      }
+    }
+  }
+}
+
+// The rule's target side, after the group's spikes have been delivered: the rule synapses onto
+// each owned neuron that spiked, except those whose source spiked too (updated above).
+template <int BS>
+__device__ __forceinline__ void event_targets(const FusedArgs& a, const EventLds& ev, int n, int nlo) {
+  for (int j = 0; j < n; ++j) {
+    const int v = ev.list[j];
+    const int64_t e1 = a.ev.post_ptr[nlo + v + 1];
+    for (int64_t e = a.ev.post_ptr[nlo + v] + threadIdx.x; e < e1; e += BS) {
+      const int u = a.ev.post_pre[e];
+      const int64_t k = (int64_t)a.ev.post_pos[e];
+      uint16_t c16;
+      const float w0 = wload_c(a.ev.wts, k, c16);
+      if ((ev.bits[u >> 5] >> (u & 31)) & 1u) continue;
+      wupdate_c(a.ev.wts, k, w0, c16, wd_weight(w0, ev.x[u], ev.xq[v], -1, ev.qg[v], ev.tab, a.G), 0.0f,
+                __builtin_inff());
+    }
+  }
+}
+
 // One quad's delivery of n entries staged in LDS, kSpikesPerQuad at a time, by the form of
 // the delivery table the launch uses.
-template <int DM>
+template <int DM, bool EV = false>
 __device__ __forceinline__ void deliver_staged(const FusedArgs& a, const uint32_t* ents, int n, int q, int p,
                                                int slot0, int BL, int nownL, int L, int64_t* sring,
                                                unsigned long long& st_del, long long q_lo, long long q_hi,
-                                               const uint16_t* slseg, const uint16_t* slrec) {
+                                               const uint16_t* slseg, const uint16_t* slrec,
+                                               const EventLds* ev = nullptr) {
+  if constexpr (EV) {
+    if (a.scale == nullptr) deliver_quad_events<false>(a, *ev, ents, n, q, p, slot0, BL, nownL, L, sring, st_del);
+    else deliver_quad_events<true>(a, *ev, ents, n, q, p, slot0, BL, nownL, L, sring, st_del);
+    return;
+  }
   for (int j0 = 0; j0 < n; j0 += kSpikesPerQuad) {
     const int m = min(kSpikesPerQuad, n - j0);
     if (DM != kDeliverCompact && a.lseg_U > 0) {
@@ -742,11 +881,12 @@ __device__ __forceinline__ void deliver_staged(const FusedArgs& a, const uint32_
 // longer lists follow eight entries at a time with their loads in flight together.
 // Returns false (in every lane of the wave) when a wait exceeded the spin limit or another
 // workgroup reported an error; the error flag is then set.
-template <int BS, int DM>
+template <int BS, int DM, bool EV>
 __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p, int par, uint32_t tag, int slot0,
                                                       int BL, int nownL, int L, int64_t* sring,
                                                       unsigned long long& st_del, long long q_lo, long long q_hi,
-                                                      const uint16_t* slseg, const uint16_t* slrec, uint32_t* sent) {
+                                                      const uint16_t* slseg, const uint16_t* slrec, uint32_t* sent,
+                                                      const EventLds* ev) {
   const int tid = threadIdx.x;
   const int lane = (int)__lane_id();
   const int quad = tid / kQuad, q = tid % kQuad;
@@ -792,7 +932,7 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
     }
     if (!ok) break;
     if (!active) continue;
-    if (DM != kDeliverCompact && a.lseg_U > 0) {
+    if (!EV && DM != kDeliverCompact && a.lseg_U > 0) {
       // LDS table: every lane delivers the entries it holds -- word q is entry q - 1, word
       // q + 4 entry q + 3 -- and longer lists eight at a time, two entries per lane
       const bool h0 = q >= 1 && q - 1 < c, h1 = q + 3 < c;
@@ -832,8 +972,8 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
     if (q >= 1 && q - 1 < c) qent[q - 1] = (uint32_t)w0;
     if (q + 3 < c) qent[q + 3] = (uint32_t)w1;
     __builtin_amdgcn_wave_barrier();
-    deliver_staged<DM>(a, qent, min(c, kQuadEnt - 1), q, p, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
-                       slrec);
+    deliver_staged<DM, EV>(a, qent, min(c, kQuadEnt - 1), q, p, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
+                           slrec, ev);
     for (int j0 = kQuadEnt - 1; j0 < c; j0 += kQuadEnt) {
       const int m = min(kQuadEnt, c - j0);
       const unsigned long long* eb = blk + 1 + j0;
@@ -855,7 +995,7 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
       if (q < m) qent[q] = (uint32_t)e0;
       if (q + kQuad < m) qent[q + kQuad] = (uint32_t)e1;
       __builtin_amdgcn_wave_barrier();
-      deliver_staged<DM>(a, qent, m, q, p, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec);
+      deliver_staged<DM, EV>(a, qent, m, q, p, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec, ev);
     }
     __builtin_amdgcn_wave_barrier();
   }
@@ -870,12 +1010,12 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
 // against the tag; (4) quads deliver kSpikesPerQuad staged entries at a time.  `scnt` is
 // LDS for P counts, `sscan` for P + 1 offsets.  Returns false when a wait failed (the error
 // flag is then set); uniform across the workgroup.
-template <int BS, int DM>
+template <int BS, int DM, bool EV>
 __device__ __forceinline__ bool tagged_gather_stage(const FusedArgs& a, int p, int par, uint32_t tag, int slot0,
                                                     int BL, int nownL, int L, int64_t* sring,
                                                     unsigned long long& st_del, long long q_lo, long long q_hi,
                                                     const uint16_t* slseg, const uint16_t* slrec, uint32_t* sent,
-                                                    int* scnt, int* sscan, int* s_ok) {
+                                                    int* scnt, int* sscan, int* s_ok, const EventLds* ev) {
   constexpr int kPer = kEntCap / BS;   // staged entries per thread and round
   const int tid = threadIdx.x;
   const int lane = (int)__lane_id();
@@ -959,8 +1099,8 @@ __device__ __forceinline__ bool tagged_gather_stage(const FusedArgs& a, int p, i
     __syncthreads();
     if (!*s_ok) return false;
     for (int j0 = quad * kSpikesPerQuad; j0 < nst; j0 += nquads * kSpikesPerQuad)
-      deliver_staged<DM>(a, sent + j0, min(kSpikesPerQuad, nst - j0), q, p, slot0, BL, nownL, L, sring, st_del,
-                         q_lo, q_hi, slseg, slrec);
+      deliver_staged<DM, EV>(a, sent + j0, min(kSpikesPerQuad, nst - j0), q, p, slot0, BL, nownL, L, sring, st_del,
+                             q_lo, q_hi, slseg, slrec, ev);
     __syncthreads();
   }
   return true;
@@ -1024,7 +1164,7 @@ __device__ __forceinline__ int partition_of_block(int b, int P) {
 
 // The group loop of one network for partition p, run by the workgroup that is member vb of
 // the network's P workgroups.
-template <int KIND, bool L1, bool PLASTIC, int BS, int DM>
+template <int KIND, bool L1, int PLASTIC, int BS, int DM>
 __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, const int vb, unsigned char* smem) {
   const int tid = threadIdx.x;
   const int lane = (int)__lane_id();
@@ -1032,8 +1172,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   const int ilo = a.ilo[p], ihi = a.ilo[p + 1];
   const int nown = nhi - nlo, iown = ihi - ilo;
   const int L = L1 ? 1 : a.L, G = a.G, B = a.B, BL = a.BL, W = a.W;
+  constexpr bool DENSE = PLASTIC == kRulesDense, EV = PLASTIC == kRulesEvents;
   const FusedLayout f = fused_layout(BL, L, W, G, a.nown_max, a.iown_max, a.xcap, a.P, a.lseg_U, a.lrec, a.cring,
-                                     a.dahead);
+                                     a.dahead, EV ? a.ev.sources : 0);
   int64_t* sring = (int64_t*)(smem + f.ring);
   uint32_t* scring = (uint32_t*)(smem + f.ring);   // count ring (a.cring)
   uint32_t* shist = (uint32_t*)(smem + f.hist);
@@ -1055,6 +1196,18 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   uint8_t* sguide = (uint8_t*)(smem + f.guide);
   uint16_t* slseg = (uint16_t*)(smem + f.lseg);
   uint16_t* slrec = (uint16_t*)(smem + f.lrec);
+  EventLds ev;
+  if constexpr (EV) {
+    ev.x = (float*)(smem + f.ev_x);
+    ev.bits = (uint32_t*)(smem + f.ev_bits);
+    ev.xq = (float*)(smem + f.ev_xq);
+    ev.qg = (int*)(smem + f.ev_qg);
+    ev.list = (int*)(smem + f.ev_list);
+    ev.tab = (float*)(smem + f.ev_tab);
+    for (int u = tid; u < a.ev.sources; u += BS) ev.x[u] = tload(a.ev.tr, 0, u);
+    for (int k = tid; k < (a.ev.sources + 31) / 32; k += BS) ev.bits[k] = 0u;
+    for (int k = tid; k < a.ev.ntab; k += BS) ev.tab[k] = a.ev.tab[k];
+  }
   __shared__ int s_ok;
   __shared__ int s_wsum[BS / kWave];
   __shared__ unsigned long long s_prof[kProfPhases];
@@ -1152,6 +1305,8 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     if (KIND != 0)
       for (int l = 0; l < L; ++l) gl[l] = a.gcond[(size_t)gi * L + l];
   }
+  float xq = 0.0f;   // kRulesEvents: postsynaptic trace of the owned neuron
+  if (EV && own) xq = tload(a.ev.tr, 1, gi);
   unsigned long long st_del = 0, st_ext = 0, st_spk = 0, st_in = 0;
   const float half_dt = 0.5f * a.dt;
   // fixed-point weights of the compact form: the full form's expression for one record
@@ -1167,7 +1322,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   // partitions keep the array; kernels of the LDS-table form never take this path)
   const bool in_ring = DM != kDeliverLdsTable && a.cring && a.nown_max > kWave && a.lseg_U == 0;
   // one wavefront holds every unit of the partition (nown_waves <= kWave)
-  const bool early = !PLASTIC && a.xquad && a.early && BS > kWave;
+  const bool early = !DENSE && a.xquad && a.early && BS > kWave;
   // population histogram of the window statistics: kStatBins consecutive bins, bin b in slot
   // b % kStatBins, collected in LDS and added to the global histogram when the next group's
   // bins would not fit (Brunel10K at 10-step bins: every 42 groups).  Adding every group's
@@ -1183,10 +1338,10 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   }
   // spike counters of the exchange list, one per group parity (the other parity's is
   // cleared while the group runs)
-  if (tid < 2) scounter[tid] = 0;
+  if (tid < 4) scounter[tid] = 0;   // (2, 3: spiking neurons listed for kRulesEvents)
   if (tid == 0) s_ok = 1;
   for (int j = tid; j < a.ext_k; j += BS) scdf[j] = a.ext_cdf[j];
-  if (!PLASTIC) {
+  if (!DENSE) {
     // this launch's exchange blocks start empty (tag 0 is never a group's tag), before any
     // of its publications
     for (int k = tid; k < 2 * a.xstride; k += BS) {
@@ -1225,9 +1380,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     const int slot0 = tidx % BL;
     // the lane's LDS addresses are computed in every group: hoisted out of the group loop they
     // would stay live across the delivery, which has no registers to spare (an empty asm, no
-    // instruction)
+    // instruction; the other kinds' label loops are faster with them kept: 7 %)
     int lt = tid;
-    asm volatile("" : "+v"(lt));
+    if constexpr (KIND == 0) asm volatile("" : "+v"(lt));
     // -- A. Poisson inputs: append this group's spikes, update histories ------------
     for (int i = tid; i < iown; i += BS) {
       const unsigned long long m = imask[i];
@@ -1321,6 +1476,20 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
       sst_s1[lt] = d1; sst_s2[lt] = d2;
     };
     unsigned long long smask_w = 0ull;
+    if constexpr (EV) {
+      // every source's trace decays by one group (from its stored value), beside the LIF;
+      // the marks of the last group's spikes are cleared
+      ev.t = t;
+      const float eg = ev.tab[5 + (G + 1) + G];
+      const int t0 = early ? kWave : 0;
+      if (tid >= t0) {
+        for (int u = tid - t0; u < a.ev.sources; u += BS - t0) {
+          const float x = ev.x[u];
+          if (x != 0.0f) ev.x[u] = (a.ev.tr.fmt ? dec16(enc16(x, a.ev.tr.fmt), a.ev.tr.fmt) : x) * eg;
+        }
+        for (int k = tid - t0; k < (a.ev.sources + 31) / 32; k += BS - t0) ev.bits[k] = 0u;
+      }
+    }
     if (early && tid >= kWave) {
       // the next group's random draws on the other wavefronts while wavefront 0 integrates
       if ((s + 1) % a.dahead == 0 && s + 1 < a.ngroups)
@@ -1471,6 +1640,18 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         }
         __builtin_amdgcn_s_setprio(0);
       }
+      if constexpr (EV) {
+        // the neuron's postsynaptic trace and spike step in the group, and its place in the
+        // list of spiking targets
+        if (own) {
+          const int qg = wd_post_step(last, t, a.dt, G);
+          if (a.ev.tr.fmt) xq = dec16(enc16(xq, a.ev.tr.fmt), a.ev.tr.fmt);
+          xq = wd_trace(xq, qg, ev.tab[0], ev.tab + 5, G, a.ev.nearest);
+          ev.xq[lt] = xq;
+          ev.qg[lt] = qg;
+          if (qg >= 0) ev.list[atomicAdd(&scounter[2 + par], 1)] = tid;
+        }
+      }
       if (!early && smask) {
         const int c = __popcll(smask);
         int pos = atomicAdd(scnt, c);
@@ -1503,11 +1684,11 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     // -- C. publish: {count, entries} block, and state other workgroups may read ------
     const int nxr = scnt[0];
     const int nx = min(nxr, a.xcap);
-    if (tid == 0) scounter[par ^ 1] = 0;
+    if (tid == 0) scounter[par ^ 1] = scounter[2 + (par ^ 1)] = 0;
     // more spikes than the exchange list holds: stop the launch with error 2
     if (tid == 0 && nxr > a.xcap) atomicExch(a.error, 2);
     const uint32_t tag = a.xtag_base + (uint32_t)s + 1u;
-    if (!PLASTIC) {
+    if (!DENSE) {
       if (!early) {
         unsigned long long* xl = a.xlist64 + ((size_t)par * a.P + p) * a.xstride;
         for (int k = tid; k < nx; k += BS) xstore64(xl + 1 + k, sxbuf[k], tag);
@@ -1518,7 +1699,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
       for (int k = tid; k < nx; k += BS) store_coherent(xl + 1 + k, sxbuf[k]);
       if (tid == 0) store_coherent(xl, (uint32_t)nx);
     }
-    if (PLASTIC) {
+    if (DENSE) {
       if (own) a.last_n[gi] = last;
       for (int k = tid; k < W * nown; k += BS) {
         const int wd = k / nown, i = k - wd * nown;
@@ -1551,7 +1732,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         }
       }
     }
-    if (!PLASTIC) {
+    if (!DENSE) {
       clk.lap(a, 2);
       // -- D. the next group's random draws while the other workgroups finish ----------
       if (!early && (s + 1) % a.dahead == 0 && s + 1 < a.ngroups)
@@ -1561,16 +1742,20 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
       // -- F. every source's list of this group, polled by its tags, delivered into the
       //    LDS ring (no grid barrier)
       if (a.xquad) {
-        if (!tagged_gather_deliver<BS, DM>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
-                                           slrec, sent))
+        if (!tagged_gather_deliver<BS, DM, EV>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
+                                               slrec, sent, &ev))
           s_ok = 0;
         __syncthreads();
       } else {
-        tagged_gather_stage<BS, DM>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec,
-                                    sent, (int*)shead, sscan, &s_ok);
+        tagged_gather_stage<BS, DM, EV>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec,
+                                        sent, (int*)shead, sscan, &s_ok, &ev);
       }
       if (!s_ok) return;
       clk.lap(a, 8);
+      if constexpr (EV) {
+        event_targets<BS>(a, ev, scounter[2 + par], nlo);
+        clk.lap(a, 5);
+      }
       continue;
     }
     __builtin_amdgcn_s_waitcnt(0);
@@ -1587,7 +1772,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     if (!s_ok) return;
     clk.lap(a, 4);
     // -- E. plasticity of the synapses onto this partition ---------------------------
-    if (PLASTIC) {
+    if (DENSE) {
       fused_plasticity<BS>(a.rules, a.n_rules, p, tidx, t);
       __syncthreads();
     }
@@ -1679,6 +1864,12 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     a.last_n[gi] = last;
     if (KIND != 0)
       for (int l = 0; l < L; ++l) a.gcond[(size_t)gi * L + l] = gl[l];
+    if (EV) tstore(a.ev.tr, 1, gi, xq);
+  }
+  if constexpr (EV) {
+    for (int i = tid; i < nown; i += BS) tstore(a.ev.tr, 0, nlo + i, ev.x[nlo + i]);
+    for (int i = tid; i < iown && a.N + ilo + i < a.ev.sources; i += BS)
+      tstore(a.ev.tr, 0, a.N + ilo + i, ev.x[a.N + ilo + i]);
   }
   // write the whole global ring slice back in its B-slot layout (zeros past the LDS window)
   {
@@ -1732,7 +1923,7 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   }
 }
 
-template <int KIND, bool L1, bool PLASTIC, int DM = kDeliverAny>
+template <int KIND, bool L1, int PLASTIC, int DM = kDeliverAny>
 __global__ __launch_bounds__(kFusedBlock) void k_fused(FusedArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   fused_body<KIND, L1, PLASTIC, kFusedBlock, DM>(a, partition_of_block(blockIdx.x, gridDim.x), blockIdx.x, smem);
@@ -1745,7 +1936,7 @@ __global__ __launch_bounds__(kFusedBlock) void k_fused(FusedArgs a) {
 // that are finishing earlier networks: every wait ends.  BS threads per workgroup: with
 // kBatchSmallBlock, two workgroups share a compute unit, so one network's partition runs
 // while the other's waits at its exchange (partitions of at most BS neurons).
-template <int KIND, bool L1, bool PLASTIC, int BS, int DM = kDeliverAny>
+template <int KIND, bool L1, int PLASTIC, int BS, int DM = kDeliverAny>
 __global__ __launch_bounds__(BS, 4) void k_fused_batch(const FusedArgs* __restrict__ nets,
                                                     const int2* __restrict__ tasks,
                                                     const int* __restrict__ task_off) {

@@ -12,10 +12,11 @@ namespace spk {
 template <int KIND, bool L1>
 FusedKernels instances() {
   FusedKernels k;
-  k.run = (const void*)k_fused<KIND, L1, false>;
-  k.run_plastic = (const void*)k_fused<KIND, L1, true>;
-  k.batch = (const void*)k_fused_batch<KIND, L1, false, kFusedBlock>;
-  k.batch_small = (const void*)k_fused_batch<KIND, L1, false, kBatchSmallBlock>;
+  k.run = (const void*)k_fused<KIND, L1, kRulesOff>;
+  k.run_plastic = (const void*)k_fused<KIND, L1, kRulesDense>;
+  k.run_events = (const void*)k_fused<KIND, L1, kRulesEvents>;
+  k.batch = (const void*)k_fused_batch<KIND, L1, kRulesOff, kFusedBlock>;
+  k.batch_small = (const void*)k_fused_batch<KIND, L1, kRulesOff, kBatchSmallBlock>;
   return k;
 }
 
@@ -32,12 +33,12 @@ FusedKernels fused_kernels_k2l1() { return instances<2, true>(); }
 #elif SPK_FUSED_PART == 5
 FusedKernels fused_kernels_k2ln() { return instances<2, false>(); }
 #else
-const void* fused_kernel_lds_table() { return (const void*)k_fused<0, true, false, kDeliverLdsTable>; }
-const void* fused_kernel_compact() { return (const void*)k_fused<0, true, false, kDeliverCompact>; }
+const void* fused_kernel_lds_table() { return (const void*)k_fused<0, true, kRulesOff, kDeliverLdsTable>; }
+const void* fused_kernel_compact() { return (const void*)k_fused<0, true, kRulesOff, kDeliverCompact>; }
 const void* batch_kernel_compact(bool small, bool tables) {
-  if (small) return (const void*)k_fused_batch<0, true, false, kBatchSmallBlock, kDeliverCompact>;   // (no tables)
-  return tables ? (const void*)k_fused_batch<0, true, false, kFusedBlock, kDeliverCompactAny>
-                : (const void*)k_fused_batch<0, true, false, kFusedBlock, kDeliverCompact>;
+  if (small) return (const void*)k_fused_batch<0, true, kRulesOff, kBatchSmallBlock, kDeliverCompact>;   // (no tables)
+  return tables ? (const void*)k_fused_batch<0, true, kRulesOff, kFusedBlock, kDeliverCompactAny>
+                : (const void*)k_fused_batch<0, true, kRulesOff, kFusedBlock, kDeliverCompact>;
 }
 #endif
 
