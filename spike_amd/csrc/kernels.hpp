@@ -209,6 +209,85 @@ __device__ __forceinline__ void wave_append(bool pred, uint32_t id, uint32_t* __
   }
 }
 
+// Device store of a spike monitor that the unit kernels write themselves (a launch of
+// k_collect per monitor and group otherwise); up to kUnitMons per population.
+struct UnitMon {
+  int32_t* ids;
+  float* times;
+  unsigned long long* count;
+  int64_t cap;
+};
+constexpr int kUnitMons = 4;
+
+// Appends the wavefront's spikes of sub-steps [g0, g0 + gn), gn <= 32: bit x of a lane's mask is
+// a spike of unit `id` (`local` within its population) at sub-step g0 + x.  Lane x reserves the
+// places of step x, so that all steps share one round trip of atomics, then the lists and the
+// monitors' stores are written.  Every lane of the wavefront must call this.
+__device__ __forceinline__ void wave_append_steps(uint32_t mask, int g0, int gn, uint32_t id, int local,
+                                                  uint32_t* __restrict__ lists, int* __restrict__ counts, int cap,
+                                                  unsigned long long* __restrict__ stat, const UnitMon* mon, int n_mons,
+                                                  float t, float dt) {
+  if (__ballot(mask != 0u) == 0) return;
+  const int lane = (int)__lane_id();
+  const uint64_t below = (1ull << lane) - 1ull;
+  int mine = 0, total = 0;
+  for (int x = 0; x < gn; ++x) {
+    const int c = __popcll(__ballot((mask >> x) & 1u));
+    total += c;
+    if (lane == x) mine = c;
+  }
+  int base = 0;
+  if (mine) base = atomicAdd(counts + g0 + lane, mine);
+  if (lane == 0) atomicAdd(stat, (unsigned long long)total);
+  unsigned long long mb[kUnitMons];
+#pragma unroll
+  for (int m = 0; m < kUnitMons; ++m) {
+    mb[m] = 0;
+    if (m < n_mons) {
+      if (lane == 0) mb[m] = atomicAdd(mon[m].count, (unsigned long long)total);
+      mb[m] = __shfl(mb[m], 0);
+    }
+  }
+  for (int x = 0; x < gn; ++x) {
+    const uint64_t b = __ballot((mask >> x) & 1u);
+    if (b == 0) continue;
+    const int pos = __shfl(base, x) + __popcll(b & below);
+    const bool in = (mask >> x) & 1u;
+    if (in && pos < cap) lists[(size_t)(g0 + x) * cap + pos] = id;
+#pragma unroll
+    for (int m = 0; m < kUnitMons; ++m) {
+      if (m < n_mons) {
+        const unsigned long long k = mb[m] + (unsigned long long)__popcll(b & below);
+        if (in && k < (unsigned long long)mon[m].cap) {
+          mon[m].ids[k] = local;
+          mon[m].times[k] = t + (float)(g0 + x) * dt;
+        }
+        mb[m] += (unsigned long long)__popcll(b);
+      }
+    }
+  }
+}
+
+// The bits [pos, pos + gn) (mod `bits`) of unit i's history ring: cleared, and set where the
+// mask has a spike; words that do not change are not written.
+__device__ __forceinline__ void hist_update(uint32_t* __restrict__ hist, int npop, int i, int bits, int pos, int gn,
+                                            uint32_t mask) {
+  int done = 0;
+  while (done < gn) {
+    const int off = pos & 31;
+    const int n = min(min(32 - off, gn - done), bits - pos);
+    const uint32_t ones = n == 32 ? 0xFFFFFFFFu : ((1u << n) - 1u);
+    const uint32_t sp = (mask >> done) & ones;
+    uint32_t* wp = hist + (size_t)(pos >> 5) * npop + i;
+    const uint32_t w0 = *wp;
+    const uint32_t w1 = (w0 & ~(ones << off)) | (sp << off);
+    if (w1 != w0) *wp = w1;
+    done += n;
+    pos += n;
+    if (pos >= bits) pos -= bits;
+  }
+}
+
 // ---------------------------------------------------------------------------------
 // group bookkeeping: clear the G per-sub-step counts of a list slot, record its time
 
@@ -279,14 +358,21 @@ struct LifArgs {
   uint64_t seed;
   StatsArgs st;
   uint32_t* rate;             // [N] spike counts of a rate monitor, or nullptr
+  int b0, slot0;              // history bit and ring slot of the group's first step
+  UnitMon mon[kUnitMons];     // spike monitors written here (k_collect writes the others)
+  int n_mons;
   int uni;                    // 1: every neuron has the parameters u_* (the arrays are not read)
   float u_v0, u_vreset, u_thr, u_c, u_rp;
 };
 
 // One lane of the LIF update for neuron i (lanes with i >= N take part in the wavefront's
-// list appends only).  Returns the neuron's last spike time after the group.
-template <int KIND>
-__device__ __forceinline__ float lif_unit(const LifArgs& a, int i) {
+// list appends only).  Returns the neuron's last spike time after the group.  The sub-steps
+// run CH at a time (1 for groups of one step, else 16): the chunk's inputs are read before the
+// recurrence, so that their loads are in flight together, and the spikes become a mask that is
+// appended once.  Bound by the latency of those loads when neurons are few, by bytes (56 per
+// neuron and step) when they are many; stores that would not change a word are left out.
+template <int KIND, int CH>
+__device__ __forceinline__ float lif_unit(const LifArgs& a, int i, const uint32_t* scdf) {
   const bool active = i < a.N;
   const int ii = active ? i : 0;
   float V = a.V[ii];
@@ -304,12 +390,8 @@ __device__ __forceinline__ float lif_unit(const LifArgs& a, int i) {
 #pragma unroll
     for (int l = 0; l < kMaxLabels; ++l) gl[l] = (l < a.L) ? a.gcond[(size_t)ii * a.L + l] : 0.0f;
   }
-  int cur_w = -1;
-  uint32_t word = 0;
   unsigned long long ext_sum = 0;
   const float half_dt = 0.5f * a.dt;
-  int64_t ext_blk = -1;
-  u32x4 ext_r{0u, 0u, 0u, 0u};
   unsigned int st_cnt = 0u, st_nisi = 0u;
   uint32_t nspk = 0u;
   float st_prev = 0.0f;
@@ -318,102 +400,141 @@ __device__ __forceinline__ float lif_unit(const LifArgs& a, int i) {
     st_cnt = a.st.count[i]; st_nisi = a.st.nisi[i]; st_prev = a.st.prev[i];
     st_s1 = a.st.s1[i]; st_s2 = a.st.s2[i];
   }
-  for (int g = 0; g < a.G; ++g) {
-    const int64_t step = (int64_t)a.tidx + g;
-    const int b = hist_bitpos(step, a.W);
-    const int w = b >> 5;
-    if (w != cur_w) {
-      if (cur_w >= 0 && active) a.hist[(size_t)cur_w * a.N + i] = word;
-      word = active ? a.hist[(size_t)w * a.N + i] : 0u;
-      cur_w = w;
-    }
-    word &= ~(1u << (b & 31));
-    // external per-neuron Poisson drive, joined to label 0 of this step's input
-    int64_t ext = 0;
+  const int bits = a.W * 32;
+  int hpos = a.b0, slot = a.slot0;
+  for (int g0 = 0; g0 < a.G; g0 += CH) {
+    const int gn = CH == 1 ? 1 : min(CH, a.G - g0);
+    // external per-neuron Poisson drive, joined to label 0 of each step's input: counts of the
+    // chunk's steps, 8 bits each
+    unsigned long long ext[2] = {0ull, 0ull};
     if (a.ext_k > 0) {
-      if ((step >> 2) != ext_blk) {
-        ext_blk = step >> 2;
-        ext_r = draw_block(a.seed, ext_blk, (uint32_t)ii, kStreamExternal);
-      }
-      const uint32_t u = pick(ext_r, (int)(step & 3));
-      int k = 0;
-      for (int j = 0; j < a.ext_k; ++j) k += (u >= a.ext_cdf[j]) ? 1 : 0;
-      ext = (int64_t)k * a.q_ext;
-      ext_sum += (unsigned long long)k;
-    }
-    const size_t slot = (size_t)((a.tidx + g) % a.B);
-    int64_t* rs = a.ring + slot * NL + (size_t)ii * a.L;
-    float dV;
-    if (KIND == 0) {
-      float total = 0.0f;
-      for (int l = 0; l < a.L; ++l) {
-        int64_t q = active ? rs[l] : 0;
-        if (l == 0) q += ext;
-        if (active) rs[l] = 0;
-        total += fixed_to_float(q) * a.inv_scale;
-      }
-      dV = total;
-    } else {
-      float total = 0.0f;
+      const int64_t s0 = (int64_t)a.tidx + g0;
+      for (int64_t blk = s0 >> 2; blk <= (s0 + gn - 1) >> 2; ++blk) {
+        const u32x4 r = draw_block(a.seed, blk, (uint32_t)ii, kStreamExternal);
+        int n4[4] = {0, 0, 0, 0};
+        for (int j = 0; j < a.ext_k; ++j) {
+          const uint32_t c = scdf[j];
 #pragma unroll
-      for (int l = 0; l < kMaxLabels; ++l) {
-        if (l < a.L) {
-          int64_t q = active ? rs[l] : 0;
-          if (l == 0) q += ext;
-          if (active) rs[l] = 0;
-          const float in = fixed_to_float(q) * a.inv_scale;
-          gl[l] = a.decay_g[l] * gl[l] + in;
-          // conductance: g (E - V) (InlineDeviceFunctions.hpp:22-51); current: the
-          // current trace itself (:52-84)
-          total += (KIND == 1) ? gl[l] * (a.erev[l] - V) : gl[l];
+          for (int k = 0; k < 4; ++k) n4[k] += (pick(r, k) >= c) ? 1 : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int x = (int)(blk * 4 + k - s0);
+          if (x >= 0 && x < gn) {
+            ext[x >> 3] |= (unsigned long long)n4[k] << ((x & 7) * 8);
+            ext_sum += (unsigned long long)n4[k];
+          }
         }
       }
-      dV = total * rp;
     }
-    const float tg = a.t + (float)g * a.dt;
-    bool spk = false;
-    if (((tg - last) - a.tref) > half_dt) {
-      V = ((cv0 + omc * V) + cib) + dV;
-      if (V >= thr) {
-        spk = true;
-        last = tg;
-        V = vr;
+    auto ext_q = [&](int x) -> int64_t {
+      return a.ext_k > 0 ? (int64_t)((ext[x >> 3] >> ((x & 7) * 8)) & 0xFFull) * a.q_ext : 0;
+    };
+    // one ring entry, cleared when it held anything
+    auto take = [&](int64_t* r) -> int64_t {
+      const int64_t q = active ? *r : 0;
+      if (q != 0) *r = 0;
+      return q;
+    };
+    uint32_t mask = 0u;
+    if (KIND == 0) {
+      float dv[CH];
+#pragma unroll
+      for (int x = 0; x < CH; ++x) {
+        dv[x] = 0.0f;
+        if (x < gn) {
+          int64_t* rs = a.ring + (size_t)slot * NL + (size_t)ii * a.L;
+          for (int l = 0; l < a.L; ++l) dv[x] += fixed_to_float(take(rs + l) + (l == 0 ? ext_q(x) : 0)) * a.inv_scale;
+          if (++slot == a.B) slot = 0;
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < CH; ++x) {
+        if (x < gn) {
+          const float tg = a.t + (float)(g0 + x) * a.dt;
+          const bool ready = ((tg - last) - a.tref) > half_dt;
+          const float vn = ((cv0 + omc * V) + cib) + dv[x];
+          const bool fire = ready && vn >= thr;
+          V = ready ? (fire ? vr : vn) : V;
+          last = fire ? tg : last;
+          mask |= (fire ? 1u : 0u) << x;
+        }
+      }
+    } else {
+      for (int x = 0; x < gn; ++x) {
+        int64_t* rs = a.ring + (size_t)slot * NL + (size_t)ii * a.L;
+        float total = 0.0f;
+#pragma unroll
+        for (int l = 0; l < kMaxLabels; ++l) {
+          if (l < a.L) {
+            const float in = fixed_to_float(take(rs + l) + (l == 0 ? ext_q(x) : 0)) * a.inv_scale;
+            gl[l] = a.decay_g[l] * gl[l] + in;
+            // conductance: g (E - V) (InlineDeviceFunctions.hpp:22-51); current: the
+            // current trace itself (:52-84)
+            total += (KIND == 1) ? gl[l] * (a.erev[l] - V) : gl[l];
+          }
+        }
+        if (++slot == a.B) slot = 0;
+        const float tg = a.t + (float)(g0 + x) * a.dt;
+        if (((tg - last) - a.tref) > half_dt) {
+          V = ((cv0 + omc * V) + cib) + total * rp;
+          if (V >= thr) {
+            last = tg;
+            V = vr;
+            mask |= 1u << x;
+          }
+        }
       }
     }
-    spk = spk && active;
-    if (spk) word |= (1u << (b & 31));
-    if (spk && a.st.on) {
-      stats_spike(a.st, step, tg, st_cnt, st_nisi, st_prev, st_s1, st_s2);
-      if (step >= a.st.t0 && step < a.st.t0 + a.st.nsteps) atomicAdd(a.st.hist + (step - a.st.t0) / a.st.bin, 1u);
+    if (!active) mask = 0u;
+    nspk += (uint32_t)__popc(mask);
+    if (a.st.on) {
+      for (uint32_t mm = mask; mm; mm &= mm - 1u) {
+        const int x = __ffs((int)mm) - 1;
+        const int64_t step = (int64_t)a.tidx + g0 + x;
+        stats_spike(a.st, step, a.t + (float)(g0 + x) * a.dt, st_cnt, st_nisi, st_prev, st_s1, st_s2);
+        if (step >= a.st.t0 && step < a.st.t0 + a.st.nsteps) atomicAdd(a.st.hist + (step - a.st.t0) / a.st.bin, 1u);
+      }
     }
-    wave_append(spk, (uint32_t)i, a.lists + (size_t)g * a.cap, a.counts + g, a.cap, a.spike_stat);
-    nspk += spk ? 1u : 0u;
+    if (active) hist_update(a.hist, a.N, i, bits, hpos, gn, mask);
+    hpos += gn;
+    if (hpos >= bits) hpos -= bits;
+    wave_append_steps(mask, g0, gn, (uint32_t)i, i, a.lists, a.counts, a.cap, a.spike_stat, a.mon, a.n_mons, a.t, a.dt);
   }
   if (active) {
-    if (cur_w >= 0) a.hist[(size_t)cur_w * a.N + i] = word;
     if (a.rate != nullptr && nspk) a.rate[i] += nspk;
     a.V[i] = V;
-    a.last[i] = last;
+    if (nspk) a.last[i] = last;
     if (KIND != 0) {
       for (int l = 0; l < a.L; ++l) a.gcond[(size_t)i * a.L + l] = gl[l];
     }
-    if (a.st.on) {
+    if (a.st.on && nspk) {
       a.st.count[i] = st_cnt; a.st.nisi[i] = st_nisi; a.st.prev[i] = st_prev;
       a.st.s1[i] = st_s1; a.st.s2[i] = st_s2;
     }
   }
   if (a.ext_k > 0) {
     // one atomic per wavefront for the event counter
-    unsigned long long s = active ? ext_sum : 0ull;
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if (__lane_id() == 0 && s) atomicAdd(a.ext_events, s);
+    unsigned long long e = active ? ext_sum : 0ull;
+    for (int off = 32; off > 0; off >>= 1) e += __shfl_xor(e, off);
+    if (__lane_id() == 0 && e) atomicAdd(a.ext_events, e);
   }
   return last;
 }
 
+// The external drive's count thresholds in LDS (scdf holds kMaxExtTable words).
+__device__ __forceinline__ void load_ext_table(const LifArgs& a, uint32_t* scdf) {
+  if (a.ext_k > 0) {
+    for (int j = threadIdx.x; j < a.ext_k; j += blockDim.x) scdf[j] = a.ext_cdf[j];
+    __syncthreads();
+  }
+}
+
 template <int KIND>
 __global__ __launch_bounds__(256) void k_lif(LifArgs a) {
-  lif_unit<KIND>(a, (int)(blockIdx.x * blockDim.x + threadIdx.x));
+  __shared__ uint32_t scdf[kMaxExtTable];
+  load_ext_table(a, scdf);
+  lif_unit<KIND, 16>(a, (int)(blockIdx.x * blockDim.x + threadIdx.x), scdf);
 }
 
 // ---------------------------------------------------------------------------------
@@ -431,53 +552,50 @@ struct PoissonArgs {
   float t, dt;
   uint64_t seed;
   uint32_t* rate;          // [Nin] spike counts of a rate monitor, or nullptr
+  int b0;                  // history bit of the group's first step
+  UnitMon mon[kUnitMons];
+  int n_mons;
 };
 
 // One lane of the Poisson inputs for input i; returns its last spike time after the group.
+template <int CH>
 __device__ __forceinline__ float poisson_unit(const PoissonArgs& a, int i) {
   const bool active = i < a.Nin;
   const int ii = active ? i : 0;
-  const uint32_t T = a.thr[ii];
+  const uint32_t T = active ? a.thr[ii] : 0u;
   float last = a.last[ii];
-  int64_t in_blk = -1;
-  u32x4 in_r{0u, 0u, 0u, 0u};
-  int cur_w = -1;
-  uint32_t word = 0;
   uint32_t nspk = 0u;
-  for (int g = 0; g < a.G; ++g) {
-    const int64_t step = (int64_t)a.tidx + g;
-    const int b = hist_bitpos(step, a.W);
-    const int w = b >> 5;
-    if (w != cur_w) {
-      if (cur_w >= 0 && active) a.hist[(size_t)cur_w * a.Nin + i] = word;
-      word = active ? a.hist[(size_t)w * a.Nin + i] : 0u;
-      cur_w = w;
+  const int bits = a.W * 32;
+  int hpos = a.b0;
+  for (int g0 = 0; g0 < a.G; g0 += CH) {
+    const int gn = CH == 1 ? 1 : min(CH, a.G - g0);
+    const int64_t s0 = (int64_t)a.tidx + g0;
+    uint32_t mask = 0u;
+    for (int64_t blk = s0 >> 2; blk <= (s0 + gn - 1) >> 2; ++blk) {
+      const u32x4 r = draw_block(a.seed, blk, (uint32_t)ii, kStreamInput);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int x = (int)(blk * 4 + k - s0);
+        if (x >= 0 && x < gn && pick(r, k) < T && s0 + x != a.arm_step) mask |= 1u << x;
+      }
     }
-    word &= ~(1u << (b & 31));
-    if ((step >> 2) != in_blk) {
-      in_blk = step >> 2;
-      in_r = draw_block(a.seed, in_blk, (uint32_t)ii, kStreamInput);
-    }
-    const uint32_t u = pick(in_r, (int)(step & 3));
-    const bool spk = active && (u < T) && (step != a.arm_step);
-    if (spk) {
-      word |= (1u << (b & 31));
-      last = a.t + (float)g * a.dt;
-      ++nspk;
-    }
-    wave_append(spk, (uint32_t)(a.N + i), a.lists + (size_t)g * a.cap, a.counts + g, a.cap,
-                a.spike_stat);
+    if (mask) last = a.t + (float)(g0 + 31 - __clz((int)mask)) * a.dt;
+    nspk += (uint32_t)__popc(mask);
+    if (active) hist_update(a.hist, a.Nin, i, bits, hpos, gn, mask);
+    hpos += gn;
+    if (hpos >= bits) hpos -= bits;
+    wave_append_steps(mask, g0, gn, (uint32_t)(a.N + i), i, a.lists, a.counts, a.cap, a.spike_stat, a.mon, a.n_mons, a.t,
+                      a.dt);
   }
-  if (active) {
-    if (cur_w >= 0) a.hist[(size_t)cur_w * a.Nin + i] = word;
+  if (active && nspk) {
     a.last[i] = last;
-    if (a.rate != nullptr && nspk) a.rate[i] += nspk;
+    if (a.rate != nullptr) a.rate[i] += nspk;
   }
   return last;
 }
 
 static __global__ __launch_bounds__(256) void k_poisson(PoissonArgs a) {
-  poisson_unit(a, (int)(blockIdx.x * blockDim.x + threadIdx.x));
+  poisson_unit<16>(a, (int)(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
 // ---------------------------------------------------------------------------------
@@ -559,6 +677,7 @@ struct PropArgs {
   unsigned long long* events;
   float scale0, two_k;
   int N, L, G, B, cap, tidx;
+  int slot0;                // ring slot of the group's first step
 };
 
 // A row is shared by kRowWaves wavefronts (wavefront c of a row takes its synapses
@@ -831,12 +950,12 @@ static __global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
 }
 
 // ---------------------------------------------------------------------------------
-// One group (G = 1) of the per-phase path in two launches, for networks with Poisson (or
-// no) inputs and at most one rule, a weight-dependent one in its spike-driven form:
-//   k_units   LIF neurons and Poisson inputs (one lane each), the rule's per-neuron traces
-//             and its list of spiking targets; clears the spike counts of the next group's
-//             list slot (so no separate group-start launch is needed);
-//   k_deliver propagation of this group's spikes and both sides of the rule:
+// One group of the per-phase path in two launches, for networks with Poisson (or no) inputs:
+//   k_units   LIF neurons and Poisson inputs (one lane each), the spike monitors' records, and
+//             for a weight-dependent rule in its spike-driven form (G = 1) the rule's
+//             per-neuron traces and its list of spiking targets; clears the spike counts of
+//             the next group's list slot (so no separate group-start launch is needed);
+//   k_deliver propagation of this group's spikes and, with that rule, both its sides:
 //             - source side: each spiking unit's row is walked once; a synapse the rule
 //               lists (bit of `mask`) is updated first and delivered with its new weight
 //               (the reference applies plasticity before propagation, SpikingModel.cpp:228-233);
@@ -844,8 +963,9 @@ static __global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
 //               did not spike in the group (those the source side does not reach).
 //             The two sides touch disjoint synapses, and propagation reads only the rows of
 //             this group's spikers, so all of it runs in one launch.
-// Results equal those of the separate kernels (k_begin_group, k_lif, k_poisson,
-// k_wd_neurons, k_wd_events, k_propagate) bit for bit.
+// Other rules run between the two launches.  Results equal those of the separate kernels
+// (k_begin_group, k_lif, k_poisson, k_wd_neurons, k_wd_events, k_propagate, k_collect) bit for
+// bit.
 
 struct UnitsArgs {
   LifArgs lif;
@@ -857,10 +977,11 @@ struct UnitsArgs {
   int slot, nb_neurons; // blocks [0, nb_neurons) run neurons, the rest inputs
 };
 
-template <int KIND, bool WD>
+template <int KIND, bool WD, int CH>
 __global__ __launch_bounds__(256) void k_units(UnitsArgs a) {
+  __shared__ uint32_t scdf[kMaxExtTable];
   if (blockIdx.x == 0) {
-    if ((int)threadIdx.x < a.lif.G) a.next_counts[threadIdx.x] = 0;
+    for (int g = threadIdx.x; g < a.lif.G; g += blockDim.x) a.next_counts[g] = 0;
     if (threadIdx.x == 0) {
       a.slot_time[a.slot] = a.lif.t;
       a.slot_tidx[a.slot] = a.lif.tidx;
@@ -868,7 +989,8 @@ __global__ __launch_bounds__(256) void k_units(UnitsArgs a) {
   }
   if ((int)blockIdx.x < a.nb_neurons) {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    const float last = lif_unit<KIND>(a.lif, i);
+    load_ext_table(a.lif, scdf);
+    const float last = lif_unit<KIND, CH>(a.lif, i, scdf);
     if (WD) {
       const bool on = i < a.lif.N;
       wd_pre_unit(a.wd, i, on, last, false);
@@ -876,7 +998,7 @@ __global__ __launch_bounds__(256) void k_units(UnitsArgs a) {
     }
   } else {
     const int i = (int)((blockIdx.x - a.nb_neurons) * blockDim.x + threadIdx.x);
-    const float last = poisson_unit(a.in, i);
+    const float last = poisson_unit<CH>(a.in, i);
     if (WD) wd_pre_unit(a.wd, a.in.N + i, i < a.in.Nin, last, false);
   }
 }
@@ -897,23 +1019,36 @@ __global__ __launch_bounds__(256) void k_deliver(DeliverArgs a) {
   const PropArgs& p = a.p;
   const WdEventArgs& r = a.wd;
   const size_t NL = (size_t)p.N * p.L;
-  const int slot0 = p.tidx % p.B;
-  const int nspk = min(p.counts[0], p.cap);
   int npost = 0;
   if (WD) {
     npost = min(r.cnt[2 * r.par + 1], r.N);
     // the other buffer is next group's: clear it (nothing reads it in this group)
     if (blockIdx.x == 0 && threadIdx.x < 2) r.cnt[2 * (r.par ^ 1) + threadIdx.x] = 0;
   }
-  const int tasks_src = nspk * a.row_waves;
-  const int tasks = tasks_src + npost * a.post_waves;
   unsigned long long ev = 0;
-  for (int w = wave; w < tasks; w += nwaves) {
-    if (w < tasks_src) {
-      const int j = w / a.row_waves, c = w - j * a.row_waves;
-      const uint32_t u = p.lists[j];
+  // source side: tasks (sub-step, spike, wavefront of its row), the sub-steps 64 at a time --
+  // lane x holds the tasks up to and including sub-step g0 + x
+  for (int g0 = 0; g0 < p.G; g0 += kWave) {
+    const int n = g0 + lane < p.G ? min(p.counts[g0 + lane], p.cap) : 0;
+    int incl = n * a.row_waves;
+    if (p.G > 1) {
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) {
+        const int y = __shfl_up(incl, off);
+        if (lane >= off) incl += y;
+      }
+    }
+    const int tasks = __shfl(incl, p.G > 1 ? kWave - 1 : 0);
+    for (int w = wave; w < tasks; w += nwaves) {
+      const int x = p.G > 1 ? __popcll(__ballot(incl <= w)) : 0;
+      const int first = p.G > 1 ? __shfl(incl - n * a.row_waves, x) : 0;
+      const int g = g0 + x;
+      const int j = (w - first) / a.row_waves, c = (w - first) - j * a.row_waves;
+      const uint32_t u = p.lists[(size_t)g * p.cap + j];
       const int64_t s0 = p.rowptr[u], s1 = p.rowptr[u + 1];
       if (lane == 0 && c == 0) ev += (unsigned long long)(s1 - s0);
+      int slot0 = p.slot0 + g;
+      while (slot0 >= p.B) slot0 -= p.B;
       float xpre = 0.0f;
       int pg = 0;
       if (WD) {
@@ -933,28 +1068,34 @@ __global__ __launch_bounds__(256) void k_deliver(DeliverArgs a) {
                          __builtin_inff());
         }
         const long long q = __float2ll_rn(wt * sc * p.two_k);
-        const int slot = (slot0 + d) % p.B;
+        int slot = slot0 + d;
+        while (slot >= p.B) slot -= p.B;
         const int l = p.label ? (int)p.label[s] : 0;
         atomicAdd((unsigned long long*)(p.ring + (size_t)slot * NL + (size_t)post * p.L + l),
                   (unsigned long long)q);
       }
-    } else if (WD) {
-      const int k = (w - tasks_src) / a.post_waves, c = (w - tasks_src) - k * a.post_waves;
-      const int v = (int)r.act[r.N + r.Nin + k];
-      const int qg = wd_post_step(r.last_n[v], r.t, r.dt, r.G);
-      const float xpost = r.xb[v];
-      const int64_t e1 = r.post_ptr[v + 1];
-      for (int64_t e = r.post_ptr[v] + c * kWave + lane; e < e1; e += (int64_t)a.post_waves * kWave) {
-        // every load of the update issued before the test (two levels of dependent loads)
-        const int u = r.post_pre[e];
-        const int64_t s = (int64_t)r.post_pos[e];
-        const float l = u < r.N ? r.last_n[u] : r.last_in[u - r.N];
-        const float xu = r.xa[u];
-        uint16_t c16;
-        const float w0 = wload_c(r.wts, s, c16);
-        const int pgu = wd_pre_step(l, r.t, r.dt, r.G);
-        if (pgu >= 0) continue;              // updated from the source side
-        wupdate_c(r.wts, s, w0, c16, wd_weight(w0, xu, xpost, pgu, qg, r.tab, r.G), 0.0f, __builtin_inff());
+    }
+    if (WD) {
+      // target side (G = 1): the wavefronts after those of the source side
+      for (int w = wave + (wave < tasks ? (tasks - wave + nwaves - 1) / nwaves * nwaves : 0) - tasks;
+           w < npost * a.post_waves; w += nwaves) {
+        const int k = w / a.post_waves, c = w - k * a.post_waves;
+        const int v = (int)r.act[r.N + r.Nin + k];
+        const int qg = wd_post_step(r.last_n[v], r.t, r.dt, r.G);
+        const float xpost = r.xb[v];
+        const int64_t e1 = r.post_ptr[v + 1];
+        for (int64_t e = r.post_ptr[v] + c * kWave + lane; e < e1; e += (int64_t)a.post_waves * kWave) {
+          // every load of the update issued before the test (two levels of dependent loads)
+          const int u = r.post_pre[e];
+          const int64_t s = (int64_t)r.post_pos[e];
+          const float l = u < r.N ? r.last_n[u] : r.last_in[u - r.N];
+          const float xu = r.xa[u];
+          uint16_t c16;
+          const float w0 = wload_c(r.wts, s, c16);
+          const int pgu = wd_pre_step(l, r.t, r.dt, r.G);
+          if (pgu >= 0) continue;              // updated from the source side
+          wupdate_c(r.wts, s, w0, c16, wd_weight(w0, xu, xpost, pgu, qg, r.tab, r.G), 0.0f, __builtin_inff());
+        }
       }
     }
   }

@@ -304,6 +304,7 @@ struct spk_network {
   double prof_us[spk::kProfPhases] = {0};
   // per-phase bookkeeping
   int cur_tidx = -1;
+  int cleared_tidx = -1;   // first step of the group whose list slot the last k_units cleared
   // start time of the latest group simulated since spk_reset_state: time only advances
   // (SpikingModel::run continues from the current time), so last-spike times never lie
   // ahead of a group, which the plasticity tables rely on
@@ -591,6 +592,7 @@ int begin_group(spk_network* n, float t, bool force = false) {
   const int tidx = (int)roundf(t / n->dt);
   if (tidx == n->cur_tidx && !force) return SPK_OK;
   n->cur_tidx = tidx;
+  n->cleared_tidx = -1;
   n->cur_slot = (tidx / n->G) % n->slots;
   hipLaunchKernelGGL(spk::k_begin_group, dim3(1), dim3(64), 0, n->stream,
                      n->d_counts + (size_t)n->cur_slot * n->Gprep, n->G, n->d_slot_time,
@@ -646,6 +648,8 @@ void fill_lif_args(spk_network* n, float t, int slot, spk::LifArgs& a) {
   a.q_ext = n->q_ext; a.seed = n->seed;
   a.st = stats_args(n, t);
   a.rate = n->d_rate[SPK_POP_NEURONS];
+  a.b0 = a.tidx % (n->W * 32);
+  a.slot0 = a.tidx % n->B;
   stats_advance(n, a.tidx, 1);
 }
 
@@ -700,6 +704,7 @@ void fill_poisson_args(spk_network* n, float t, int slot, spk::PoissonArgs& a) {
   a.N = n->N; a.Nin = n->Nin; a.G = n->G; a.W = n->W; a.cap = n->cap; a.tidx = tidx;
   a.arm_step = n->arm_step; a.t = t; a.dt = n->dt; a.seed = n->seed;
   a.rate = n->d_rate[SPK_POP_INPUTS];
+  a.b0 = tidx % (n->W * 32);
 }
 
 int launch_inputs(spk_network* n, float t, int slot) {
@@ -813,6 +818,7 @@ void fill_prop_args(spk_network* n, float t, int slot, spk::PropArgs& a) {
   a.scale0 = n->scale0; a.two_k = ldexpf(1.0f, n->frac);
   a.N = n->N; a.L = n->L; a.G = n->G; a.B = n->B; a.cap = n->cap;
   a.tidx = (int)roundf(t / n->dt);
+  a.slot0 = a.tidx % n->B;
 }
 
 int launch_propagate(spk_network* n, float t, int slot) {
@@ -824,32 +830,50 @@ int launch_propagate(spk_network* n, float t, int slot) {
   return SPK_OK;
 }
 
-// Groups of the per-phase path that run as two launches (k_units, k_deliver): G = 1,
-// LIF neurons, Poisson or no inputs, and no rule applied or one weight-dependent rule in
-// its spike-driven form.
-bool fast_group_ok(const spk_network* n, bool plastic) {
-  if (n->G != 1 || n->Gprep != 1 || n->gen || n->N == 0 || n->S == 0 || n->slots < 2) return false;
-  if (n->rules.empty() || !plastic) return true;
-  if (n->rules.size() != 1) return false;
+// Groups of the per-phase path that run as two launches (k_units, k_deliver), with the rules'
+// kernels between them: LIF neurons, Poisson or no inputs.
+bool fast_group_ok(const spk_network* n) {
+  return !n->gen && n->N > 0 && n->S > 0 && n->slots >= 2;
+}
+
+// A weight-dependent rule that k_units and k_deliver apply themselves (in its spike-driven form).
+bool rule_folds(const spk_network* n, bool plastic) {
+  if (!plastic || n->rules.size() != 1 || n->G != 1 || n->Gprep != 1) return false;
   const RuleHost& r = n->rules[0];
   return r.kind == 0 && r.ev_ok && r.cnt > 0 && !r.dense_next && n->d_wd_mask != nullptr;
 }
 
+// Workgroups of a delivery launch: two units' rows per workgroup keep the chip full for the
+// largest networks, and a launch of many idle workgroups costs a small network more than its
+// delivery (4096 workgroups: 4.4 us with nothing to do).
 constexpr int kDeliverBlocks = 4096;
+int deliver_blocks(const spk_network* n) {
+  return std::min(kDeliverBlocks, std::max(256, (n->nu() + 1) / 2));
+}
 
-// One group in two launches.  The current slot's spike counts were cleared by the previous
-// group's k_units, or, when `clear_now`, are cleared here by a group-start launch.
-int launch_group_fast(spk_network* n, float t, bool plastic, bool clear_now) {
-  if (clear_now) {
+template <int KIND, int CH>
+const void* units_kernel(bool wd) {
+  if (CH == 1 && wd) return (const void*)spk::k_units<KIND, true, 1>;
+  return (const void*)spk::k_units<KIND, false, CH>;
+}
+
+int launch_collect(spk_network* n, int mid, int slot0, int nslots);
+
+// One group in two launches, monitors included.  The slot's spike counts were cleared by the
+// previous group's k_units when that was the group before this one, else a group-start launch
+// clears them.
+int launch_group_fast(spk_network* n, float t, bool plastic) {
+  const int tidx = (int)roundf(t / n->dt);
+  if (n->cleared_tidx != tidx) {
     if (int rc = begin_group(n, t, true)) return rc;
   } else {
     if (int rc = check_time(n, t)) return rc;
-    n->cur_tidx = (int)roundf(t / n->dt);
-    n->cur_slot = (n->cur_tidx / n->G) % n->slots;
+    n->cur_tidx = tidx;
+    n->cur_slot = (tidx / n->G) % n->slots;
   }
   const int slot = n->cur_slot;
-  const int next = (n->cur_tidx / n->G + 1) % n->slots;
-  const bool wd = plastic && !n->rules.empty();
+  const int next = (tidx / n->G + 1) % n->slots;
+  const bool wd = rule_folds(n, plastic);
   RuleHost* r = wd ? &n->rules[0] : nullptr;
   spk::UnitsArgs u{};
   if (wd) {
@@ -862,33 +886,51 @@ int launch_group_fast(spk_network* n, float t, bool plastic, bool clear_now) {
   }
   fill_lif_args(n, t, slot, u.lif);
   if (n->Nin > 0) fill_poisson_args(n, t, slot, u.in);
+  std::vector<int> collect;   // monitors beyond kUnitMons of a population
+  for (int m = 0; m < (int)n->mons.size(); ++m) {
+    const MonitorHost& mh = n->mons[m];
+    const spk::UnitMon um{mh.d_ids, mh.d_times, mh.d_count, mh.capacity};
+    if (mh.pop == SPK_POP_NEURONS && u.lif.n_mons < spk::kUnitMons) u.lif.mon[u.lif.n_mons++] = um;
+    else if (mh.pop == SPK_POP_INPUTS && u.in.n_mons < spk::kUnitMons) u.in.mon[u.in.n_mons++] = um;
+    else collect.push_back(m);
+  }
   u.next_counts = n->d_counts + (size_t)next * n->Gprep;
   u.slot_time = n->d_slot_time;
   u.slot_tidx = n->d_slot_tidx;
   u.slot = slot;
-  u.nb_neurons = grid_for(n->N, 256);
-  const int blocks = u.nb_neurons + (n->Nin > 0 ? grid_for(n->Nin, 256) : 0);
+  // one wavefront per workgroup spreads few neurons over more compute units
+  const int bs = n->nu() <= 65536 ? 64 : 256;
+  u.nb_neurons = grid_for(n->N, bs);
+  const int blocks = u.nb_neurons + (n->Nin > 0 ? grid_for(n->Nin, bs) : 0);
+  const bool one = n->G == 1;
   const void* fn;
-  if (n->kind == SPK_SYN_VOLTAGE) fn = wd ? (const void*)spk::k_units<0, true> : (const void*)spk::k_units<0, false>;
-  else if (n->kind == SPK_SYN_CONDUCTANCE) fn = wd ? (const void*)spk::k_units<1, true> : (const void*)spk::k_units<1, false>;
-  else fn = wd ? (const void*)spk::k_units<2, true> : (const void*)spk::k_units<2, false>;
+  if (n->kind == SPK_SYN_VOLTAGE) fn = one ? units_kernel<0, 1>(wd) : units_kernel<0, 16>(wd);
+  else if (n->kind == SPK_SYN_CONDUCTANCE) fn = one ? units_kernel<1, 1>(wd) : units_kernel<1, 16>(wd);
+  else fn = one ? units_kernel<2, 1>(wd) : units_kernel<2, 16>(wd);
   void* uargs[] = {&u};
-  SPK_HIP(hipLaunchKernel(fn, dim3(blocks), dim3(256), uargs, 0, n->stream));
+  SPK_HIP(hipLaunchKernel(fn, dim3(blocks), dim3(bs), uargs, 0, n->stream));
+  n->cleared_tidx = tidx + n->G;
+  if (plastic && !wd)
+    for (int q = 0; q < (int)n->rules.size(); ++q)
+      if (int rc = launch_rule(n, q, t)) return rc;
   spk::DeliverArgs d{};
   fill_prop_args(n, t, slot, d.p);
   d.row_waves = (int)std::min<int64_t>(64, std::max<int64_t>(1, (n->max_row + spk::kWave - 1) / spk::kWave));
+  const int db = deliver_blocks(n);
   if (wd) {
     d.wd = u.wd;
     d.mask = n->d_wd_mask;
     d.post_waves = (int)std::min<int64_t>(64, std::max<int64_t>(1, (r->max_post + spk::kWave - 1) / spk::kWave));
-    hipLaunchKernelGGL(spk::k_deliver<true>, dim3(kDeliverBlocks), dim3(256), 0, n->stream, d);
+    hipLaunchKernelGGL(spk::k_deliver<true>, dim3(db), dim3(256), 0, n->stream, d);
     r->par ^= 1;
     r->syn_tr = false;
   } else {
     d.post_waves = 1;
-    hipLaunchKernelGGL(spk::k_deliver<false>, dim3(kDeliverBlocks), dim3(256), 0, n->stream, d);
+    hipLaunchKernelGGL(spk::k_deliver<false>, dim3(db), dim3(256), 0, n->stream, d);
   }
   SPK_HIP(hipGetLastError());
+  for (int m : collect)
+    if (int rc = launch_collect(n, m, slot, 1)) return rc;
   return SPK_OK;
 }
 
@@ -905,6 +947,21 @@ int launch_collect(spk_network* n, int mid, int slot0, int nslots) {
   a.Gs = n->Gprep;
   hipLaunchKernelGGL(spk::k_collect, dim3(8, nslots * n->G), dim3(256), 0, n->stream, a);
   SPK_HIP(hipGetLastError());
+  return SPK_OK;
+}
+
+// One group in a launch per phase: generator inputs, networks without neurons or synapses.
+int launch_group_phases(spk_network* n, float t, bool plastic) {
+  int rc;
+  if ((rc = begin_group(n, t, true))) return rc;
+  if ((rc = launch_neurons(n, t, n->cur_slot))) return rc;
+  if ((rc = launch_inputs(n, t, n->cur_slot))) return rc;
+  if (plastic)
+    for (int r = 0; r < (int)n->rules.size(); ++r)
+      if ((rc = launch_rule(n, r, t))) return rc;
+  if ((rc = launch_propagate(n, t, n->cur_slot))) return rc;
+  for (int m = 0; m < (int)n->mons.size(); ++m)
+    if ((rc = launch_collect(n, m, n->cur_slot, 1))) return rc;
   return SPK_OK;
 }
 
@@ -2157,6 +2214,7 @@ int spk_prepare(spk_network* n, int G) {
     if ((rc = upload(n->d_ilo, n->h_ilo.data(), (size_t)n->P + 1, st))) return rc;
     if ((rc = upload(n->d_seg, seg.data(), seg.size(), st))) return rc;
     SPK_HIP(hipMemsetAsync(n->d_xlist, 0, sizeof(uint64_t) * 2 * n->P * spk::fused_xstride(n->xcap), st));
+    SPK_HIP(hipMemsetAsync(n->d_err, 0, sizeof(int), st));   // read before the first launch, too
   }
   // rules: synapses grouped by the partition of their postsynaptic neuron
   for (auto& r : n->rules) {
@@ -2304,7 +2362,7 @@ int spk_set_timestep_grouping(spk_network* n, int G) {
   if (G < 1 || G > n->Gprep) return fail(SPK_ERR_ARG, "grouping must be in [1, prepared grouping]");
   if (G > n->dmin && n->S > 0) return fail(SPK_ERR_ARG, "grouping larger than the minimum delay");
   n->G = G;
-  n->cur_tidx = -1;
+  n->cur_tidx = n->cleared_tidx = -1;
   return SPK_OK;
 }
 
@@ -2377,7 +2435,7 @@ int spk_reset_state(spk_network* n) {
     }
     r.syn_tr = r.neu_tr = true;
   }
-  n->cur_tidx = -1;
+  n->cur_tidx = n->cleared_tidx = -1;
   n->t_hi = -INFINITY;
   return spk_reset_inputs(n);
 }
@@ -2434,25 +2492,15 @@ int spk_run(spk_network* n, float start, int64_t ngroups, int flags) {
     }
     const bool plastic = (flags & SPK_RUN_PLASTICITY) != 0;
     int since_drain = 0;
-    bool cleared = false;   // the previous group cleared this group's spike counts
+    n->cleared_tidx = -1;
     for (int64_t s = 0; s < ngroups; ++s) {
       const float t = start + (float)(s * n->G) * n->dt;
       int rc;
-      if (fast_group_ok(n, plastic)) {
-        if ((rc = launch_group_fast(n, t, plastic, !cleared))) return rc;
-        cleared = true;
+      if (fast_group_ok(n)) {
+        if ((rc = launch_group_fast(n, t, plastic))) return rc;
       } else {
-        cleared = false;
-        if ((rc = begin_group(n, t, true))) return rc;
-        if ((rc = launch_neurons(n, t, n->cur_slot))) return rc;
-        if ((rc = launch_inputs(n, t, n->cur_slot))) return rc;
-        if (plastic)
-          for (int r = 0; r < (int)n->rules.size(); ++r)
-            if ((rc = launch_rule(n, r, t))) return rc;
-        if ((rc = launch_propagate(n, t, n->cur_slot))) return rc;
+        if ((rc = launch_group_phases(n, t, plastic))) return rc;
       }
-      for (int m = 0; m < (int)n->mons.size(); ++m)
-        if ((rc = launch_collect(n, m, n->cur_slot, 1))) return rc;
       if (!n->mons.empty() && ++since_drain == 64) {
         since_drain = 0;
         for (auto& m : n->mons)
@@ -2480,25 +2528,18 @@ int spk_run(spk_network* n, float start, int64_t ngroups, int flags) {
 
 int spk_step_group(spk_network* n, float t, int flags) {
   if (int rc = check_prepared(n)) return rc;
-  const bool use_fused = n->fused_ok && !(flags & SPK_RUN_FORCE_LAUNCHES) && n->G == n->Gprep;
-  if (use_fused) {
+  // A launch of the persistent kernel for one group spends its time loading and storing the
+  // partitions' state (45-150 us per group); the two-launch form takes 10-20 us.  Networks
+  // generated on the device keep no lists for it.
+  if (n->generated && !(flags & SPK_RUN_FORCE_LAUNCHES) && n->G == n->Gprep) {
     if (int rc = check_time(n, t)) return rc;
     spk::FusedArgs a;
     if (int rc = fill_fused_args(n, rules_mode(n, (flags & SPK_RUN_PLASTICITY) != 0), a)) return rc;
     return launch_fused(n, a, t, 0, 1);
   }
   if (int rc = check_listed(n)) return rc;
-  int rc;
-  if ((rc = begin_group(n, t, true))) return rc;
-  if ((rc = launch_neurons(n, t, n->cur_slot))) return rc;
-  if ((rc = launch_inputs(n, t, n->cur_slot))) return rc;
-  if (flags & SPK_RUN_PLASTICITY)
-    for (int r = 0; r < (int)n->rules.size(); ++r)
-      if ((rc = launch_rule(n, r, t))) return rc;
-  if ((rc = launch_propagate(n, t, n->cur_slot))) return rc;
-  for (int m = 0; m < (int)n->mons.size(); ++m)
-    if ((rc = launch_collect(n, m, n->cur_slot, 1))) return rc;
-  return SPK_OK;
+  const bool plastic = (flags & SPK_RUN_PLASTICITY) != 0;
+  return fast_group_ok(n) ? launch_group_fast(n, t, plastic) : launch_group_phases(n, t, plastic);
 }
 
 int spk_get_counters(spk_network* n, spk_timing* t) {
@@ -2891,6 +2932,7 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
     return bail(rc);
   }
   SPK_HIP(hipMemsetAsync(n->d_xlist, 0, sizeof(uint64_t) * 2 * P * spk::fused_xstride(n->xcap), st));
+  SPK_HIP(hipMemsetAsync(n->d_err, 0, sizeof(int), st));
   SPK_HIP(hipMemsetAsync(n->d_stats, 0, sizeof(unsigned long long) * 4, st));
   SPK_HIP(hipMemsetAsync(d_count, 0, sizeof(unsigned int) * NN * P, st));
   SPK_HIP(hipMemsetAsync(d_cursor, 0, sizeof(unsigned int) * NN * P, st));
