@@ -174,6 +174,7 @@ struct MonitorHost {
   unsigned long long* d_count = nullptr;
   std::vector<int32_t> h_ids;  // drained by spk_run
   std::vector<float> h_times;
+  int64_t lo = INT64_MAX, hi = INT64_MIN;   // steps [lo, hi) recorded since the last drain
 };
 
 }  // namespace
@@ -316,6 +317,12 @@ struct spk_network {
   std::vector<std::vector<uint32_t>> rate_base;
   int cur_slot = 0;
   // timing
+  // ordering of a drained monitor's records (k_raster_*), grown as needed
+  uint32_t *d_ras_bits = nullptr, *d_ras_time = nullptr, *d_ras_tile = nullptr;
+  int32_t* d_ras_ids = nullptr;
+  float* d_ras_times = nullptr;
+  int* d_ras_flag = nullptr;
+  int64_t ras_words = 0, ras_rows = 0, ras_n = 0;
   hipEvent_t ev_a = nullptr, ev_b = nullptr;
   std::vector<hipEvent_t> ev_kernel;
   spk_timing timing{};
@@ -389,6 +396,16 @@ void free_device(spk_network* n) {
   dfree(n->d_st_s1); dfree(n->d_st_s2); dfree(n->d_st_out);
   for (auto& m : n->mons) {
     dfree(m.d_ids); dfree(m.d_times); dfree(m.d_count);
+  }
+  dfree(n->d_ras_bits); dfree(n->d_ras_time); dfree(n->d_ras_tile); dfree(n->d_ras_ids); dfree(n->d_ras_times);
+  dfree(n->d_ras_flag);
+}
+
+// Groups covering the steps [first, first + count) record into the network's monitors.
+void note_steps(spk_network* n, int64_t first, int64_t count) {
+  for (auto& m : n->mons) {
+    m.lo = std::min(m.lo, first);
+    m.hi = std::max(m.hi, first + count);
   }
 }
 
@@ -886,6 +903,7 @@ int launch_group_fast(spk_network* n, float t, bool plastic) {
   }
   fill_lif_args(n, t, slot, u.lif);
   if (n->Nin > 0) fill_poisson_args(n, t, slot, u.in);
+  note_steps(n, tidx, n->G);
   std::vector<int> collect;   // monitors beyond kUnitMons of a population
   for (int m = 0; m < (int)n->mons.size(); ++m) {
     const MonitorHost& mh = n->mons[m];
@@ -936,6 +954,7 @@ int launch_group_fast(spk_network* n, float t, bool plastic) {
 
 int launch_collect(spk_network* n, int mid, int slot0, int nslots) {
   MonitorHost& m = n->mons[mid];
+  note_steps(n, n->cur_tidx, n->G);
   spk::CollectArgs a{};
   a.lists = n->d_lists; a.counts = n->d_counts; a.slot_time = n->d_slot_time;
   a.ids = m.d_ids; a.times = m.d_times; a.count = m.d_count; a.store_cap = m.capacity;
@@ -965,6 +984,102 @@ int launch_group_phases(spk_network* n, float t, bool plastic) {
   return SPK_OK;
 }
 
+// Records from which the device orders a drained monitor: below, sorting them on the host costs
+// no more than the launches and fills do (about 30 ns a record against 60 us).
+constexpr int64_t kRasterMin = 2048;
+constexpr int64_t kRasterMaxWords = (int64_t)1 << 24;   // 64 MB of bits
+// Steps below which a record's step and its time determine each other: the float time of step
+// k is within 2^-22 k steps of k.
+constexpr int64_t kRasterMaxStep = (int64_t)1 << 20;
+
+// The monitor's `cnt` records in (time, id) order at the ends of ids and times, ordered on the
+// device; `done` stays false when that form does not apply (the store is left as it is).
+int order_on_device(spk_network* n, const MonitorHost& m, int64_t cnt, std::vector<int32_t>& ids,
+                    std::vector<float>& times, bool& done) {
+  done = false;
+  const int64_t row0 = m.lo - 1, nrows = m.hi - m.lo + 2;
+  if (cnt < kRasterMin || cnt > INT32_MAX || m.lo < 0 || m.hi <= m.lo || m.hi > kRasterMaxStep) return SPK_OK;
+  const int64_t wpr = ((m.pop == SPK_POP_NEURONS ? n->N : n->Nin) + 31) / 32;
+  const int64_t words = nrows * wpr;
+  if (words > kRasterMaxWords) return SPK_OK;
+  int rc;
+  if (!n->d_ras_flag && (rc = dalloc(&n->d_ras_flag, 2))) return rc;
+  const int64_t tiles = (words + spk::kRasterTile - 1) / spk::kRasterTile;
+  if (words > n->ras_words) {
+    const int64_t cap = std::min(kRasterMaxWords, words + words / 2);
+    dfree(n->d_ras_bits); dfree(n->d_ras_tile);
+    n->ras_words = 0;
+    if ((rc = dalloc(&n->d_ras_bits, (size_t)cap))) return rc;
+    if ((rc = dalloc(&n->d_ras_tile, (size_t)(cap + spk::kRasterTile - 1) / spk::kRasterTile))) return rc;
+    n->ras_words = cap;
+    SPK_HIP(hipMemsetAsync(n->d_ras_bits, 0, sizeof(uint32_t) * cap, n->stream));   // k_raster_emit keeps it zero
+  }
+  if (nrows > n->ras_rows) {
+    dfree(n->d_ras_time);
+    n->ras_rows = 0;
+    if ((rc = dalloc(&n->d_ras_time, (size_t)(nrows + nrows / 2)))) return rc;
+    n->ras_rows = nrows + nrows / 2;
+  }
+  if (cnt > n->ras_n) {
+    dfree(n->d_ras_ids); dfree(n->d_ras_times);
+    n->ras_n = 0;
+    if ((rc = dalloc(&n->d_ras_ids, (size_t)(cnt + cnt / 2)))) return rc;
+    if ((rc = dalloc(&n->d_ras_times, (size_t)(cnt + cnt / 2)))) return rc;
+    n->ras_n = cnt + cnt / 2;
+  }
+  spk::RasterArgs a{};
+  a.ids = m.d_ids; a.times = m.d_times; a.n = cnt; a.dt = n->dt;
+  a.row0 = (int)row0; a.nrows = (int)nrows; a.wpr = (int)wpr;
+  a.bits = n->d_ras_bits; a.steptime = n->d_ras_time; a.tile = n->d_ras_tile;
+  a.out_ids = n->d_ras_ids; a.out_times = n->d_ras_times; a.flag = n->d_ras_flag;
+  SPK_HIP(hipMemsetAsync(n->d_ras_time, 0xFF, sizeof(uint32_t) * nrows, n->stream));
+  SPK_HIP(hipMemsetAsync(n->d_ras_flag, 0, sizeof(int) * 2, n->stream));
+  hipLaunchKernelGGL(spk::k_raster_mark, dim3((int)std::min<int64_t>(1024, (cnt + 255) / 256)), dim3(256), 0, n->stream, a);
+  hipLaunchKernelGGL(spk::k_raster_tiles, dim3((int)tiles), dim3(spk::kRasterBlock), 0, n->stream, a);
+  hipLaunchKernelGGL(spk::k_raster_emit, dim3((int)tiles), dim3(spk::kRasterBlock), 0, n->stream, a);
+  SPK_HIP(hipGetLastError());
+  const size_t at = ids.size();
+  ids.resize(at + (size_t)cnt);
+  times.resize(at + (size_t)cnt);
+  int flag[2] = {0, 0};
+  SPK_HIP(hipMemcpyAsync(flag, n->d_ras_flag, sizeof(flag), hipMemcpyDeviceToHost, n->stream));
+  SPK_HIP(hipMemcpyAsync(ids.data() + at, n->d_ras_ids, cnt * sizeof(int32_t), hipMemcpyDeviceToHost, n->stream));
+  SPK_HIP(hipMemcpyAsync(times.data() + at, n->d_ras_times, cnt * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+  SPK_HIP(hipStreamSynchronize(n->stream));
+  done = flag[0] == 0 && (int64_t)flag[1] == cnt;
+  if (!done) {
+    ids.resize(at);
+    times.resize(at);
+  }
+  return SPK_OK;
+}
+
+// The same on the host: the records as 64-bit keys, time above id (float order as unsigned
+// order), sorted.
+int order_on_host(spk_network* n, const MonitorHost& m, int64_t cnt, std::vector<int32_t>& ids,
+                  std::vector<float>& times) {
+  std::vector<int32_t> bi(cnt);
+  std::vector<float> bt(cnt);
+  SPK_HIP(hipMemcpyAsync(bi.data(), m.d_ids, cnt * sizeof(int32_t), hipMemcpyDeviceToHost, n->stream));
+  SPK_HIP(hipMemcpyAsync(bt.data(), m.d_times, cnt * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+  SPK_HIP(hipStreamSynchronize(n->stream));
+  std::vector<uint64_t> key(cnt);
+  for (int64_t i = 0; i < cnt; ++i) {
+    const uint32_t b = spk::f32_bits(bt[i] + 0.0f);   // (-0 as +0)
+    key[i] = (uint64_t)(b & 0x80000000u ? ~b : b | 0x80000000u) << 32 | (uint32_t)bi[i];
+  }
+  std::sort(key.begin(), key.end());
+  const size_t at = ids.size();
+  ids.resize(at + (size_t)cnt);
+  times.resize(at + (size_t)cnt);
+  for (int64_t i = 0; i < cnt; ++i) {
+    const uint32_t b = (uint32_t)(key[i] >> 32);
+    ids[at + i] = (int32_t)(uint32_t)key[i];
+    times[at + i] = spk::bits_f32(b & 0x80000000u ? b & 0x7FFFFFFFu : ~b);
+  }
+  return SPK_OK;
+}
+
 // Drain a monitor's device store into its host vectors, sorted by (time, id).
 int drain_monitor(spk_network* n, MonitorHost& m, std::vector<int32_t>& ids,
                   std::vector<float>& times) {
@@ -974,24 +1089,15 @@ int drain_monitor(spk_network* n, MonitorHost& m, std::vector<int32_t>& ids,
   if ((int64_t)cnt > m.capacity)
     return fail(SPK_ERR_CAPACITY, "spike monitor device store overflowed (" +
                                       std::to_string(cnt) + " > " + std::to_string(m.capacity) + ")");
-  std::vector<int32_t> bi(cnt);
-  std::vector<float> bt(cnt);
   if (cnt) {
-    SPK_HIP(hipMemcpyAsync(bi.data(), m.d_ids, cnt * sizeof(int32_t), hipMemcpyDeviceToHost, n->stream));
-    SPK_HIP(hipMemcpyAsync(bt.data(), m.d_times, cnt * sizeof(float), hipMemcpyDeviceToHost, n->stream));
+    bool done = false;
+    if (int rc = order_on_device(n, m, (int64_t)cnt, ids, times, done)) return rc;
+    if (!done)
+      if (int rc = order_on_host(n, m, (int64_t)cnt, ids, times)) return rc;
+    SPK_HIP(hipMemsetAsync(m.d_count, 0, sizeof(unsigned long long), n->stream));
   }
-  SPK_HIP(hipMemsetAsync(m.d_count, 0, sizeof(unsigned long long), n->stream));
-  SPK_HIP(hipStreamSynchronize(n->stream));
-  std::vector<size_t> order(cnt);
-  for (size_t i = 0; i < cnt; ++i) order[i] = i;
-  std::sort(order.begin(), order.end(), [&](size_t a, size_t b) {
-    if (bt[a] != bt[b]) return bt[a] < bt[b];
-    return bi[a] < bi[b];
-  });
-  for (size_t i : order) {
-    ids.push_back(bi[i]);
-    times.push_back(bt[i]);
-  }
+  m.lo = INT64_MAX;
+  m.hi = INT64_MIN;
   return SPK_OK;
 }
 
@@ -1246,6 +1352,11 @@ int stage_fused(spk_network* n, spk::FusedArgs& a, float start, int64_t group0, 
   a.arm_step = n->Nin > 0 ? n->arm_step : -1;
   a.st = stats_args(n, start);
   stats_advance(n, (int64_t)roundf(start / n->dt), group0 + ng);
+  if (ng > 0 && !n->mons.empty()) {
+    auto step_of = [&](int64_t g) { return (int64_t)roundf((start + (float)(g * n->G) * n->dt) / n->dt); };
+    note_steps(n, step_of(group0), 0);
+    note_steps(n, step_of(group0 + ng - 1), n->G);
+  }
   a.start = start;
   a.group0 = group0;
   a.ngroups = ng;
@@ -1306,7 +1417,8 @@ int run_fused(spk_network* n, float start, int64_t ngroups, int flags) {
   for (auto& m : n->mons) {
     const int64_t pop = std::max<int64_t>(1, m.pop == SPK_POP_NEURONS ? n->N : n->Nin);
     const int64_t per_group = pop * G;
-    const int64_t want = std::max<int64_t>(m.capacity, std::min<int64_t>(per_group * 256, (int64_t)1 << 27));
+    const int64_t want = std::max<int64_t>(m.capacity, std::max(std::min<int64_t>(per_group * 256, (int64_t)1 << 27),
+                                                                std::min<int64_t>(per_group * chunk, (int64_t)1 << 24)));
     if (int rc = ensure_monitor_capacity(n, m, std::max<int64_t>(want, per_group))) return rc;
     chunk = std::max<int64_t>(1, std::min<int64_t>(chunk, m.capacity / per_group));
   }
@@ -2665,6 +2777,8 @@ int spk_monitor_reset(spk_network* n, int mid) {
   if (mid < 0 || mid >= (int)n->mons.size()) return fail(SPK_ERR_ARG, "bad monitor");
   MonitorHost& m = n->mons[mid];
   SPK_HIP(hipMemsetAsync(m.d_count, 0, sizeof(unsigned long long), n->stream));
+  m.lo = INT64_MAX;
+  m.hi = INT64_MIN;
   m.h_ids.clear();
   m.h_times.clear();
   return SPK_OK;
