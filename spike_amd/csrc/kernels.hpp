@@ -1454,6 +1454,45 @@ static __global__ __launch_bounds__(kRasterBlock) void k_raster_emit(RasterArgs 
 }
 
 // ---------------------------------------------------------------------------------
+// The dynamic state of SpikingModel::reset_state (SpikingModel.cpp:181-190) and the window
+// statistics' start, each in one launch of 3 us that nothing waits for (a copy or fill per array
+// and a wait before: 33 us a reset).
+struct ResetArgs {
+  const float* v0;
+  float *V, *last_n, *g, *last_in;
+  uint32_t *hist_n, *hist_in;
+  int64_t* ring;
+  int64_t N, NL, ring_n, hist_nn, Nin, hist_in_n;   // N = 0: inputs only
+};
+
+static __global__ __launch_bounds__(256) void k_reset_state(ResetArgs a) {
+  const int64_t k0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  if (a.N > 0) {
+    for (int64_t i = k0; i < a.N; i += step) {
+      a.V[i] = a.v0[i];
+      a.last_n[i] = -1000.0f;
+    }
+    for (int64_t i = k0; i < a.NL; i += step) a.g[i] = 0.0f;
+    for (int64_t i = k0; i < a.hist_nn; i += step) a.hist_n[i] = 0u;
+    for (int64_t i = k0; i < a.ring_n; i += step) a.ring[i] = 0;
+  }
+  for (int64_t i = k0; i < a.Nin; i += step) a.last_in[i] = -1000.0f;
+  for (int64_t i = k0; i < a.hist_in_n; i += step) a.hist_in[i] = 0u;
+}
+
+static __global__ __launch_bounds__(256) void k_stats_clear(StatsArgs st, int64_t n, int64_t bins) {
+  const int64_t k0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = k0; i < n; i += step) {
+    st.count[i] = 0u;
+    st.nisi[i] = 0u;
+    st.prev[i] = 0.0f;
+    st.s1[i] = 0.0;
+    st.s2[i] = 0.0;
+  }
+  for (int64_t i = k0; i < bins; i += step) st.hist[i] = 0u;
+}
+
+// ---------------------------------------------------------------------------------
 // FP64 reduction of the window statistics (one workgroup; fixed summation order, so the
 // result is reproducible):
 //   rate      = spikes / (N * nsteps * dt)

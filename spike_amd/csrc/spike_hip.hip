@@ -1080,6 +1080,30 @@ int order_on_host(spk_network* n, const MonitorHost& m, int64_t cnt, std::vector
   return SPK_OK;
 }
 
+// Reset of the inputs and, when `neurons`, of the neurons' state and input ring; enqueued.
+int launch_reset(spk_network* n, bool neurons) {
+  spk::ResetArgs a{};
+  if (neurons) {
+    a.N = n->N;
+    a.NL = (int64_t)n->N * n->L;
+    a.ring_n = (int64_t)n->B * n->N * n->L;
+    a.hist_nn = (int64_t)n->W * n->N;
+  }
+  a.Nin = n->Nin;
+  a.hist_in_n = (int64_t)n->W * n->Nin;
+  a.v0 = n->d_v0; a.V = n->d_V; a.last_n = n->d_last_n; a.g = n->d_g; a.last_in = n->d_last_in;
+  a.hist_n = n->d_hist_n; a.hist_in = n->d_hist_in; a.ring = n->d_ring;
+  const int64_t most = std::max(std::max(a.ring_n, a.hist_nn), std::max(a.Nin, a.hist_in_n));
+  if (most > 0) {
+    hipLaunchKernelGGL(spk::k_reset_state, dim3((int)std::min<int64_t>(2048, (most + 1023) / 1024)), dim3(256), 0,
+                       n->stream, a);
+    SPK_HIP(hipGetLastError());
+  }
+  n->pending_arm = true;
+  n->arm_step = -1;
+  return SPK_OK;
+}
+
 // Drain a monitor's device store into its host vectors, sorted by (time, id).
 int drain_monitor(spk_network* n, MonitorHost& m, std::vector<int32_t>& ids,
                   std::vector<float>& times) {
@@ -1165,20 +1189,14 @@ size_t fused_lds_limit(const spk_network* n) {
 
 // The compact form's delivery table of each partition -- a 16-bit local start per source
 // unit and the partition's 2-byte targets -- stays in LDS for the whole launch when the
-// largest partition's table fits beside the rest (fewer than 2^16 targets).  `seg` is the
-// [U][P+1] segment table.
-int plan_lds_table(spk_network* n, const uint32_t* seg, int U) {
+// largest partition's table fits beside the rest (fewer than 2^16 targets).  `mx`: targets of
+// the partition with most.
+int plan_lds_table(spk_network* n, int64_t mx, int U) {
   n->fused_lds_base = n->fused_lds;
   n->lseg_U = 0;
   n->lrec = 0;
   if (!n->fused_ok || !n->compact || !n->rules.empty() || U <= 0 || U >= (1 << 24)) return SPK_OK;
   const int P = n->P;
-  std::vector<int64_t> cnt(P, 0);
-  for (int u = 0; u < U; ++u) {
-    const uint32_t* r = seg + (size_t)u * (P + 1);
-    for (int q = 0; q < P; ++q) cnt[q] += r[q + 1] - r[q];
-  }
-  const int64_t mx = *std::max_element(cnt.begin(), cnt.end());
   if (mx > 65535) return SPK_OK;
   const size_t full = spk::fused_lds_bytes(n->BL, n->L, n->W, n->G, n->nown_max, n->iown_max, n->xcap, P,
                                            U, (int)mx, n->cring_ok ? 1 : 0);
@@ -2266,7 +2284,12 @@ int spk_prepare(spk_network* n, int G) {
     if (n->cring_ok)
       n->fused_lds = spk::fused_lds_bytes(n->BL, n->L, n->W, G, n->nown_max, n->iown_max, n->xcap, n->P, 0, 0, 1);
   }
-  if (int rc = plan_lds_table(n, seg.data(), U)) return rc;
+  {
+    std::vector<int64_t> cnt(n->P, 0);   // synapses onto each partition
+    if (n->compact)
+      for (int64_t s = 0; s < S; ++s) cnt[owner[n->h_post[s]]]++;
+    if (int rc = plan_lds_table(n, *std::max_element(cnt.begin(), cnt.end()), U)) return rc;
+  }
   // list capacity: every neuron of both populations may spike once per sub-step; two
   // slots, so that a group can clear the next group's counts (k_units)
   n->cap = std::max(1, U);
@@ -2503,29 +2526,12 @@ int spk_get_info(const spk_network* n, spk_info* info) {
 
 int spk_reset_inputs(spk_network* n) {
   if (int rc = check_prepared(n)) return rc;
-  if (n->Nin > 0) {
-    std::vector<float> ls(n->Nin, -1000.0f);
-    if (int rc = upload(n->d_last_in, ls.data(), ls.size(), n->stream)) return rc;
-    SPK_HIP(hipMemsetAsync(n->d_hist_in, 0, sizeof(uint32_t) * n->W * n->Nin, n->stream));
-  }
-  n->pending_arm = true;
-  n->arm_step = -1;
-  SPK_HIP(hipStreamSynchronize(n->stream));
-  return SPK_OK;
+  return launch_reset(n, false);
 }
 
 int spk_reset_state(spk_network* n) {
   if (int rc = check_prepared(n)) return rc;
   hipStream_t st = n->stream;
-  if (n->N > 0) {
-    if (int rc = upload(n->d_V, n->v0.data(), (size_t)n->N, st)) return rc;
-    std::vector<float> ls(n->N, -1000.0f);
-    if (int rc = upload(n->d_last_n, ls.data(), ls.size(), st)) return rc;
-    SPK_HIP(hipMemsetAsync(n->d_hist_n, 0, sizeof(uint32_t) * n->W * n->N, st));
-    SPK_HIP(hipMemsetAsync(n->d_ring, 0, sizeof(int64_t) * n->B * n->N * n->L, st));
-    SPK_HIP(hipMemsetAsync(n->d_g, 0, sizeof(float) * n->N * n->L, st));
-    SPK_HIP(hipStreamSynchronize(st));
-  }
   for (auto& r : n->rules) {
     const size_t P = (size_t)r.cnt;
     if (P && r.kind != 4) {   // (weight normalization keeps its initial weights there)
@@ -2549,7 +2555,7 @@ int spk_reset_state(spk_network* n) {
   }
   n->cur_tidx = n->cleared_tidx = -1;
   n->t_hi = -INFINITY;
-  return spk_reset_inputs(n);
+  return launch_reset(n, true);
 }
 
 int spk_update_neurons(spk_network* n, float t) {
@@ -2685,12 +2691,13 @@ int spk_stats_begin(spk_network* n, int bin_steps, int64_t max_steps) {
     if (int rc = dalloc(&n->d_st_hist, (size_t)nb)) return rc;
     n->st_nbins = nb;
   }
-  SPK_HIP(hipMemsetAsync(n->d_st_cnt, 0, N * sizeof(unsigned int), n->stream));
-  SPK_HIP(hipMemsetAsync(n->d_st_nisi, 0, N * sizeof(unsigned int), n->stream));
-  SPK_HIP(hipMemsetAsync(n->d_st_prev, 0, N * sizeof(float), n->stream));
-  SPK_HIP(hipMemsetAsync(n->d_st_s1, 0, N * sizeof(double), n->stream));
-  SPK_HIP(hipMemsetAsync(n->d_st_s2, 0, N * sizeof(double), n->stream));
-  SPK_HIP(hipMemsetAsync(n->d_st_hist, 0, (size_t)nb * sizeof(unsigned int), n->stream));
+  spk::StatsArgs st{};
+  st.count = n->d_st_cnt; st.nisi = n->d_st_nisi; st.prev = n->d_st_prev;
+  st.s1 = n->d_st_s1; st.s2 = n->d_st_s2; st.hist = n->d_st_hist;
+  const int64_t most = std::max<int64_t>((int64_t)N, nb);
+  hipLaunchKernelGGL(spk::k_stats_clear, dim3((int)std::min<int64_t>(1024, (most + 255) / 256)), dim3(256), 0, n->stream,
+                     st, (int64_t)N, nb);
+  SPK_HIP(hipGetLastError());
   n->st_on = true;
   n->st_pending = true;
   n->st_bin = bin_steps;
@@ -3018,79 +3025,71 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   ALLOC(n->d_ring, (size_t)n->B * NN); ALLOC(n->d_g, NN);
   ALLOC(n->d_decay, 1); ALLOC(n->d_erev, 1); ALLOC(n->d_in_thr, 1);
   ALLOC(n->d_ext_cdf, std::max<size_t>(1, n->ext_cdf.size()));
-  ALLOC(n->d_syn, (size_t)std::max<int64_t>(1, S));
+  // deliveries read the compact records only
   ALLOC(n->d_syn16, (size_t)(std::max<int64_t>(1, S) + 7) / 8 * 8 + 8);   // whole 16-byte chunks
   ALLOC(n->d_stats, 4);
   ALLOC(n->d_nlo, (size_t)P + 1); ALLOC(n->d_ilo, (size_t)P + 1);
   ALLOC(n->d_seg, (size_t)N * (P + 1));
   ALLOC(n->d_xlist, (size_t)2 * 2 * P * spk::fused_xstride(n->xcap));   // 64-bit words
   ALLOC(n->d_bar, (size_t)(spk::kBarGroups + 2) * spk::kBarStride); ALLOC(n->d_err, 1);
-  int* d_owner = nullptr;
-  unsigned int *d_count = nullptr, *d_off = nullptr, *d_cursor = nullptr;
-  ALLOC(d_owner, NN);
-  ALLOC(d_count, NN * P); ALLOC(d_off, NN * P); ALLOC(d_cursor, NN * P);
+  // tiles: about 512 workgroups for the largest LDS form, whole partitions otherwise
+  spk::BrunelGenArgs ga{};
+  ga.seed = n->seed; ga.N = N; ga.ne = p->n_exc; ga.ni = p->n_inh; ga.ce = p->ce; ga.ci = p->ci; ga.P = P;
+  const bool lds_gen = N <= spk::kGenLdsSources;
+  ga.tq = lds_gen ? std::max(1, std::min(n->nown_max, 512 / P)) : 1;
+  ga.ts = (n->nown_max + ga.tq - 1) / ga.tq;
+  ga.tq = (n->nown_max + ga.ts - 1) / ga.ts;
+  const int tiles = P * ga.tq;
+  unsigned int* d_cnt = nullptr;
+  ALLOC(d_cnt, ((size_t)tiles + 1) * NN);
 #undef ALLOC
   hipStream_t st = n->stream;
-  auto cleanup = [&]() { dfree(d_owner); dfree(d_count); dfree(d_off); dfree(d_cursor); };
-  std::vector<int> owner(N);
-  for (int q = 0; q < P; ++q)
-    for (int i = n->h_nlo[q]; i < n->h_nlo[q + 1]; ++i) owner[i] = q;
-  if ((rc = upload(n->d_v0, n->v0.data(), NN, st)) || (rc = upload(n->d_vreset, n->vreset.data(), NN, st)) ||
-      (rc = upload(n->d_thr, n->thr.data(), NN, st)) || (rc = upload(n->d_c, n->c.data(), NN, st)) ||
-      (rc = upload(n->d_rp, n->rp.data(), NN, st)) || (rc = upload(n->d_decay, n->decay_g.data(), 1, st)) ||
-      (rc = upload(n->d_erev, n->erev.data(), 1, st)) ||
-      (rc = upload(n->d_ext_cdf, n->ext_cdf.data(), n->ext_cdf.size(), st)) ||
-      (rc = upload(n->d_nlo, n->h_nlo.data(), (size_t)P + 1, st)) ||
-      (rc = upload(n->d_ilo, n->h_ilo.data(), (size_t)P + 1, st)) || (rc = upload(d_owner, owner.data(), NN, st))) {
-    cleanup();
-    return bail(rc);
-  }
-  SPK_HIP(hipMemsetAsync(n->d_xlist, 0, sizeof(uint64_t) * 2 * P * spk::fused_xstride(n->xcap), st));
-  SPK_HIP(hipMemsetAsync(n->d_err, 0, sizeof(int), st));
-  SPK_HIP(hipMemsetAsync(n->d_stats, 0, sizeof(unsigned long long) * 4, st));
-  SPK_HIP(hipMemsetAsync(d_count, 0, sizeof(unsigned int) * NN * P, st));
-  SPK_HIP(hipMemsetAsync(d_cursor, 0, sizeof(unsigned int) * NN * P, st));
-  spk::BrunelGenArgs ga{};
-  ga.seed = n->seed; ga.ne = p->n_exc; ga.ni = p->n_inh; ga.ce = p->ce; ga.ci = p->ci; ga.P = P;
-  ga.owner = d_owner; ga.nlo = n->d_nlo; ga.count = d_count; ga.off = d_off; ga.cursor = d_cursor;
-  ga.syn = n->d_syn; ga.syn16 = n->d_syn16;
-  ga.delay_bits = (uint32_t)G << 20; ga.we = p->weight_exc; ga.wi = p->weight_inh;
+  auto cleanup = [&]() { dfree(d_cnt); };
+#define GEN_HIP(expr)                                                                                  \
+  do {                                                                                                 \
+    hipError_t e_ = (expr);                                                                            \
+    if (e_ != hipSuccess) {                                                                            \
+      cleanup();                                                                                       \
+      return bail(fail(SPK_ERR_HIP, std::string(#expr) + " failed: " + hipGetErrorString(e_)));        \
+    }                                                                                                  \
+  } while (0)
+  ga.cnt = d_cnt; ga.rowbase = d_cnt + (size_t)tiles * NN; ga.seg = n->d_seg; ga.syn16 = n->d_syn16;
+  spk::BrunelInitArgs ia{};
+  ia.N = N; ia.P = P; ia.ext_k = (int)n->ext_cdf.size();
+  ia.v0 = p->v0; ia.vreset = p->vreset; ia.thr = p->threshold; ia.c = p->decay_c; ia.rp = p->resist;
+  ia.d_v0 = n->d_v0; ia.d_vreset = n->d_vreset; ia.d_thr = n->d_thr; ia.d_c = n->d_c; ia.d_rp = n->d_rp;
+  ia.d_decay = n->d_decay; ia.d_erev = n->d_erev; ia.nlo = n->d_nlo; ia.ilo = n->d_ilo; ia.ext_cdf = n->d_ext_cdf;
+  ia.xlist = (unsigned long long*)n->d_xlist; ia.xwords = (int64_t)2 * P * spk::fused_xstride(n->xcap);
+  ia.stats = n->d_stats; ia.err = n->d_err;
+  std::copy(n->ext_cdf.begin(), n->ext_cdf.end(), ia.cdf);
+  hipLaunchKernelGGL(spk::k_brunel_init, dim3(64), dim3(256), 0, st, ia);
+  GEN_HIP(hipGetLastError());
   // every excitatory source weighs weight_exc, every inhibitory one weight_inh, one delay
   n->compact = S > 0;
   n->cw_lo = p->weight_exc; n->cw_hi = p->weight_inh; n->csplit = p->n_exc; n->cdelay = G;
-  const int grid = (int)std::min<int64_t>(8192, std::max<int64_t>(1, (S + 255) / 256));
-  if (S > 0) {
-    hipLaunchKernelGGL(spk::k_gen_count, dim3(grid), dim3(256), 0, st, ga, S);
-    SPK_HIP(hipGetLastError());
+  const size_t gen_lds = lds_gen ? NN * sizeof(unsigned int) : 0;
+  const void* fcount = lds_gen ? (const void*)spk::k_gen_count<true> : (const void*)spk::k_gen_count<false>;
+  const void* fscatter = lds_gen ? (const void*)spk::k_gen_scatter<true> : (const void*)spk::k_gen_scatter<false>;
+  if (gen_lds > 65536) {
+    GEN_HIP(hipFuncSetAttribute(fcount, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gen_lds));
+    GEN_HIP(hipFuncSetAttribute(fscatter, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gen_lds));
   }
-  // exclusive scan of the key counts: the segment table seg[u][P+1]
-  std::vector<unsigned int> cnt(NN * P), off(NN * P);
-  SPK_HIP(hipMemcpyAsync(cnt.data(), d_count, sizeof(unsigned int) * NN * P, hipMemcpyDeviceToHost, st));
-  SPK_HIP(hipStreamSynchronize(st));
-  std::vector<uint32_t> seg(NN * (P + 1));
-  uint64_t run = 0;
-  for (size_t u = 0; u < NN; ++u) {
-    for (int q = 0; q < P; ++q) {
-      off[u * P + q] = (unsigned int)run;
-      seg[u * (P + 1) + q] = (uint32_t)run;
-      run += cnt[u * P + q];
-    }
-    seg[u * (P + 1) + P] = (uint32_t)run;
-  }
-  if ((rc = upload(d_off, off.data(), NN * P, st)) || (rc = upload(n->d_seg, seg.data(), seg.size(), st))) {
+  void* gargs[] = {&ga};
+  GEN_HIP(hipLaunchKernel(fcount, dim3(tiles), dim3(spk::kGenBlock), gargs, gen_lds, st));
+  hipLaunchKernelGGL(spk::k_gen_rows, dim3((N + spk::kRowsWidth - 1) / spk::kRowsWidth),
+                     dim3(spk::kRowsWidth * spk::kRowsParts), 0, st, ga);
+  hipLaunchKernelGGL(spk::k_gen_rowbase, dim3(1), dim3(1024), 0, st, ga);
+  hipLaunchKernelGGL(spk::k_gen_seg, dim3((int)std::min<int64_t>(2048, ((int64_t)N * (P + 1) + 255) / 256)), dim3(256), 0, st, ga);
+  GEN_HIP(hipGetLastError());
+  if (S > 0) GEN_HIP(hipLaunchKernel(fscatter, dim3(tiles), dim3(spk::kGenBlock), gargs, gen_lds, st));
+  // every neuron has C afferents, so the largest partition's delivery table is known here
+  if ((rc = plan_lds_table(n, (int64_t)n->nown_max * C, N))) {
     cleanup();
     return bail(rc);
   }
-  if ((rc = plan_lds_table(n, seg.data(), N))) {
-    cleanup();
-    return bail(rc);
-  }
-  if (S > 0) {
-    hipLaunchKernelGGL(spk::k_gen_scatter, dim3(grid), dim3(256), 0, st, ga, S);
-    SPK_HIP(hipGetLastError());
-  }
-  SPK_HIP(hipStreamSynchronize(st));
+  GEN_HIP(hipStreamSynchronize(st));
   cleanup();
+#undef GEN_HIP
   int per_cu = 0;
   SPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fused_kernel(n, spk::kRulesOff), spk::kFusedBlock, n->fused_lds));
   if ((int64_t)per_cu * n->cu_count < P) return bail(fail(SPK_ERR_ARG, "partitions exceed co-resident workgroups"));
