@@ -1951,4 +1951,10 @@ __global__ __launch_bounds__(BS, 4) void k_fused_batch(const FusedArgs* __restri
   }
 }
 
+// The networks' error flags after a batch, into (pinned) host memory.
+static __global__ __launch_bounds__(256) void k_gather_errors(const FusedArgs* __restrict__ nets, int n, int* out) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) out[k] = *nets[k].error;
+}
+
 }  // namespace spk

@@ -1506,21 +1506,30 @@ struct StatsOut {
 
 constexpr int kStatsBlock = 1024;
 
-static __device__ double block_sum_f64(double v, double* sh) {
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = kStatsBlock / 2; off > 0; off >>= 1) {
-    if ((int)threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-    __syncthreads();
+// Sums of M values over the workgroup, in a fixed order: within each wavefront, then the
+// wavefronts' sums one after another by every thread.
+template <int M>
+static __device__ __forceinline__ void block_sums_f64(double (&v)[M], double* sh) {
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    for (int off = kWave / 2; off > 0; off >>= 1) v[m] += __shfl_xor(v[m], off);
   }
-  const double r = sh[0];
   __syncthreads();
-  return r;
+  if ((int)threadIdx.x % kWave == 0) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) sh[((int)threadIdx.x / kWave) * M + m] = v[m];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    v[m] = 0.0;
+    for (int w = 0; w < kStatsBlock / kWave; ++w) v[m] += sh[w * M + m];
+  }
 }
 
 static __global__ __launch_bounds__(kStatsBlock) void k_stats_reduce(StatsArgs st, int N, int64_t steps, float dt,
                                                               StatsOut* out) {
-  __shared__ double sh[kStatsBlock];
+  __shared__ double sh[4 * (kStatsBlock / kWave)];
   double spikes = 0.0, cv = 0.0, ncv = 0.0;
   for (int i = threadIdx.x; i < N; i += kStatsBlock) {
     spikes += (double)st.count[i];
@@ -1536,17 +1545,18 @@ static __global__ __launch_bounds__(kStatsBlock) void k_stats_reduce(StatsArgs s
   const int64_t nb = steps > 0 ? (steps + st.bin - 1) / st.bin : 0;
   double hs = 0.0;
   for (int64_t b = threadIdx.x; b < nb; b += kStatsBlock) hs += (double)st.hist[b];
-  const double S = block_sum_f64(spikes, sh);
-  const double CV = block_sum_f64(cv, sh);
-  const double NCV = block_sum_f64(ncv, sh);
-  const double HS = block_sum_f64(hs, sh);
+  double sums[4] = {spikes, cv, ncv, hs};
+  block_sums_f64(sums, sh);
+  const double S = sums[0], CV = sums[1], NCV = sums[2], HS = sums[3];
   const double mean = nb > 0 ? HS / (double)nb : 0.0;
   double hv = 0.0;
   for (int64_t b = threadIdx.x; b < nb; b += kStatsBlock) {
     const double d = (double)st.hist[b] - mean;
     hv += d * d;
   }
-  const double HV = block_sum_f64(hv, sh);
+  double hvs[1] = {hv};
+  block_sums_f64(hvs, sh);
+  const double HV = hvs[0];
   if (threadIdx.x == 0) {
     StatsOut o;
     o.spikes = (long long)S;

@@ -10,6 +10,8 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -51,6 +53,116 @@ template <typename T>
 void dfree(T*& p) {
   if (p) (void)hipFree((void*)p);
   p = nullptr;
+}
+
+// One allocation cut into arrays (each on a 256-byte boundary): a generated network's device
+// memory.  hipFree takes 28 us and hipMalloc 4 us a call, and such a network has 25 arrays.
+struct Slab {
+  char* base = nullptr;
+  size_t bytes = 0;
+  struct Want { void** p; size_t bytes; };
+  std::vector<Want> wants;
+  template <typename T>
+  void want(T** p, size_t n) {
+    *p = nullptr;
+    wants.push_back({(void**)p, (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256});
+  }
+  int allocate() {
+    size_t total = 0;
+    for (auto& w : wants) total += w.bytes;
+    if (int rc = dalloc(&base, total)) return rc;
+    bytes = total;
+    size_t o = 0;
+    for (auto& w : wants) {
+      *w.p = base + o;
+      o += w.bytes;
+    }
+    wants.clear();
+    return SPK_OK;
+  }
+  bool owns(const void* p) const { return base && (const char*)p >= base && (const char*)p < base + bytes; }
+  void release() {
+    dfree(base);
+    bytes = 0;
+  }
+};
+
+// Facts of a device that do not change while the process runs, looked up once (hipGetDeviceCount
+// alone takes 80 us a call).
+struct DeviceFacts {
+  bool gfx950 = false;
+  std::string arch;
+  int cus = 0;
+  size_t lds = 0;
+  std::map<const void*, size_t> static_lds;   // of the persistent kernels
+};
+
+std::mutex g_device_mu;
+std::map<int, DeviceFacts> g_devices;
+
+int device_facts(int dev, DeviceFacts& out) {
+  std::lock_guard<std::mutex> lock(g_device_mu);
+  auto it = g_devices.find(dev);
+  if (it == g_devices.end()) {
+    hipDeviceProp_t prop;
+    SPK_HIP(hipGetDeviceProperties(&prop, dev));
+    DeviceFacts f;
+    f.arch = prop.gcnArchName;
+    f.gfx950 = std::strncmp(prop.gcnArchName, "gfx950", 6) == 0;
+    f.cus = prop.multiProcessorCount;
+    f.lds = prop.sharedMemPerBlock;
+    it = g_devices.emplace(dev, std::move(f)).first;
+  }
+  out.gfx950 = it->second.gfx950;
+  out.arch = it->second.arch;
+  out.cus = it->second.cus;
+  out.lds = it->second.lds;
+  return SPK_OK;
+}
+
+size_t static_lds(int dev, const void* fn) {
+  std::lock_guard<std::mutex> lock(g_device_mu);
+  auto& m = g_devices[dev].static_lds;
+  auto it = m.find(fn);
+  if (it == m.end()) {
+    hipFuncAttributes fa;
+    it = m.emplace(fn, hipFuncGetAttributes(&fa, fn) == hipSuccess ? fa.sharedSizeBytes : 0).first;
+  }
+  return it->second;
+}
+
+// Streams of closed networks and batches, kept for the next ones (creating and destroying one
+// takes 0.34 and 0.44 ms): at most kIdleStreams per device, the rest are destroyed; a stream is
+// handed back only after it has been waited for.
+constexpr size_t kIdleStreams = 64;
+std::mutex g_stream_mu;
+std::map<int, std::vector<hipStream_t>> g_idle_streams;
+
+hipError_t take_stream(int dev, hipStream_t* s) {
+  {
+    std::lock_guard<std::mutex> lock(g_stream_mu);
+    auto& idle = g_idle_streams[dev];
+    if (!idle.empty()) {
+      *s = idle.back();
+      idle.pop_back();
+      return hipSuccess;
+    }
+  }
+  return hipStreamCreateWithFlags(s, hipStreamNonBlocking);
+}
+
+void give_stream(int dev, hipStream_t s) {
+  if (!s) return;
+  const bool good = hipStreamSynchronize(s) == hipSuccess;
+  {
+    std::lock_guard<std::mutex> lock(g_stream_mu);
+    auto& idle = g_idle_streams[dev];
+    if (good && idle.size() < kIdleStreams) {
+      idle.push_back(s);
+      return;
+    }
+  }
+  (void)hipStreamDestroy(s);
 }
 
 // Bernoulli threshold of a Poisson input with rate r: floor((1 - exp(-r*dt)) * 2^32).
@@ -185,6 +297,8 @@ struct spk_network {
   hipStream_t stream = nullptr;
   bool own_stream = false;
   int device = 0;
+  Slab slab;      // arrays of a generated network
+  Slab st_slab;   // per-neuron window statistics
   // host parameters
   std::vector<float> v0, vreset, thr, c, rp;
   float tref = 0.002f, ibg = 0.0f;
@@ -373,6 +487,10 @@ int check_listed(const spk_network* n) {
 }
 
 void free_device(spk_network* n) {
+  auto dfree = [&](auto*& p) {
+    if (p && !n->slab.owns(p) && !n->st_slab.owns(p)) (void)hipFree((void*)p);
+    p = nullptr;
+  };
   dfree(n->d_V); dfree(n->d_v0); dfree(n->d_vreset); dfree(n->d_thr); dfree(n->d_c);
   dfree(n->d_rp); dfree(n->d_last_n); dfree(n->d_last_in); dfree(n->d_hist_n);
   dfree(n->d_hist_in); dfree(n->d_ring); dfree(n->d_g); dfree(n->d_decay); dfree(n->d_erev);
@@ -399,6 +517,8 @@ void free_device(spk_network* n) {
   }
   dfree(n->d_ras_bits); dfree(n->d_ras_time); dfree(n->d_ras_tile); dfree(n->d_ras_ids); dfree(n->d_ras_times);
   dfree(n->d_ras_flag);
+  n->slab.release();
+  n->st_slab.release();
 }
 
 // Groups covering the steps [first, first + count) record into the network's monitors.
@@ -1176,14 +1296,11 @@ const void* fused_kernel(const spk_network* n, int rules) {
 // with its own scan scratch).  Without it a partition sized just under the limit would
 // leave the grid no co-resident workgroup.
 size_t fused_lds_limit(const spk_network* n) {
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, n->device) != hipSuccess) return 0;
+  DeviceFacts dev;
+  if (device_facts(n->device, dev) != SPK_OK) return 0;
   size_t st = 0;
-  for (int rules : {spk::kRulesOff, spk::kRulesDense}) {
-    hipFuncAttributes fa;
-    if (hipFuncGetAttributes(&fa, fused_kernel(n, rules)) == hipSuccess) st = std::max(st, fa.sharedSizeBytes);
-  }
-  const size_t lim = (size_t)prop.sharedMemPerBlock;
+  for (int rules : {spk::kRulesOff, spk::kRulesDense}) st = std::max(st, static_lds(n->device, fused_kernel(n, rules)));
+  const size_t lim = dev.lds;
   return lim > st + 512 ? lim - st - 512 : 0;
 }
 
@@ -1521,15 +1638,11 @@ int spk_create(int n_neurons, int n_inputs, int synapse_kind, int n_labels, floa
   if (n_labels < 1 || n_labels > spk::kMaxLabels)
     return fail(SPK_ERR_ARG, "n_labels must be in [1, 8]");
   if (!(timestep > 0.0f)) return fail(SPK_ERR_ARG, "timestep must be > 0");
-  int ndev = 0;
-  if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
-    return fail(SPK_ERR_NODEVICE, "no HIP device visible");
   int dev = 0;
-  SPK_HIP(hipGetDevice(&dev));
-  hipDeviceProp_t prop;
-  SPK_HIP(hipGetDeviceProperties(&prop, dev));
-  if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0)
-    return fail(SPK_ERR_NODEVICE, std::string("device is ") + prop.gcnArchName + ", need gfx950");
+  if (hipGetDevice(&dev) != hipSuccess) return fail(SPK_ERR_NODEVICE, "no HIP device visible");
+  DeviceFacts facts;
+  if (int rc = device_facts(dev, facts)) return rc;
+  if (!facts.gfx950) return fail(SPK_ERR_NODEVICE, "device is " + facts.arch + ", need gfx950");
   spk_network* n = new spk_network();
   n->N = n_neurons;
   n->Nin = n_inputs;
@@ -1539,7 +1652,7 @@ int spk_create(int n_neurons, int n_inputs, int synapse_kind, int n_labels, floa
   n->device = dev;
   n->decay_g.assign(n_labels, 1.0f);
   n->erev.assign(n_labels, 0.0f);
-  hipError_t e = hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking);
+  hipError_t e = take_stream(dev, &n->stream);
   if (e != hipSuccess) {
     delete n;
     return fail(SPK_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e));
@@ -1558,7 +1671,7 @@ int spk_destroy(spk_network* n) {
   if (n->ev_a) (void)hipEventDestroy(n->ev_a);
   if (n->ev_b) (void)hipEventDestroy(n->ev_b);
   for (auto e : n->ev_kernel) (void)hipEventDestroy(e);
-  if (n->own_stream && n->stream) (void)hipStreamDestroy(n->stream);
+  if (n->own_stream) give_stream(n->device, n->stream);
   delete n;
   return SPK_OK;
 }
@@ -1567,7 +1680,7 @@ int spk_set_stream(spk_network* n, void* s) {
   if (int rc = check_net(n)) return rc;
   SPK_HIP(hipStreamSynchronize(n->stream));
   if (!s) return SPK_OK;
-  if (n->own_stream) (void)hipStreamDestroy(n->stream);
+  if (n->own_stream) give_stream(n->device, n->stream);
   n->stream = (hipStream_t)s;
   n->own_stream = false;
   return SPK_OK;
@@ -2119,10 +2232,9 @@ int spk_prepare(spk_network* n, int G) {
   n->q_ext = n->ext_cdf.empty() ? 0 : (int64_t)std::llrint(std::ldexp((double)n->ext_w, n->frac));
   // ---- partitions of the persistent kernel: contiguous neuron / input ranges ----
   {
-    int dev_cu = 0;
-    hipDeviceProp_t prop;
-    SPK_HIP(hipGetDeviceProperties(&prop, n->device));
-    dev_cu = prop.multiProcessorCount;
+    DeviceFacts facts;
+    if (int rc = device_facts(n->device, facts)) return rc;
+    const int dev_cu = facts.cus;
     n->cu_count = dev_cu;
     int P = n->req_partitions > 0 ? n->req_partitions : std::min(dev_cu, std::max(1, (n->N + 7) / 8));
     P = std::max(1, std::min(P, std::max(1, n->N)));
@@ -2681,10 +2793,13 @@ int spk_stats_begin(spk_network* n, int bin_steps, int64_t max_steps) {
   if (nb > ((int64_t)1 << 31)) return fail(SPK_ERR_ARG, "statistics window too long");
   const size_t N = (size_t)std::max(1, n->N);
   if (!n->d_st_cnt) {
-    int rc;
-    if ((rc = dalloc(&n->d_st_cnt, N)) || (rc = dalloc(&n->d_st_nisi, N)) || (rc = dalloc(&n->d_st_prev, N)) ||
-        (rc = dalloc(&n->d_st_s1, N)) || (rc = dalloc(&n->d_st_s2, N)) || (rc = dalloc(&n->d_st_out, 1)))
-      return rc;
+    n->st_slab.want(&n->d_st_cnt, N);
+    n->st_slab.want(&n->d_st_nisi, N);
+    n->st_slab.want(&n->d_st_prev, N);
+    n->st_slab.want(&n->d_st_s1, N);
+    n->st_slab.want(&n->d_st_s2, N);
+    n->st_slab.want(&n->d_st_out, 1);
+    if (int rc = n->st_slab.allocate()) return rc;
   }
   if (nb > n->st_nbins) {
     dfree(n->d_st_hist);
@@ -2991,9 +3106,9 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   if (!n->ext_cdf.empty()) mx += (double)n->ext_cdf.size() * std::fabs((double)n->ext_w);
   n->frac = choose_frac_bits(mx);
   n->q_ext = n->ext_cdf.empty() ? 0 : (int64_t)std::llrint(std::ldexp((double)n->ext_w, n->frac));
-  hipDeviceProp_t prop;
-  SPK_HIP(hipGetDeviceProperties(&prop, n->device));
-  n->cu_count = prop.multiProcessorCount;
+  DeviceFacts facts;
+  if (int rc = device_facts(n->device, facts)) return bail(rc);
+  n->cu_count = facts.cus;
   int P = partitions > 0 ? partitions : std::min(n->cu_count, std::max(1, (N + 7) / 8));
   P = std::max(1, std::min(P, N));
   n->P = P;
@@ -3018,7 +3133,7 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   n->slots = 1;
   int rc;
   const size_t NN = (size_t)N;
-#define ALLOC(ptr, cnt) if ((rc = dalloc(&(ptr), (cnt)))) return bail(rc)
+#define ALLOC(ptr, cnt) n->slab.want(&(ptr), (cnt))
   ALLOC(n->d_V, NN); ALLOC(n->d_v0, NN); ALLOC(n->d_vreset, NN); ALLOC(n->d_thr, NN);
   ALLOC(n->d_c, NN); ALLOC(n->d_rp, NN); ALLOC(n->d_last_n, NN); ALLOC(n->d_last_in, 1);
   ALLOC(n->d_hist_n, (size_t)n->W * NN); ALLOC(n->d_hist_in, 1);
@@ -3032,6 +3147,8 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   ALLOC(n->d_seg, (size_t)N * (P + 1));
   ALLOC(n->d_xlist, (size_t)2 * 2 * P * spk::fused_xstride(n->xcap));   // 64-bit words
   ALLOC(n->d_bar, (size_t)(spk::kBarGroups + 2) * spk::kBarStride); ALLOC(n->d_err, 1);
+#undef ALLOC
+  if ((rc = n->slab.allocate())) return bail(rc);
   // tiles: about 512 workgroups for the largest LDS form, whole partitions otherwise
   spk::BrunelGenArgs ga{};
   ga.seed = n->seed; ga.N = N; ga.ne = p->n_exc; ga.ni = p->n_inh; ga.ce = p->ce; ga.ci = p->ci; ga.P = P;
@@ -3041,8 +3158,7 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   ga.tq = (n->nown_max + ga.ts - 1) / ga.ts;
   const int tiles = P * ga.tq;
   unsigned int* d_cnt = nullptr;
-  ALLOC(d_cnt, ((size_t)tiles + 1) * NN);
-#undef ALLOC
+  if ((rc = dalloc(&d_cnt, ((size_t)tiles + 1) * NN))) return bail(rc);
   hipStream_t st = n->stream;
   auto cleanup = [&]() { dfree(d_cnt); };
 #define GEN_HIP(expr)                                                                                  \
@@ -3114,6 +3230,7 @@ struct spk_batch {
   size_t lds = 0;
   bool lds_tables = true;     // networks keep their delivery tables in LDS where planned
   hipStream_t stream = nullptr;
+  int device = 0;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   spk::FusedArgs* d_args = nullptr;
   int2* d_tasks = nullptr;
@@ -3136,6 +3253,7 @@ struct spk_batch {
   int2* h_tasks = nullptr;
   size_t h_tasks_cap = 0;
   int* h_off = nullptr;
+  int* h_err = nullptr;   // [networks] error flags of the last run (pinned, written by the device)
   int64_t captures = 0, replays = 0;
 };
 
@@ -3207,6 +3325,7 @@ int spk_batch_create(spk_network* const* nets, int n_nets, int workgroups, spk_b
       per_cu = per_cu_s;
     }
   }
+  b->device = nets[0]->device;
   const int cap = per_cu * nets[0]->cu_count;
   b->nb = workgroups > 0 ? std::min(workgroups, cap) : cap;
   int pmax = 0;
@@ -3215,7 +3334,7 @@ int spk_batch_create(spk_network* const* nets, int n_nets, int workgroups, spk_b
     delete b;
     return fail(SPK_ERR_ARG, "a network has more partitions than the batch has co-resident workgroups");
   }
-  if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) { delete b; return fail(SPK_ERR_HIP, "hipStreamCreate"); }
+  if (take_stream(nets[0]->device, &b->stream) != hipSuccess) { delete b; return fail(SPK_ERR_HIP, "hipStreamCreate"); }
   (void)hipEventCreate(&b->e0);
   (void)hipEventCreate(&b->e1);
   if (int rc = dalloc(&b->d_args, b->nets.size())) { delete b; return rc; }
@@ -3230,12 +3349,13 @@ int spk_batch_destroy(spk_batch* b) {
   if (b->h_args) (void)hipHostFree(b->h_args);
   if (b->h_tasks) (void)hipHostFree(b->h_tasks);
   if (b->h_off) (void)hipHostFree(b->h_off);
+  if (b->h_err) (void)hipHostFree(b->h_err);
   dfree(b->d_args);
   dfree(b->d_tasks);
   dfree(b->d_off);
   if (b->e0) (void)hipEventDestroy(b->e0);
   if (b->e1) (void)hipEventDestroy(b->e1);
-  if (b->stream) (void)hipStreamDestroy(b->stream);
+  give_stream(b->device, b->stream);
   delete b;
   return SPK_OK;
 }
@@ -3328,6 +3448,7 @@ int spk_batch_run(spk_batch* b, const float* starts, const int64_t* ngroups, int
   }
   // this run's arguments in pinned staging buffers: the copies read them when they execute
   if (!b->h_args) SPK_HIP(hipHostMalloc((void**)&b->h_args, sizeof(spk::FusedArgs) * (size_t)K));
+  if (!b->h_err) SPK_HIP(hipHostMalloc((void**)&b->h_err, sizeof(int) * (size_t)K));
   if (!b->h_off) SPK_HIP(hipHostMalloc((void**)&b->h_off, sizeof(int) * ((size_t)b->nb + 1)));
   if (tasks.size() > b->h_tasks_cap) {
     if (b->h_tasks) SPK_HIP(hipHostFree(b->h_tasks));
@@ -3380,7 +3501,10 @@ int spk_batch_run(spk_batch* b, const float* starts, const int64_t* ngroups, int
     if (e != hipSuccess) return fail(SPK_ERR_HIP, std::string("batch launch: ") + hipGetErrorString(e));
   }
   SPK_HIP(hipEventRecord(b->e1, b->stream));
-  SPK_HIP(hipEventSynchronize(b->e1));
+  // every network's error flag into one host array (a copy per network: 14 us each)
+  hipLaunchKernelGGL(spk::k_gather_errors, dim3((K + 255) / 256), dim3(256), 0, b->stream, b->d_args, K, b->h_err);
+  SPK_HIP(hipGetLastError());
+  SPK_HIP(hipStreamSynchronize(b->stream));
   float ms = 0.0f;
   SPK_HIP(hipEventElapsedTime(&ms, b->e0, b->e1));
   b->last_ms = ms;
@@ -3393,9 +3517,9 @@ int spk_batch_run(spk_batch* b, const float* starts, const int64_t* ngroups, int
     for (int i = 0; i < spk::kProfPhases; ++i)
       n->prof_us[i] = rate_khz > 0 ? (double)ticks[i] * 1e3 / (double)rate_khz : 0.0;
   }
-  for (auto* n : b->nets) {
-    int err = 0;
-    SPK_HIP(hipMemcpy(&err, n->d_err, sizeof(int), hipMemcpyDeviceToHost));
+  for (int k = 0; k < K; ++k) {
+    spk_network* n = b->nets[k];
+    const int err = b->h_err[k];
     if (err) {
       n->bar_clear = true;
       if (err == 2) return fail(SPK_ERR_CAPACITY, "batched persistent kernel: spikes of a group exceeded the exchange list");
