@@ -1454,6 +1454,29 @@ static __global__ __launch_bounds__(kRasterBlock) void k_raster_emit(RasterArgs 
 }
 
 // ---------------------------------------------------------------------------------
+// Weights between the caller's order and the CSR's (pos[s]: CSR position of caller synapse s;
+// nullptr: the same order), so that 4 bytes per synapse cross the bus, in the order they are
+// used in, instead of the CSR's 8-byte records that the host then picks from.
+template <typename I>
+__global__ __launch_bounds__(256) void k_weights_out(Weights W, const I* __restrict__ pos, int64_t S,
+                                                     float* __restrict__ out) {
+  for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < S; s += (int64_t)gridDim.x * blockDim.x)
+    out[s] = wload(W, pos ? (int64_t)pos[s] : s);
+}
+
+// The records' weights and, for 16-bit storage, the words (compensations cleared).
+template <typename I>
+__global__ __launch_bounds__(256) void k_weights_in(Weights W, const I* __restrict__ pos, int64_t S,
+                                                    const float* __restrict__ in) {
+  for (int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; s < S; s += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t k = pos ? (int64_t)pos[s] : s;
+    const float w = in[s];
+    W.w[(size_t)k * kWStride] = w;
+    if (W.fmt) W.wc[k] = enc16(w, W.fmt);
+  }
+}
+
+// ---------------------------------------------------------------------------------
 // The dynamic state of SpikingModel::reset_state (SpikingModel.cpp:181-190) and the window
 // statistics' start, each in one launch of 3 us that nothing waits for (a copy or fill per array
 // and a wait before: 33 us a reset).

@@ -365,6 +365,12 @@ struct spk_network {
   uint32_t* d_wc = nullptr;   // per synapse: 16-bit weight | compensation << 16
   float cw_lo = 0.0f, cw_hi = 0.0f;
   int csplit = 0, cdelay = 0;
+  // CSR position of each caller synapse (none for generated synapses: the same order);
+  // 64-bit from 2^32 synapses on
+  uint32_t* d_pos = nullptr;
+  int64_t* d_pos64 = nullptr;
+  float* d_wstage = nullptr;  // caller weights on their way in or out, wstage_n at a time
+  int64_t wstage_n = 0;
   float* d_scale = nullptr;
   uint16_t* d_delay = nullptr;
   uint8_t* d_label = nullptr;
@@ -516,7 +522,7 @@ void free_device(spk_network* n) {
     dfree(m.d_ids); dfree(m.d_times); dfree(m.d_count);
   }
   dfree(n->d_ras_bits); dfree(n->d_ras_time); dfree(n->d_ras_tile); dfree(n->d_ras_ids); dfree(n->d_ras_times);
-  dfree(n->d_ras_flag);
+  dfree(n->d_ras_flag); dfree(n->d_pos); dfree(n->d_pos64); dfree(n->d_wstage);
   n->slab.release();
   n->st_slab.release();
 }
@@ -712,9 +718,6 @@ int build_wd_mask(spk_network* n) {
   SPK_HIP(hipGetLastError());
   return SPK_OK;
 }
-
-// CSR position of caller synapse s (the identity for generated fixed out-degree synapses).
-inline int64_t csr_pos(const spk_network* n, int64_t s) { return n->od ? s : n->perm[(size_t)s]; }
 
 int check_time(spk_network* n, float t) {
   if (!(t >= n->t_hi - 0.5f * n->dt))
@@ -1101,6 +1104,34 @@ int launch_group_phases(spk_network* n, float t, bool plastic) {
   if ((rc = launch_propagate(n, t, n->cur_slot))) return rc;
   for (int m = 0; m < (int)n->mons.size(); ++m)
     if ((rc = launch_collect(n, m, n->cur_slot, 1))) return rc;
+  return SPK_OK;
+}
+
+// Staging buffer of spk_get_weights / spk_set_weights (64 MB at most).
+constexpr int64_t kWeightPiece = (int64_t)1 << 24;
+int weight_staging(spk_network* n) {
+  if (n->d_wstage) return SPK_OK;
+  const int64_t cnt = std::min<int64_t>(n->S, kWeightPiece);
+  if (int rc = dalloc(&n->d_wstage, (size_t)cnt)) return rc;
+  n->wstage_n = cnt;
+  return SPK_OK;
+}
+
+// Caller synapses [s0, s0 + cnt) from the CSR into the staging buffer (`out`) or back.
+int launch_weights(spk_network* n, int64_t s0, int64_t cnt, bool out) {
+  spk::Weights w = weights_of(n);
+  if (n->od) {   // the CSR's order is the caller's
+    w.w += (size_t)s0 * spk::kWStride;
+    if (w.wc) w.wc += s0;
+  }
+  const uint32_t* p32 = n->d_pos ? n->d_pos + s0 : nullptr;
+  const int64_t* p64 = n->d_pos64 ? n->d_pos64 + s0 : nullptr;
+  const dim3 grid((int)std::min<int64_t>(4096, (cnt + 255) / 256)), block(256);
+  if (out && p64) hipLaunchKernelGGL(spk::k_weights_out<int64_t>, grid, block, 0, n->stream, w, p64, cnt, n->d_wstage);
+  else if (out) hipLaunchKernelGGL(spk::k_weights_out<uint32_t>, grid, block, 0, n->stream, w, p32, cnt, n->d_wstage);
+  else if (p64) hipLaunchKernelGGL(spk::k_weights_in<int64_t>, grid, block, 0, n->stream, w, p64, cnt, n->d_wstage);
+  else hipLaunchKernelGGL(spk::k_weights_in<uint32_t>, grid, block, 0, n->stream, w, p32, cnt, n->d_wstage);
+  SPK_HIP(hipGetLastError());
   return SPK_OK;
 }
 
@@ -2435,6 +2466,17 @@ int spk_prepare(spk_network* n, int G) {
     });
     if ((rc = upload(n->d_syn, rec.data(), S, st))) return rc;
   }
+  if (S >= ((int64_t)1 << 32)) {
+    if ((rc = dalloc(&n->d_pos64, S))) return rc;
+    if ((rc = upload(n->d_pos64, n->perm.data(), S, st))) return rc;
+  } else {
+    hvec<uint32_t> pos(S);
+    host_chunks(S, T, [&](int, int64_t a, int64_t b) {
+      for (int64_t k = a; k < b; ++k) pos[k] = (uint32_t)n->perm[k];
+    });
+    if ((rc = dalloc(&n->d_pos, S))) return rc;
+    if ((rc = upload(n->d_pos, pos.data(), S, st))) return rc;
+  }
   if (n->wfmt != SPK_WEIGHTS_FP32) {
     // 16-bit weights of the records' weights, compensations zero
     hvec<uint32_t> wc(S);
@@ -2940,33 +2982,27 @@ int spk_monitor_take(spk_network* n, int mid, int32_t* ids, float* times, int64_
 int spk_get_weights(spk_network* n, float* out) {
   if (int rc = check_listed(n)) return rc;
   if (!out && n->S) return fail(SPK_ERR_ARG, "null output");
-  if (n->wfmt != SPK_WEIGHTS_FP32) {
-    std::vector<uint32_t> wc(n->S);
-    if (n->S) SPK_HIP(hipMemcpyAsync(wc.data(), n->d_wc, n->S * sizeof(uint32_t), hipMemcpyDeviceToHost, n->stream));
-    SPK_HIP(hipStreamSynchronize(n->stream));
-    for (int64_t s = 0; s < n->S; ++s) out[s] = spk::dec16((uint16_t)(wc[csr_pos(n, s)] & 0xFFFFu), n->wfmt);
-    return SPK_OK;
+  if (n->S == 0) return SPK_OK;
+  if (int rc = weight_staging(n)) return rc;
+  for (int64_t s0 = 0; s0 < n->S; s0 += n->wstage_n) {
+    const int64_t cnt = std::min(n->wstage_n, n->S - s0);
+    if (int rc = launch_weights(n, s0, cnt, true)) return rc;
+    SPK_HIP(hipMemcpyAsync(out + s0, n->d_wstage, cnt * sizeof(float), hipMemcpyDeviceToHost, n->stream));
   }
-  std::vector<uint2> rec(n->S);
-  if (n->S) SPK_HIP(hipMemcpyAsync(rec.data(), n->d_syn, n->S * sizeof(uint2), hipMemcpyDeviceToHost, n->stream));
   SPK_HIP(hipStreamSynchronize(n->stream));
-  for (int64_t s = 0; s < n->S; ++s) std::memcpy(&out[s], &rec[csr_pos(n, s)].y, sizeof(float));
   return SPK_OK;
 }
 
 int spk_set_weights(spk_network* n, const float* in) {
   if (int rc = check_listed(n)) return rc;
   if (!in && n->S) return fail(SPK_ERR_ARG, "null input");
-  std::vector<uint2> rec(n->S);
-  if (n->S) SPK_HIP(hipMemcpyAsync(rec.data(), n->d_syn, n->S * sizeof(uint2), hipMemcpyDeviceToHost, n->stream));
-  SPK_HIP(hipStreamSynchronize(n->stream));
-  for (int64_t s = 0; s < n->S; ++s) std::memcpy(&rec[csr_pos(n, s)].y, &in[s], sizeof(float));
-  if (n->S) SPK_HIP(hipMemcpyAsync(n->d_syn, rec.data(), n->S * sizeof(uint2), hipMemcpyHostToDevice, n->stream));
-  if (n->wfmt != SPK_WEIGHTS_FP32 && n->S) {
-    // the 16-bit words of the caller's weights; compensations start again from zero
-    std::vector<uint32_t> wc(n->S);
-    for (int64_t s = 0; s < n->S; ++s) wc[csr_pos(n, s)] = spk::enc16(in[s], n->wfmt);
-    SPK_HIP(hipMemcpyAsync(n->d_wc, wc.data(), n->S * sizeof(uint32_t), hipMemcpyHostToDevice, n->stream));
+  if (n->S) {
+    if (int rc = weight_staging(n)) return rc;
+  }
+  for (int64_t s0 = 0; s0 < n->S; s0 += n->wstage_n) {
+    const int64_t cnt = std::min(n->wstage_n, n->S - s0);
+    SPK_HIP(hipMemcpyAsync(n->d_wstage, in + s0, cnt * sizeof(float), hipMemcpyHostToDevice, n->stream));
+    if (int rc = launch_weights(n, s0, cnt, false)) return rc;
   }
   SPK_HIP(hipStreamSynchronize(n->stream));
   n->compact = false;   // caller weights: deliveries read the full records from now on

@@ -55,3 +55,23 @@ def test_rules(rule, dmin):
     p = builders.wd_params(w_max=4e-3) if rule == RULE_WD else builders.vogels_params(lr=1e-5)
     d.rules.append(Rule(rule, syn, p))
     _check(d, 120)
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("p", [0.0, 0.002, 0.21])
+def test_weights_out_and_in(fmt, p):
+    """Weights read and set in the caller's (shuffled) order, no synapses included."""
+    d = builders.random_net(n_neurons=77, n_inputs=19, p=p, seed=3, whi=1.0, monitors=())
+    o = np.random.default_rng(5).permutation(d.n_synapses)
+    d.pre, d.post, d.weight, d.delay = d.pre[o], d.post[o], d.weight[o], d.delay[o]
+    d.weight_format = fmt
+    d.grouping = 1
+    gpu = abi.Network(d)
+    if fmt:
+        d0 = gpu.weights()
+        assert np.all(np.abs(d0 - d.weight) <= 0.004 * d.weight + 1e-7)   # half a step of 8 bits
+    else:
+        assert np.array_equal(gpu.weights(), d.weight)
+    w = (np.arange(d.n_synapses) % 128 - 64).astype(np.float32)           # exact in every format
+    gpu.set_weights(w)
+    assert np.array_equal(gpu.weights(), w)
