@@ -60,27 +60,36 @@ struct FusedRule {
 };
 
 // How a persistent kernel applies plasticity: not at all, per synapse behind a grid barrier
-// (any rules), or driven by spikes (one weight-dependent rule; no grid barrier).
-enum { kRulesOff = 0, kRulesDense = 1, kRulesEvents = 2 };
+// (any rules), or driven by spikes (one rule; no grid barrier) -- the weight-dependent rule, or
+// one of the rules that see delayed presynaptic spikes when all its delays equal the group.
+enum { kRulesOff = 0, kRulesDense = 1, kRulesEvents = 2, kRulesDelayed = 3 };
 
-// The weight-dependent rule driven by spikes (kRulesEvents; the per-phase form of kernels.hpp,
-// k_wd_neurons and k_wd_events, inside the group loop).  Every workgroup keeps the presynaptic
-// trace of every source the rule may have in LDS and advances all of them each group: a
-// source's trace depends only on its own spikes, which every workgroup receives through the
-// exchange, so no workgroup reads another's state and no grid barrier is needed.  Weights are
-// touched only by the workgroup that owns their target.  Bound by the exchange's latency: 6000
-// neurons x 500 synapses (3.1e6, delays from one step) take 5.1 us per group; per synapse, with
-// the barrier's cache write-backs, 51 us.
+// A rule driven by spikes inside the group loop.  A source's trace depends only on its own
+// spikes, which every workgroup receives through the exchange: every workgroup keeps the
+// presynaptic trace of every source in LDS and advances all of them each group, so that no
+// workgroup reads another's state and no grid barrier is needed.  A weight moves only when its
+// source or its target has a spike in the group; it is touched only by the workgroup that owns
+// its target.  Bound by the exchange's latency: weight-dependent rule, 6000 neurons x 500
+// synapses (3.1e6, delays from one step) 5.1 us per group; per synapse, with the barrier's cache
+// write-backs, 51 us.
+//   kRulesEvents   the weight-dependent rule (the per-phase form of kernels.hpp, k_wd_neurons
+//                  and k_wd_events): this group's spikes of the sources, after the exchange;
+//   kRulesDelayed  Vogels, Evans, Custom (DelayedRule): with all delays equal to the group's
+//                  length the spikes that arrive in a group are those of the group before, kept
+//                  as a mask per source, so the rule runs while this group's lists travel.
 struct EventRule {
   Traces tr;               // stored traces per neuron: a [sources], b [N]
   Weights wts;
-  const float* tab;        // wd_weight's table, `ntab` floats
+  const float* tab;        // the rule's table, `ntab` floats
   const uint32_t* mask;    // bit k: CSR position k belongs to the rule
   const int64_t* post_ptr; // the rule's synapses onto neuron v: positions and sources
   const uint32_t* post_pos;
   const int32_t* post_pre;
-  int sources;             // N, or N + Nin when inputs have rule synapses
-  int ntab, nearest;
+  double dterm;
+  int src0, sources;       // units [src0, src0 + sources): kRulesEvents from 0 to N, or to
+                           // N + Nin when inputs have rule synapses; kRulesDelayed from the
+                           // first to the last unit with rule synapses
+  int ntab, nearest, kind;
 };
 
 struct FusedArgs {
@@ -198,7 +207,7 @@ struct PhaseClock {
 // spike masks take 64-bit LDS atomics, which need 8-byte aligned addresses).
 struct FusedLayout {
   size_t ring, hist, ext, imask, inp, xbuf, head, scan, ent, counter, st_cnt, st_nisi, st_prev, st_s1,
-      st_s2, st_g, cdf, guide, lseg, lrec, ev_x, ev_bits, ev_xq, ev_qg, ev_list, ev_tab, total;
+      st_s2, st_g, cdf, guide, lseg, lrec, ev_x, ev_bits, ev_xq, ev_qg, ev_list, ev_tab, ev_src, ev_ptr, total;
 };
 
 constexpr int kHeadWords = 12;         // words of a source block fetched in the first trip
@@ -214,7 +223,7 @@ __host__ __device__ inline size_t align16(size_t x) { return (x + 15) & ~(size_t
 // table is read from global memory).
 __host__ __device__ inline FusedLayout fused_layout(int BL, int L, int W, int G, int nown, int iown,
                                                     int xcap, int P, int segU = 0, int lrec = 0, int cring = 0,
-                                                    int dahead = 1, int ev_src = 0) {
+                                                    int dahead = 1, int ev_src = 0, bool delayed = false) {
   FusedLayout f;
   size_t o = 0;
   f.ring = o;    o = align16(o + (size_t)BL * nown * L * (cring ? 4 : 8));
@@ -240,22 +249,25 @@ __host__ __device__ inline FusedLayout fused_layout(int BL, int L, int W, int G,
   f.guide = o;   o = align16(o + 256);                          // guide table of the thresholds
   f.lseg = o;    o = align16(o + (segU ? (size_t)(segU + 1) * 2 : 0));   // local starts
   f.lrec = o;    o = align16(o + (size_t)lrec * 2);             // this partition's targets
-  // kRulesEvents: presynaptic traces of `ev_src` sources and a bit per source that spiked in
-  // the group, traces and spike steps of the owned neurons, the spiking ones, the rule's table
+  // rules driven by spikes: presynaptic traces of `ev_src` sources; a bit per source that spiked
+  // in the group (kRulesDelayed: a mask per source and group parity, and a list of sources whose
+  // spikes arrive); traces and spikes of the owned neurons, the spiking ones, the rule's table
   f.ev_x = o;    o = align16(o + (size_t)ev_src * 4);
-  f.ev_bits = o; o = align16(o + (size_t)(ev_src + 31) / 32 * 4);
+  f.ev_bits = o; o = align16(o + (delayed ? (size_t)ev_src * 8 : (size_t)(ev_src + 31) / 32 * 4));
   f.ev_xq = o;   o = align16(o + (ev_src ? (size_t)nown * 4 : 0));
   f.ev_qg = o;   o = align16(o + (ev_src ? (size_t)nown * 4 : 0));
   f.ev_list = o; o = align16(o + (ev_src ? (size_t)nown * 4 : 0));
   f.ev_tab = o;  o = align16(o + (ev_src ? (size_t)(5 + 4 * (G + 1)) * 4 : 0));
+  f.ev_src = o;  o = align16(o + (delayed ? (size_t)ev_src * 2 + 16 : 0));   // count, then 16-bit ids
+  f.ev_ptr = o;  o = align16(o + (delayed ? (size_t)(nown + 1) * 4 : 0));
   f.total = o;
   return f;
 }
 
 __host__ __device__ inline size_t fused_lds_bytes(int BL, int L, int W, int G, int nown, int iown,
                                                   int xcap, int P, int segU = 0, int lrec = 0, int cring = 0,
-                                                  int dahead = 1, int ev_src = 0) {
-  return fused_layout(BL, L, W, G, nown, iown, xcap, P, segU, lrec, cring, dahead, ev_src).total;
+                                                  int dahead = 1, int ev_src = 0, bool delayed = false) {
+  return fused_layout(BL, L, W, G, nown, iown, xcap, P, segU, lrec, cring, dahead, ev_src, delayed).total;
 }
 
 __host__ __device__ inline int fused_xstride(int xcap) { return ((1 + xcap + 7) / 8) * 8; }
@@ -746,14 +758,19 @@ constexpr int kQuadEnt = 8;   // entries of one source a quad stages in LDS at a
 // memory (a kernel holding only the form it runs keeps its registers for it).
 enum { kDeliverAny = 0, kDeliverLdsTable = 1, kDeliverCompact = 2, kDeliverCompactAny = 3 };
 
-// LDS state of the spike-driven rule (kRulesEvents) and the group's start time.
+// LDS state of the spike-driven rule and the group's start time.
 struct EventLds {
-  float* x;              // presynaptic traces, decayed for this group
-  uint32_t* bits;        // sources that spiked in the group
-  float* xq;             // postsynaptic traces of the owned neurons
-  int* qg;               // steps of their last spikes within the group (negative: before it)
+  float* x;              // presynaptic traces (kRulesEvents: decayed for this group)
+  uint32_t* bits;        // kRulesEvents: sources that spiked in the group
+  uint32_t* em;          // kRulesDelayed: [2][sources] spikes of a group (bit g), by its parity
+  float* xq;             // postsynaptic traces of the owned neurons at the group's start
+  int* qg;               // steps of their last spikes within the group (negative: before it);
+                         // kRulesDelayed: their spikes of the group (bit g)
   int* list;             // owned neurons that spiked
   float* tab;
+  uint32_t* ptr;         // kRulesDelayed: the owned neurons' starts in the target lists
+  int* nsrc;             // kRulesDelayed: sources whose spikes arrive in the group
+  uint16_t* src;
   float t;
 };
 
@@ -846,6 +863,77 @@ __device__ __forceinline__ void event_targets(const FusedArgs& a, const EventLds
   }
 }
 
+// One synapse under a delayed rule: the group's sub-steps from both sides' traces at its start
+// and their spikes.
+__device__ __forceinline__ void delayed_update(const FusedArgs& a, const DelayedRule& rule, int64_t k, float w0,
+                                               uint16_t c16, float xa, float xb, uint32_t am, uint32_t sm) {
+  float w = w0;
+  for (int g = 0; g < a.G; ++g) rule.step(w, xa, xb, (am >> g) & 1u, (sm >> g) & 1u);
+  wupdate_c(a.ev.wts, k, w0, c16, w, 0.0f, rule.hi());
+}
+
+// The delayed rule's group: the synapses of the sources whose spikes arrive (list ev.src), a
+// quad each from the first wavefront on, and beside them those onto the owned neurons that
+// spiked, except from these sources, a team of whole wavefronts each from the last one on;
+// afterwards the sources' traces advance and their masks are cleared for the next group but
+// one.  Bound by dependent loads (segment or target list, record, weight): all that do not
+// depend on each other are issued together.  COBA network (4000 neurons, 51000 rule synapses):
+// 3.3 us per group (6.9 with every unit as a source, the target pass in the same wavefronts and
+// loads behind the mask's branch); per synapse 8.1 us behind a grid barrier of 4.3 us.
+template <int BS>
+__device__ __forceinline__ void delayed_group(const FusedArgs& a, const EventLds& ev, int p, int par, int nlist) {
+  const DelayedRule rule{a.ev.kind, a.ev.nearest, ev.tab, a.ev.dterm};
+  uint32_t* am = ev.em + (size_t)(par ^ 1) * a.ev.sources;
+  for (int u = threadIdx.x; u < a.ev.sources; u += BS)
+    if (am[u]) ev.src[atomicAdd(ev.nsrc, 1)] = (uint16_t)u;
+  __syncthreads();
+  const uint32_t* synw = (const uint32_t*)a.syn;
+  const int ns = *ev.nsrc, q = (int)threadIdx.x % kQuad;
+  for (int j = (int)threadIdx.x / kQuad; j < ns; j += BS / kQuad) {
+    const int u = ev.src[j];
+    const size_t sb = (size_t)(a.ev.src0 + u) * (a.P + 1) + p;
+    const uint32_t s1 = a.seg[sb + 1];
+    for (uint32_t k = a.seg[sb] + (uint32_t)q; k < s1; k += kQuad) {
+      const uint32_t mw = a.ev.mask[k >> 5], loc = synw[(size_t)k * 2] & 0xFFFFFu;
+      uint16_t c16;
+      const float w0 = wload_c(a.ev.wts, (int64_t)k, c16);
+      if ((mw >> (k & 31)) & 1u)
+        delayed_update(a, rule, (int64_t)k, w0, c16, ev.x[u], ev.xq[loc], am[u], (uint32_t)ev.qg[loc]);
+    }
+  }
+  int team = BS;
+  while (team > kWave && team * nlist > BS) team >>= 1;
+  const int back = BS - 1 - (int)threadIdx.x;
+  for (int j = back / team; j < nlist; j += BS / team) {
+    const int v = ev.list[j];
+    const uint32_t e1 = ev.ptr[v + 1];
+    for (uint32_t e = ev.ptr[v] + (uint32_t)(back % team); e < e1; e += team) {
+      const int64_t k = a.ev.post_pos[e];
+      const int u = a.ev.post_pre[e] - a.ev.src0;
+      uint16_t c16;
+      const float w0 = wload_c(a.ev.wts, k, c16);
+      if (am[u] == 0u) delayed_update(a, rule, k, w0, c16, ev.x[u], ev.xq[v], 0u, (uint32_t)ev.qg[v]);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) *ev.nsrc = 0;
+  for (int u = threadIdx.x; u < a.ev.sources; u += BS) {
+    const uint32_t m = am[u];
+    float x = ev.x[u];
+    if (m == 0u && x == 0.0f) continue;
+    float w = 0.0f, y = 0.0f;
+    for (int g = 0; g < a.G; ++g) rule.step(w, x, y, (m >> g) & 1u, false);
+    ev.x[u] = a.ev.tr.fmt ? dec16(enc16(x, a.ev.tr.fmt), a.ev.tr.fmt) : x;
+    am[u] = 0u;
+  }
+}
+
+// A spike of the exchange, kept for the group in which it arrives.
+__device__ __forceinline__ void delayed_mark(const FusedArgs& a, uint32_t* em, uint32_t e) {
+  const int u = (int)(e & kIdMask) - a.ev.src0;
+  if (u >= 0 && u < a.ev.sources) atomicOr(em + u, 1u << (e >> 24));
+}
+
 // One quad's delivery of n entries staged in LDS, kSpikesPerQuad at a time, by the form of
 // the delivery table the launch uses.
 template <int DM, bool EV = false>
@@ -881,12 +969,14 @@ __device__ __forceinline__ void deliver_staged(const FusedArgs& a, const uint32_
 // longer lists follow eight entries at a time with their loads in flight together.
 // Returns false (in every lane of the wave) when a wait exceeded the spin limit or another
 // workgroup reported an error; the error flag is then set.
-template <int BS, int DM, bool EV>
+template <int BS, int DM, int RULES>
 __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p, int par, uint32_t tag, int slot0,
                                                       int BL, int nownL, int L, int64_t* sring,
                                                       unsigned long long& st_del, long long q_lo, long long q_hi,
                                                       const uint16_t* slseg, const uint16_t* slrec, uint32_t* sent,
                                                       const EventLds* ev) {
+  constexpr bool EV = RULES == kRulesEvents, DV = RULES == kRulesDelayed;
+  uint32_t* em = DV ? ev->em + (size_t)par * a.ev.sources : nullptr;
   const int tid = threadIdx.x;
   const int lane = (int)__lane_id();
   const int quad = tid / kQuad, q = tid % kQuad;
@@ -932,7 +1022,7 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
     }
     if (!ok) break;
     if (!active) continue;
-    if (!EV && DM != kDeliverCompact && a.lseg_U > 0) {
+    if (RULES == kRulesOff && DM != kDeliverCompact && a.lseg_U > 0) {
       // LDS table: every lane delivers the entries it holds -- word q is entry q - 1, word
       // q + 4 entry q + 3 -- and longer lists eight at a time, two entries per lane
       const bool h0 = q >= 1 && q - 1 < c, h1 = q + 3 < c;
@@ -971,6 +1061,8 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
     // word q holds entry q - 1, word q + 4 entry q + 3
     if (q >= 1 && q - 1 < c) qent[q - 1] = (uint32_t)w0;
     if (q + 3 < c) qent[q + 3] = (uint32_t)w1;
+    if (DV && q >= 1 && q - 1 < c) delayed_mark(a, em, (uint32_t)w0);
+    if (DV && q + 3 < c) delayed_mark(a, em, (uint32_t)w1);
     __builtin_amdgcn_wave_barrier();
     deliver_staged<DM, EV>(a, qent, min(c, kQuadEnt - 1), q, p, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
                            slrec, ev);
@@ -994,6 +1086,8 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
       __builtin_amdgcn_wave_barrier();
       if (q < m) qent[q] = (uint32_t)e0;
       if (q + kQuad < m) qent[q + kQuad] = (uint32_t)e1;
+      if (DV && q < m) delayed_mark(a, em, (uint32_t)e0);
+      if (DV && q + kQuad < m) delayed_mark(a, em, (uint32_t)e1);
       __builtin_amdgcn_wave_barrier();
       deliver_staged<DM, EV>(a, qent, m, q, p, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec, ev);
     }
@@ -1010,12 +1104,13 @@ __device__ __forceinline__ bool tagged_gather_deliver(const FusedArgs& a, int p,
 // against the tag; (4) quads deliver kSpikesPerQuad staged entries at a time.  `scnt` is
 // LDS for P counts, `sscan` for P + 1 offsets.  Returns false when a wait failed (the error
 // flag is then set); uniform across the workgroup.
-template <int BS, int DM, bool EV>
+template <int BS, int DM, int RULES>
 __device__ __forceinline__ bool tagged_gather_stage(const FusedArgs& a, int p, int par, uint32_t tag, int slot0,
                                                     int BL, int nownL, int L, int64_t* sring,
                                                     unsigned long long& st_del, long long q_lo, long long q_hi,
                                                     const uint16_t* slseg, const uint16_t* slrec, uint32_t* sent,
                                                     int* scnt, int* sscan, int* s_ok, const EventLds* ev) {
+  constexpr bool EV = RULES == kRulesEvents, DV = RULES == kRulesDelayed;
   constexpr int kPer = kEntCap / BS;   // staged entries per thread and round
   const int tid = threadIdx.x;
   const int lane = (int)__lane_id();
@@ -1094,6 +1189,7 @@ __device__ __forceinline__ bool tagged_gather_stage(const FusedArgs& a, int p, i
         w[u] = xload64(xb + wo[u]);
       }
       sent[tid + u * BS] = (uint32_t)w[u];
+      if (DV && ok) delayed_mark(a, ev->em + (size_t)par * a.ev.sources, (uint32_t)w[u]);
     }
     if (!ok) *s_ok = 0;
     __syncthreads();
@@ -1118,9 +1214,9 @@ __device__ __forceinline__ void fused_plasticity(const FusedRule* rules, int n_r
     const int64_t j0 = rules[r].part[p], j1 = rules[r].part[p + 1];
     for (int64_t j = j0 + threadIdx.x; j < j1; j += BS) {
       if (kind == 0) stdp_wd_one(ra, j);
-      else if (kind == 1) stdp_vogels_one(ra, j);
-      else if (kind == 2) stdp_evans_one(ra, j);
-      else stdp_custom_one(ra, j);
+      else if (kind == 1) stdp_delayed_one<1>(ra, j);
+      else if (kind == 2) stdp_delayed_one<2>(ra, j);
+      else stdp_delayed_one<3>(ra, j);
     }
   }
 }
@@ -1153,6 +1249,45 @@ __device__ __forceinline__ uint32_t lif_block(const float* in, float t, float dt
   return mk;
 }
 
+// Sub-steps [g0, g0 + gn) of one neuron with conductance (KIND 1) or current synapses of LL
+// labels, inputs `in[x * LL + l]`: the inputs are read before the recurrence, whose chain of
+// dependent operations is what bounds it (COBA network, per group of 8 sub-steps: 4.7 us with the
+// reads, and the labels' constants loaded, in the chain, 1.3 us apart).  In chunks of kStep sub-steps: one for groups of one step (16 there: plain network
+// of 1000 neurons 5 % slower per step).  Returns the spike mask, shifted by g0.
+template <int KIND, int LL, int kStep>
+__device__ __forceinline__ unsigned long long cond_block(const float* in, int g0, int gn, const float* dec,
+                                                         const float* rev, float* gl, float t, float dt, float tref,
+                                                         float half_dt, float cv0, float omc, float cib, float thr,
+                                                         float vr, float rp, float& V, float& last) {
+  unsigned long long mk = 0ull;
+  for (int y0 = 0; y0 < gn; y0 += kStep) {
+    float ins[kStep * LL];
+#pragma unroll
+    for (int y = 0; y < kStep * LL; ++y) ins[y] = y0 * LL + y < gn * LL ? in[y0 * LL + y] : 0.0f;
+#pragma unroll
+    for (int y = 0; y < kStep; ++y) {
+      if (y0 + y < gn) {
+        const int g = g0 + y0 + y;
+        float total = 0.0f;
+#pragma unroll
+        for (int l = 0; l < LL; ++l) {
+          gl[l] = dec[l] * gl[l] + ins[y * LL + l];
+          total += (KIND == 1) ? gl[l] * (rev[l] - V) : gl[l];
+        }
+        const float dV = total * rp;
+        const float tg = t + (float)g * dt;
+        const bool ready = ((tg - last) - tref) > half_dt;
+        const float vn = ((cv0 + omc * V) + cib) + dV;
+        const bool fire = ready && (vn >= thr);
+        V = ready ? (fire ? vr : vn) : V;
+        last = fire ? tg : last;
+        mk |= (fire ? 1ull : 0ull) << g;
+      }
+    }
+  }
+  return mk;
+}
+
 // Partition of a workgroup.  Workgroups are dispatched to the XCDs round-robin, so block
 // b runs on XCD b % 8; mapping the blocks of one XCD to consecutive partitions keeps that
 // XCD's synapse segments contiguous inside every CSR row (its L2 then fetches only its own
@@ -1172,9 +1307,9 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   const int ilo = a.ilo[p], ihi = a.ilo[p + 1];
   const int nown = nhi - nlo, iown = ihi - ilo;
   const int L = L1 ? 1 : a.L, G = a.G, B = a.B, BL = a.BL, W = a.W;
-  constexpr bool DENSE = PLASTIC == kRulesDense, EV = PLASTIC == kRulesEvents;
+  constexpr bool DENSE = PLASTIC == kRulesDense, EV = PLASTIC == kRulesEvents, DV = PLASTIC == kRulesDelayed;
   const FusedLayout f = fused_layout(BL, L, W, G, a.nown_max, a.iown_max, a.xcap, a.P, a.lseg_U, a.lrec, a.cring,
-                                     a.dahead, EV ? a.ev.sources : 0);
+                                     a.dahead, EV || DV ? a.ev.sources : 0, DV);
   int64_t* sring = (int64_t*)(smem + f.ring);
   uint32_t* scring = (uint32_t*)(smem + f.ring);   // count ring (a.cring)
   uint32_t* shist = (uint32_t*)(smem + f.hist);
@@ -1197,16 +1332,38 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   uint16_t* slseg = (uint16_t*)(smem + f.lseg);
   uint16_t* slrec = (uint16_t*)(smem + f.lrec);
   EventLds ev;
-  if constexpr (EV) {
+  if constexpr (EV || DV) {
     ev.x = (float*)(smem + f.ev_x);
-    ev.bits = (uint32_t*)(smem + f.ev_bits);
+    ev.bits = ev.em = (uint32_t*)(smem + f.ev_bits);
     ev.xq = (float*)(smem + f.ev_xq);
     ev.qg = (int*)(smem + f.ev_qg);
     ev.list = (int*)(smem + f.ev_list);
     ev.tab = (float*)(smem + f.ev_tab);
-    for (int u = tid; u < a.ev.sources; u += BS) ev.x[u] = tload(a.ev.tr, 0, u);
-    for (int k = tid; k < (a.ev.sources + 31) / 32; k += BS) ev.bits[k] = 0u;
+    for (int u = tid; u < a.ev.sources; u += BS) ev.x[u] = tload(a.ev.tr, 0, a.ev.src0 + u);
+    if constexpr (EV)
+      for (int k = tid; k < (a.ev.sources + 31) / 32; k += BS) ev.bits[k] = 0u;
     for (int k = tid; k < a.ev.ntab; k += BS) ev.tab[k] = a.ev.tab[k];
+  }
+  if constexpr (DV) {
+    // the spikes that arrive in the first group: those of the G steps before it, from the history
+    ev.nsrc = (int*)(smem + f.ev_src);
+    ev.src = (uint16_t*)(smem + f.ev_src + 16);
+    if (tid == 0) *ev.nsrc = 0;
+    float t0;
+    int ti;
+    group_time(a, 0, t0, ti);
+    ev.ptr = (uint32_t*)(smem + f.ev_ptr);
+    for (int i = tid; i <= nown; i += BS) ev.ptr[i] = (uint32_t)a.ev.post_ptr[nlo + i];
+    for (int u = tid; u < a.ev.sources; u += BS) {
+      const int id = a.ev.src0 + u;
+      uint32_t m = 0u;
+      for (int g = 0; g < G; ++g)
+        m |= (id < a.N ? hist_get(a.hist_n, a.N, W, id, (int64_t)ti - G + g)
+                       : hist_get(a.hist_in, a.Nin, W, id - a.N, (int64_t)ti - G + g))
+                 ? 1u << g : 0u;
+      ev.em[u] = 0u;
+      ev.em[a.ev.sources + u] = m;
+    }
   }
   __shared__ int s_ok;
   __shared__ int s_wsum[BS / kWave];
@@ -1302,11 +1459,24 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     thr = a.thr[gi];
     vr = a.vreset[gi];
     rp = a.rp[gi];
-    if (KIND != 0)
-      for (int l = 0; l < L; ++l) gl[l] = a.gcond[(size_t)gi * L + l];
+    if (KIND != 0) {
+#pragma unroll
+      for (int l = 0; l < kMaxLabels; ++l)
+        if (l < L) gl[l] = a.gcond[(size_t)gi * L + l];
+    }
   }
-  float xq = 0.0f;   // kRulesEvents: postsynaptic trace of the owned neuron
-  if (EV && own) xq = tload(a.ev.tr, 1, gi);
+  // constants of the labels of the specialised recurrences (cond_block)
+  float cdec[2] = {0.0f, 0.0f}, crev[2] = {0.0f, 0.0f};
+  if (KIND != 0) {
+#pragma unroll
+    for (int l = 0; l < 2; ++l)
+      if (l < L) {
+        cdec[l] = a.decay_g[l];
+        crev[l] = a.erev[l];
+      }
+  }
+  float xq = 0.0f;   // rules driven by spikes: postsynaptic trace of the owned neuron
+  if ((EV || DV) && own) xq = tload(a.ev.tr, 1, gi);
   unsigned long long st_del = 0, st_ext = 0, st_spk = 0, st_in = 0;
   const float half_dt = 0.5f * a.dt;
   // fixed-point weights of the compact form: the full form's expression for one record
@@ -1561,6 +1731,15 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
               }
             }
             smask |= mk;
+          } else if (L <= 2) {
+            const float* in = sinp + ((size_t)lt * G + g0) * L;
+#define SPK_COND(LL, STEP) \
+            smask |= cond_block<KIND, LL, STEP>(in, g0, gn, cdec, crev, gl, t, a.dt, a.tref, half_dt, cv0, omc, cib, thr, vr, rp, V, last)
+            if (L == 1 && G == 1) SPK_COND(1, 1);
+            else if (L == 1) SPK_COND(1, kPrefetch);
+            else if (G == 1) SPK_COND(2, 1);
+            else SPK_COND(2, kPrefetch / 2);
+#undef SPK_COND
           } else {
             for (int x = 0; x < gn; ++x) {
               const int g = g0 + x;
@@ -1652,6 +1831,20 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
           if (qg >= 0) ev.list[atomicAdd(&scounter[2 + par], 1)] = tid;
         }
       }
+      if constexpr (DV) {
+        // the neuron's trace at the group's start and its spikes, for its synapses; then the
+        // trace advances
+        if (own) {
+          const uint32_t sm = (uint32_t)smask;
+          ev.xq[lt] = xq;
+          ev.qg[lt] = (int)sm;
+          if (sm) ev.list[atomicAdd(&scounter[2 + par], 1)] = tid;
+          const DelayedRule rule{a.ev.kind, a.ev.nearest, ev.tab, a.ev.dterm};
+          float w = 0.0f, x = 0.0f;
+          for (int g = 0; g < G; ++g) rule.step(w, x, xq, false, (sm >> g) & 1u);
+          if (a.ev.tr.fmt) xq = dec16(enc16(xq, a.ev.tr.fmt), a.ev.tr.fmt);
+        }
+      }
       if (!early && smask) {
         const int c = __popcll(smask);
         int pos = atomicAdd(scnt, c);
@@ -1739,15 +1932,20 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
         draw_groups<BS>(a, s + 1, min(a.dahead, a.ngroups - s - 1), sext, simask, nlo, nown, ilo, iown, st_ext,
                         scdf, sguide);
       clk.lap(a, 3);
+      if constexpr (DV) {
+        delayed_group<BS>(a, ev, p, par, scounter[2 + par]);
+        __syncthreads();
+        clk.lap(a, 5);
+      }
       // -- F. every source's list of this group, polled by its tags, delivered into the
       //    LDS ring (no grid barrier)
       if (a.xquad) {
-        if (!tagged_gather_deliver<BS, DM, EV>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
+        if (!tagged_gather_deliver<BS, DM, PLASTIC>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg,
                                                slrec, sent, &ev))
           s_ok = 0;
         __syncthreads();
       } else {
-        tagged_gather_stage<BS, DM, EV>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec,
+        tagged_gather_stage<BS, DM, PLASTIC>(a, p, par, tag, slot0, BL, nownL, L, sring, st_del, q_lo, q_hi, slseg, slrec,
                                         sent, (int*)shead, sscan, &s_ok, &ev);
       }
       if (!s_ok) return;
@@ -1862,14 +2060,20 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
   if (own) {
     a.V[gi] = V;
     a.last_n[gi] = last;
-    if (KIND != 0)
-      for (int l = 0; l < L; ++l) a.gcond[(size_t)gi * L + l] = gl[l];
-    if (EV) tstore(a.ev.tr, 1, gi, xq);
+    if (KIND != 0) {
+#pragma unroll
+      for (int l = 0; l < kMaxLabels; ++l)
+        if (l < L) a.gcond[(size_t)gi * L + l] = gl[l];
+    }
+    if (EV || DV) tstore(a.ev.tr, 1, gi, xq);
   }
-  if constexpr (EV) {
-    for (int i = tid; i < nown; i += BS) tstore(a.ev.tr, 0, nlo + i, ev.x[nlo + i]);
-    for (int i = tid; i < iown && a.N + ilo + i < a.ev.sources; i += BS)
-      tstore(a.ev.tr, 0, a.N + ilo + i, ev.x[a.N + ilo + i]);
+  if constexpr (EV || DV) {
+    auto put = [&](int id) {
+      const int u = id - a.ev.src0;
+      if (u >= 0 && u < a.ev.sources) tstore(a.ev.tr, 0, id, ev.x[u]);
+    };
+    for (int i = tid; i < nown; i += BS) put(nlo + i);
+    for (int i = tid; i < iown; i += BS) put(a.N + ilo + i);
   }
   // write the whole global ring slice back in its B-slot layout (zeros past the LDS window)
   {

@@ -15,6 +15,7 @@ FusedKernels instances() {
   k.run = (const void*)k_fused<KIND, L1, kRulesOff>;
   k.run_plastic = (const void*)k_fused<KIND, L1, kRulesDense>;
   k.run_events = (const void*)k_fused<KIND, L1, kRulesEvents>;
+  k.run_delayed = (const void*)k_fused<KIND, L1, kRulesDelayed>;
   k.batch = (const void*)k_fused_batch<KIND, L1, kRulesOff, kFusedBlock>;
   k.batch_small = (const void*)k_fused_batch<KIND, L1, kRulesOff, kBatchSmallBlock>;
   return k;

@@ -9,6 +9,7 @@ struct FusedKernels {
   const void* run;            // k_fused, no plasticity
   const void* run_plastic;    // k_fused with plasticity, every rule per synapse
   const void* run_events;     // k_fused with one spike-driven weight-dependent rule
+  const void* run_delayed;    // k_fused with one spike-driven Vogels, Evans or Custom rule
   const void* batch;          // k_fused_batch of kFusedBlock threads
   const void* batch_small;    // k_fused_batch of kBatchSmallBlock threads
 };

@@ -1143,115 +1143,92 @@ __device__ __forceinline__ bool pre_bit(const StdpArgs& a, int u, int64_t step) 
                    : hist_get(a.hist_in, a.Nin, a.W, u - a.N, step);
 }
 
-// InhibitorySTDPPlasticity.cu:72-155. tab = {decay, lr}; dterm = lr*(2*rate*tau) (double)
-__device__ __forceinline__ void stdp_vogels_one(const StdpArgs& a, int64_t j) {
-  const int64_t s = a.pos[j];
-  const int u = a.pre[j];
-  const int post = a.tgt[s];
-  const int d = a.delay[s];
-  const float decay = a.tab[0], lr = a.tab[1];
-  float xpre = tload(a.tr, 0, j), xpost = tload(a.tr, 1, j);
-  const float w0 = wload(a.wts, s);
-  float w = w0;
-  for (int g = 0; g < a.G; ++g) {
-    xpre *= decay;
-    xpost *= decay;
-    const int64_t step = (int64_t)a.tidx + g;
-    const bool pr = pre_bit(a, u, step - d);
-    const bool po = hist_get(a.hist_n, a.N, a.W, post, step);
-    if (pr) xpre += 1.0f;
-    if (po) xpost += 1.0f;
-    float upd = 0.0f;
-    if (pr) {
-      upd += lr * xpost;
-      upd = (float)((double)upd + (-a.dterm));
+// The rules whose traces see the delayed presynaptic spikes, one sub-step at a time: xa is the
+// presynaptic, xb the postsynaptic trace, pr / po whether a presynaptic spike arrives / the
+// postsynaptic neuron spikes in the step.
+struct DelayedRule {
+  int kind;               // 1 Vogels, 2 Evans, 3 Custom
+  int nearest;
+  const float* tab;
+  double dterm;
+
+  // upper bound of the weights (the lower one is 0)
+  __device__ __forceinline__ float hi() const { return kind == 2 ? 1.0f : __builtin_inff(); }
+
+  __device__ __forceinline__ void step(float& w, float& xa, float& xb, bool pr, bool po) const {
+    if (kind == 1) {
+      // InhibitorySTDPPlasticity.cu:72-155. tab = {decay, lr}; dterm = lr*(2*rate*tau) (double)
+      const float decay = tab[0], lr = tab[1];
+      xa *= decay;
+      xb *= decay;
+      if (pr) xa += 1.0f;
+      if (po) xb += 1.0f;
+      float upd = 0.0f;
+      if (pr) {
+        upd += lr * xb;
+        upd = (float)((double)upd + (-dterm));
+      }
+      if (po) upd += lr * xa;
+      w += upd;
+      if (w < 0.0f) w = 0.0f;
+    } else if (kind == 2) {
+      // EvansSTDPPlasticity.cu:59-143. tab = {dC, dD, aC, aD}
+      const float dC = tab[0], dD = tab[1], aC = tab[2], aD = tab[3];
+      xa = dC * xa;
+      xb = dD * xb;
+      if (pr) xa += aC * (1.0f - xa);
+      if (po) xb += aD * (1.0f - xb);
+      float upd = 0.0f;
+      const float wo = w;
+      if (pr) upd -= wo * xb;
+      if (po) upd += (1.0f - wo) * xa;
+      w = wo + upd;
+      if (w < 0.0f) w = 0.0f;
+      if (w > 1.0f) w = 1.0f;
+    } else {
+      // CustomSTDPPlasticity.cu:67-155. tab = {post decay expf(-dt/tau_minus), pre decay
+      // expf(-dt/tau_plus), a_plus, a_minus, a_star, w_max, learning_rate}; nearest: a spike
+      // sets its trace to the amplitude instead of adding it.  Weights clamped at 0 only.
+      const float dpost = tab[0], dpre = tab[1], ap = tab[2], am = tab[3], ast = tab[4];
+      const float wmax = tab[5], lr = tab[6];
+      xb *= dpost;
+      xa *= dpre;
+      if (pr) xa = nearest ? ap : xa + ap;
+      if (po) xb = nearest ? am : xb + am;
+      float upd = 0.0f;
+      const float wo = w;
+      if (pr) upd -= ((lr * (wo / wmax)) * xb + lr * ast);
+      if (po) upd += lr * xa;
+      w = wo + upd;
+      if (w < 0.0f) w = 0.0f;
     }
-    if (po) upd += lr * xpre;
-    w += upd;
-    if (w < 0.0f) w = 0.0f;
   }
-  wupdate(a.wts, s, w0, w, 0.0f, __builtin_inff());
-  tstore(a.tr, 0, j, xpre);
-  tstore(a.tr, 1, j, xpost);
-}
+};
 
-static __global__ __launch_bounds__(256) void k_stdp_vogels(StdpArgs a) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < a.P) stdp_vogels_one(a, j);
-}
-
-// EvansSTDPPlasticity.cu:59-143. tab = {dC, dD, aC, aD}
-__device__ __forceinline__ void stdp_evans_one(const StdpArgs& a, int64_t j) {
+// Every sub-step of one synapse's group, from the spike histories.
+template <int KIND>
+__device__ __forceinline__ void stdp_delayed_one(const StdpArgs& a, int64_t j) {
   const int64_t s = a.pos[j];
   const int u = a.pre[j];
   const int post = a.tgt[s];
   const int d = a.delay[s];
-  const float dC = a.tab[0], dD = a.tab[1], aC = a.tab[2], aD = a.tab[3];
-  float C = tload(a.tr, 0, j), D = tload(a.tr, 1, j);
+  const DelayedRule rule{KIND, a.nearest, a.tab, a.dterm};
+  float xa = tload(a.tr, 0, j), xb = tload(a.tr, 1, j);
   const float w0 = wload(a.wts, s);
   float w = w0;
   for (int g = 0; g < a.G; ++g) {
-    C = dC * C;
-    D = dD * D;
     const int64_t step = (int64_t)a.tidx + g;
-    const bool pr = pre_bit(a, u, step - d);
-    const bool po = hist_get(a.hist_n, a.N, a.W, post, step);
-    if (pr) C += aC * (1.0f - C);
-    if (po) D += aD * (1.0f - D);
-    float upd = 0.0f;
-    const float wo = w;
-    if (pr) upd -= wo * D;
-    if (po) upd += (1.0f - wo) * C;
-    w = wo + upd;
-    if (w < 0.0f) w = 0.0f;
-    if (w > 1.0f) w = 1.0f;
+    rule.step(w, xa, xb, pre_bit(a, u, step - d), hist_get(a.hist_n, a.N, a.W, post, step));
   }
-  wupdate(a.wts, s, w0, w, 0.0f, 1.0f);
-  tstore(a.tr, 0, j, C);
-  tstore(a.tr, 1, j, D);
+  wupdate(a.wts, s, w0, w, 0.0f, rule.hi());
+  tstore(a.tr, 0, j, xa);
+  tstore(a.tr, 1, j, xb);
 }
 
-static __global__ __launch_bounds__(256) void k_stdp_evans(StdpArgs a) {
+template <int KIND>
+__global__ __launch_bounds__(256) void k_stdp_delayed(StdpArgs a) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < a.P) stdp_evans_one(a, j);
-}
-
-// CustomSTDPPlasticity.cu:67-155. tab = {post decay expf(-dt/tau_minus), pre decay
-// expf(-dt/tau_plus), a_plus, a_minus, a_star, w_max, learning_rate}; nearest: a spike
-// sets its trace to the amplitude instead of adding it.  Weights clamped at 0 only.
-__device__ __forceinline__ void stdp_custom_one(const StdpArgs& a, int64_t j) {
-  const int64_t s = a.pos[j];
-  const int u = a.pre[j];
-  const int post = a.tgt[s];
-  const int d = a.delay[s];
-  const float dpost = a.tab[0], dpre = a.tab[1], ap = a.tab[2], am = a.tab[3], ast = a.tab[4];
-  const float wmax = a.tab[5], lr = a.tab[6];
-  float xpre = tload(a.tr, 0, j), xpost = tload(a.tr, 1, j);
-  const float w0 = wload(a.wts, s);
-  float w = w0;
-  for (int g = 0; g < a.G; ++g) {
-    xpost *= dpost;
-    xpre *= dpre;
-    const int64_t step = (int64_t)a.tidx + g;
-    const bool pr = pre_bit(a, u, step - d);
-    const bool po = hist_get(a.hist_n, a.N, a.W, post, step);
-    if (pr) xpre = a.nearest ? ap : xpre + ap;
-    if (po) xpost = a.nearest ? am : xpost + am;
-    float upd = 0.0f;
-    const float wo = w;
-    if (pr) upd -= ((lr * (wo / wmax)) * xpost + lr * ast);
-    if (po) upd += lr * xpre;
-    w = wo + upd;
-    if (w < 0.0f) w = 0.0f;
-  }
-  wupdate(a.wts, s, w0, w, 0.0f, __builtin_inff());
-  tstore(a.tr, 0, j, xpre);
-  tstore(a.tr, 1, j, xpost);
-}
-
-static __global__ __launch_bounds__(256) void k_stdp_custom(StdpArgs a) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < a.P) stdp_custom_one(a, j);
+  if (j < a.P) stdp_delayed_one<KIND>(a, j);
 }
 
 // WeightNormSTDPPlasticity.cu:68-172.  One lane per postsynaptic neuron of the rule: the

@@ -252,9 +252,12 @@ struct RuleHost {
   hvec<int64_t> order;            // device order j -> index into syn (grouped by post partition)
   std::vector<int64_t> part;      // [P+1] offsets of each postsynaptic partition
   int64_t* d_part = nullptr;
-  // spike-driven form of the weight-dependent rule (per-phase kernels): rule indices by
-  // presynaptic and by postsynaptic neuron, traces per neuron, the listed neurons
+  // spike-driven form (weight-dependent rule: per-phase and persistent kernels; delayed rules:
+  // persistent kernel): rule indices by presynaptic and by postsynaptic neuron, traces per
+  // neuron, the listed neurons
   bool ev_ok = false;
+  int src_lo = 0, src_hi = 0;     // units [src_lo, src_hi) hold every source with synapses of the rule
+  int delay = 0;                  // the delay of all synapses of a delayed rule with that form
   int64_t* d_ev_pre_ptr = nullptr;
   int32_t* d_ev_pre_idx = nullptr;   // nullptr: rule order already groups by presynaptic neuron
   int64_t* d_ev_post_ptr = nullptr;
@@ -406,11 +409,11 @@ struct spk_network {
   // weight-dependent rule driven by spikes inside the persistent kernel (kRulesEvents): the
   // sources whose traces every workgroup keeps, and the launch's dynamic LDS
   bool ev_fused = false;
-  int ev_sources = 0;
+  int ev_src0 = 0, ev_sources = 0;
   size_t fused_lds_ev = 0;
   bool generated = false;        // connectivity generated on the device (persistent kernel only)
-  size_t lds_attr[3] = {0, 0, 0};  // dynamic LDS limit set for the kernel of each kRules* mode
-  const void* lds_fn[3] = {nullptr, nullptr, nullptr};  // ... and the kernel it was set for
+  size_t lds_attr[4] = {0, 0, 0, 0};  // dynamic LDS limit set for the kernel of each kRules* mode
+  const void* lds_fn[4] = {nullptr, nullptr, nullptr, nullptr};  // ... and the kernel it was set for
   // window statistics (spk_stats_begin)
   unsigned int *d_st_cnt = nullptr, *d_st_nisi = nullptr, *d_st_hist = nullptr;
   float* d_st_prev = nullptr;
@@ -592,6 +595,23 @@ int host_threads() {
 }
 
 // Per-rule device constants that depend on G.
+// Constants of the rules other than the weight-dependent one (at most 7); their count.
+int rule_constants(const spk_network* n, RuleHost& r, float* v) {
+  const float dt = n->dt;
+  auto put = [&](std::initializer_list<float> c) { std::copy(c.begin(), c.end(), v); return (int)c.size(); };
+  if (r.kind == 3)
+    return put({expf(-dt / r.cu.tau_minus), expf(-dt / r.cu.tau_plus), r.cu.a_plus, r.cu.a_minus,
+                r.cu.a_star, r.cu.w_max, r.cu.learning_rate});
+  if (r.kind == 1) {
+    r.dterm = (double)r.vg.learningrate * (2.0 * (double)r.vg.targetrate * (double)r.vg.tau_istdp);
+    return put({expf(-dt / r.vg.tau_istdp), r.vg.learningrate});
+  }
+  if (r.kind == 4) return put({0.0f});   // weight normalization keeps no per-rule constants
+  return put({1.0f - (dt / r.ev.decay_term_tau_C), 1.0f - (dt / r.ev.decay_term_tau_D),
+              dt * r.ev.synaptic_neurotransmitter_concentration_alpha_C,
+              dt * r.ev.model_parameter_alpha_D});
+}
+
 int refresh_rule_tables(spk_network* n, RuleHost& r) {
   if (r.tab_G == n->G && r.d_tab) return SPK_OK;
   std::vector<float> tab;
@@ -609,18 +629,9 @@ int refresh_rule_tables(spk_network* n, RuleHost& r) {
     for (int k = 0; k <= G; ++k) tab.push_back(Ep[k]);
     for (int k = 0; k <= G; ++k) tab.push_back(1.0f / Em[k]);
     for (int k = 0; k <= G; ++k) tab.push_back(1.0f / Ep[k]);
-  } else if (r.kind == 3) {
-    tab = {expf(-dt / r.cu.tau_minus), expf(-dt / r.cu.tau_plus), r.cu.a_plus, r.cu.a_minus,
-           r.cu.a_star, r.cu.w_max, r.cu.learning_rate};
-  } else if (r.kind == 1) {
-    tab = {expf(-dt / r.vg.tau_istdp), r.vg.learningrate};
-    r.dterm = (double)r.vg.learningrate * (2.0 * (double)r.vg.targetrate * (double)r.vg.tau_istdp);
-  } else if (r.kind == 4) {
-    tab = {0.0f};   // weight normalization keeps no per-rule constants
   } else {
-    tab = {1.0f - (dt / r.ev.decay_term_tau_C), 1.0f - (dt / r.ev.decay_term_tau_D),
-           dt * r.ev.synaptic_neurotransmitter_concentration_alpha_C,
-           dt * r.ev.model_parameter_alpha_D};
+    tab.resize(7);
+    tab.resize(rule_constants(n, r, tab.data()));
   }
   dfree(r.d_tab);
   n->rules_uploaded = false;
@@ -629,6 +640,19 @@ int refresh_rule_tables(spk_network* n, RuleHost& r) {
   SPK_HIP(hipMemcpy(r.d_tab, tab.data(), tab.size() * sizeof(float), hipMemcpyHostToDevice));
   r.tab_G = n->G;
   return SPK_OK;
+}
+
+// Whether a rule's parameters and delays let it run by spikes (refresh_rule_tables' values are
+// finite: a trace at rest then stays there, and a weight without spikes keeps its value).
+bool event_rule_values(const spk_network* n, RuleHost& r) {
+  if (r.kind == 0) return true;
+  if (r.kind == 4 || !n->fused_ok || n->rules.size() != 1 || n->G > 32) return false;
+  r.delay = n->G;
+  for (int64_t s : r.syn)
+    if (n->h_delay[s] != r.delay) return false;
+  float v[7] = {};
+  rule_constants(n, r, v);
+  return std::all_of(v, v + 7, [](float x) { return std::isfinite(x); }) && std::isfinite(r.dterm);
 }
 
 // Device state of the neurons, inputs, spike lists and counters (every prepared network
@@ -704,11 +728,11 @@ int alloc_monitors(spk_network* n) {
   return SPK_OK;
 }
 
-// Bitmask of the CSR positions of a network's single spike-driven weight-dependent rule
-// (the source side of k_deliver); other networks keep none.
+// Bitmask of the CSR positions of a network's single spike-driven rule (the source side of
+// k_deliver, and of the persistent kernel's spike-driven rules); other networks keep none.
 int build_wd_mask(spk_network* n) {
   dfree(n->d_wd_mask);
-  if (n->rules.size() != 1 || n->rules[0].kind != 0 || !n->rules[0].ev_ok || n->rules[0].cnt == 0) return SPK_OK;
+  if (n->rules.size() != 1 || !n->rules[0].ev_ok || n->rules[0].cnt == 0) return SPK_OK;
   const size_t words = (size_t)(n->S + 31) / 32;
   if (int rc = dalloc(&n->d_wd_mask, words)) return rc;
   SPK_HIP(hipMemsetAsync(n->d_wd_mask, 0, sizeof(uint32_t) * words, n->stream));
@@ -941,9 +965,9 @@ int launch_rule(spk_network* n, int rid, float t) {
   a.tidx = (int)roundf(t / n->dt); a.nearest = r.nearest; a.t = t; a.dt = n->dt;
   const int grid = grid_for(a.P, 256);
   if (r.kind == 0) hipLaunchKernelGGL(spk::k_stdp_wd, dim3(grid), dim3(256), 0, n->stream, a);
-  else if (r.kind == 1) hipLaunchKernelGGL(spk::k_stdp_vogels, dim3(grid), dim3(256), 0, n->stream, a);
-  else if (r.kind == 2) hipLaunchKernelGGL(spk::k_stdp_evans, dim3(grid), dim3(256), 0, n->stream, a);
-  else hipLaunchKernelGGL(spk::k_stdp_custom, dim3(grid), dim3(256), 0, n->stream, a);
+  else if (r.kind == 1) hipLaunchKernelGGL(spk::k_stdp_delayed<1>, dim3(grid), dim3(256), 0, n->stream, a);
+  else if (r.kind == 2) hipLaunchKernelGGL(spk::k_stdp_delayed<2>, dim3(grid), dim3(256), 0, n->stream, a);
+  else hipLaunchKernelGGL(spk::k_stdp_delayed<3>, dim3(grid), dim3(256), 0, n->stream, a);
   SPK_HIP(hipGetLastError());
   return SPK_OK;
 }
@@ -1319,7 +1343,8 @@ const void* fused_kernel(const spk_network* n, int rules) {
   if (rules == spk::kRulesOff && n->kind == SPK_SYN_VOLTAGE && l1 && n->compact && n->rules.empty())
     return n->lseg_U > 0 ? spk::fused_kernel_lds_table() : spk::fused_kernel_compact();
   const spk::FusedKernels k = spk::fused_kernels(n->kind, l1);
-  return rules == spk::kRulesOff ? k.run : (rules == spk::kRulesDense ? k.run_plastic : k.run_events);
+  const void* by_rules[] = {k.run, k.run_plastic, k.run_events, k.run_delayed};   // kRules*
+  return by_rules[rules];
 }
 
 // Dynamic LDS a persistent workgroup may take: the per-workgroup limit less the static LDS
@@ -1361,23 +1386,30 @@ int plan_lds_table(spk_network* n, int64_t mx, int U) {
   return SPK_OK;
 }
 
-// Whether the persistent kernel can run the network's rule by spikes: one weight-dependent
-// rule in its spike-driven form, every unit of the rule spiking at most once per group (a
-// source's row is then walked, and its trace raised, once), and the traces of all its sources
-// beside the rest of the LDS layout.  Otherwise the rules run per synapse behind the grid
-// barrier.  Measured on 6000 neurons with 500 synapses each, delays from one step: 51 us per
-// group per synapse, 5.6 us by spikes; the spike-driven form has no size from which it is
-// slower (its cost per group is one pass over the sources, that of the other one pass over
-// the rule's synapses, and a source has at least one).
+// The spike-driven mode of the persistent kernel for the network's rule (kRulesEvents: the
+// weight-dependent rule; kRulesDelayed: the others).
+int event_mode(const spk_network* n) { return n->rules[0].kind == 0 ? spk::kRulesEvents : spk::kRulesDelayed; }
+
+// Whether the persistent kernel can run the network's rule by spikes: one rule in its
+// spike-driven form and the state of all its sources beside the rest of the LDS layout; for the
+// weight-dependent rule also every unit of the rule spiking at most once per group (a source's
+// row is then walked, and its trace raised, once).  Otherwise the rules run per synapse behind
+// the grid barrier.  Weight-dependent rule, 6000 neurons with 500 synapses each, delays from one
+// step: 51 us per group per synapse, 5.6 us by spikes.  The spike-driven form has no size from
+// which it is slower: its cost per group is one pass over the sources, that of the other one
+// pass over the rule's synapses, and a source has at least one.
 int plan_event_rule(spk_network* n, bool input_sources) {
   n->ev_fused = false;
-  if (!n->fused_ok || n->rules.size() != 1 || !n->d_wd_mask) return SPK_OK;   // (a mask: kind 0, ev_ok, synapses)
-  if (max_spikes_per_group(n->tref, n->dt, n->G) != 1 || (input_sources && n->G != 1)) return SPK_OK;
-  n->ev_sources = input_sources ? n->nu() : n->N;
+  if (!n->fused_ok || n->rules.size() != 1 || !n->d_wd_mask) return SPK_OK;   // (a mask: ev_ok, synapses)
+  const bool delayed = event_mode(n) == spk::kRulesDelayed;
+  if (!delayed && (max_spikes_per_group(n->tref, n->dt, n->G) != 1 || (input_sources && n->G != 1))) return SPK_OK;
+  n->ev_src0 = delayed ? n->rules[0].src_lo : 0;
+  n->ev_sources = delayed ? n->rules[0].src_hi - n->rules[0].src_lo : (input_sources ? n->nu() : n->N);
+  if (delayed && n->ev_sources > 65535) return SPK_OK;   // (16-bit list of arriving sources)
   const size_t lds = spk::fused_lds_bytes(n->BL, n->L, n->W, n->G, n->nown_max, n->iown_max, n->xcap, n->P, 0, 0, 0, 1,
-                                          n->ev_sources);
+                                          n->ev_sources, delayed);
   if (lds > fused_lds_limit(n)) return SPK_OK;
-  const void* fn = fused_kernel(n, spk::kRulesEvents);
+  const void* fn = fused_kernel(n, event_mode(n));
   if (lds > 65536) SPK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   int per_cu = 0;
   SPK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, spk::kFusedBlock, lds));
@@ -1387,10 +1419,28 @@ int plan_event_rule(spk_network* n, bool input_sources) {
   return SPK_OK;
 }
 
-// How a launch applies the network's rules.
-int rules_mode(const spk_network* n, bool plastic) {
+// Time step of group `g` of a run from `start`, as the kernels compute it.
+int64_t group_step(const spk_network* n, float start, int64_t g) {
+  return (int64_t)roundf((start + (float)(g * n->G) * n->dt) / n->dt);
+}
+
+// Whether a run of `ngroups` groups may apply the rule by spikes.  A delayed rule then takes the
+// spikes of one group for the arrivals of the next: all its delays equal the group's length, and
+// the groups' steps follow each other without a gap or an overlap (not so where float32 times
+// no longer resolve the step).
+bool event_run_ok(const spk_network* n, float start, int64_t ngroups) {
+  if (!n->ev_fused) return false;
+  if (event_mode(n) == spk::kRulesEvents) return true;
+  if (n->rules[0].delay != n->G) return false;
+  for (int64_t g = 1; g < ngroups; ++g)
+    if (group_step(n, start, g) != group_step(n, start, g - 1) + n->G) return false;
+  return true;
+}
+
+// How a launch applies the network's rules; `events`: event_run_ok.
+int rules_mode(const spk_network* n, bool plastic, bool events) {
   if (!plastic || n->rules.empty()) return spk::kRulesOff;
-  return n->ev_fused && !n->rules[0].dense_next ? spk::kRulesEvents : spk::kRulesDense;
+  return events && !n->rules[0].dense_next ? event_mode(n) : spk::kRulesDense;
 }
 
 // Kernel arguments of the persistent kernel (all but the run position); `rules`: kRules*.
@@ -1417,7 +1467,7 @@ int fill_fused_args(spk_network* n, int rules, spk::FusedArgs& a) {
     a.lrec = n->lrec;
     a.cring = n->cring_ok ? 1 : 0;
   }
-  if (rules == spk::kRulesEvents) {
+  if (rules == spk::kRulesEvents || rules == spk::kRulesDelayed) {
     RuleHost& r = n->rules[0];
     if (!r.neu_tr) {
       if (int rc = copy_traces(n, r, true)) return rc;
@@ -1428,7 +1478,9 @@ int fill_fused_args(spk_network* n, int rules, spk::FusedArgs& a) {
     a.ev.wts = weights_of(n);
     a.ev.tab = r.d_tab; a.ev.mask = n->d_wd_mask;
     a.ev.post_ptr = r.d_ev_post_ptr; a.ev.post_pos = r.d_ev_post_pos; a.ev.post_pre = r.d_ev_post_pre;
-    a.ev.sources = n->ev_sources; a.ev.ntab = 5 + 4 * (G + 1); a.ev.nearest = r.nearest;
+    a.ev.src0 = n->ev_src0; a.ev.sources = n->ev_sources; a.ev.nearest = r.nearest; a.ev.kind = r.kind; a.ev.dterm = r.dterm;
+    const int ntab[] = {5 + 4 * (G + 1), 2, 4, 7};   // refresh_rule_tables
+    a.ev.ntab = ntab[r.kind];
   }
   a.n_rules = plastic ? (int)n->rules.size() : 0;
   for (int r = 0; r < a.n_rules; ++r) {
@@ -1519,9 +1571,8 @@ int stage_fused(spk_network* n, spk::FusedArgs& a, float start, int64_t group0, 
   a.st = stats_args(n, start);
   stats_advance(n, (int64_t)roundf(start / n->dt), group0 + ng);
   if (ng > 0 && !n->mons.empty()) {
-    auto step_of = [&](int64_t g) { return (int64_t)roundf((start + (float)(g * n->G) * n->dt) / n->dt); };
-    note_steps(n, step_of(group0), 0);
-    note_steps(n, step_of(group0 + ng - 1), n->G);
+    note_steps(n, group_step(n, start, group0), 0);
+    note_steps(n, group_step(n, start, group0 + ng - 1), n->G);
   }
   a.start = start;
   a.group0 = group0;
@@ -1544,7 +1595,7 @@ int launch_fused(spk_network* n, spk::FusedArgs& a, float start, int64_t group0,
   if (int rc = stage_fused(n, a, start, group0, ng, n->stream)) return rc;
   const int fi = a.plastic;
   const void* fn = fused_kernel(n, fi);
-  const size_t lds = fi == spk::kRulesEvents ? n->fused_lds_ev : n->fused_lds;
+  const size_t lds = fi == spk::kRulesEvents || fi == spk::kRulesDelayed ? n->fused_lds_ev : n->fused_lds;
   if (lds > 65536 && (n->lds_attr[fi] < lds || n->lds_fn[fi] != fn)) {
     SPK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     n->lds_attr[fi] = lds;
@@ -1591,8 +1642,9 @@ int run_fused(spk_network* n, float start, int64_t ngroups, int flags) {
   spk::FusedArgs a;
   // a rule that runs by spikes takes its first group after prepare or set_weights per synapse
   // (RuleHost::dense_next): a launch of one group
-  const int64_t first = n->ev_fused && rules_mode(n, plastic) == spk::kRulesDense ? 1 : 0;
-  if (int rc = fill_fused_args(n, rules_mode(n, plastic), a)) return rc;
+  const bool events = plastic && event_run_ok(n, start, ngroups);
+  const int64_t first = events && rules_mode(n, plastic, events) == spk::kRulesDense ? 1 : 0;
+  if (int rc = fill_fused_args(n, rules_mode(n, plastic, events), a)) return rc;
   if (n->profiling) {
     if (!n->d_prof) {
       if (int rc = dalloc(&n->d_prof, spk::kProfPhases)) return rc;
@@ -1611,7 +1663,7 @@ int run_fused(spk_network* n, float start, int64_t ngroups, int flags) {
     ng = s0 < first ? first : std::min<int64_t>(chunk, ngroups - s0);
     if (first && s0 == first) {
       unsigned long long* prof = a.prof;
-      if (int rc = fill_fused_args(n, rules_mode(n, plastic), a)) return rc;
+      if (int rc = fill_fused_args(n, rules_mode(n, plastic, events), a)) return rc;
       a.prof = prof;
     }
     if (int rc = launch_fused(n, a, start, s0, (int)ng, n->ev_kernel[2 * li], n->ev_kernel[2 * li + 1])) return rc;
@@ -2546,9 +2598,10 @@ int spk_prepare(spk_network* n, int G) {
     if ((rc = upload(r.d_pos, pos.data(), P, st))) return rc;
     if ((rc = upload(r.d_pre, pre.data(), P, st))) return rc;
     if ((rc = upload(r.d_part, r.part.data(), (size_t)n->P + 1, st))) return rc;
-    // the weight-dependent rule's spike-driven form: its rule indices grouped by
-    // presynaptic neuron (already so in CSR order) and by postsynaptic neuron
-    r.ev_ok = r.kind == 0 && P > 0 && P < (size_t)INT32_MAX && S < (int64_t)UINT32_MAX;
+    // the rule's spike-driven form: its rule indices grouped by presynaptic neuron (already so
+    // in CSR order) and by postsynaptic neuron.  Rules that see delayed presynaptic spikes have
+    // one when all their delays are one group's length, of at most 32 steps.
+    r.ev_ok = P > 0 && P < (size_t)INT32_MAX && S < (int64_t)UINT32_MAX && event_rule_values(n, r);
     if (r.ev_ok) {
       const int U = n->nu();
       std::vector<int64_t> pp, qp;
@@ -2564,6 +2617,10 @@ int spk_prepare(spk_network* n, int G) {
                       qs[k] = (uint32_t)pos[j];
                       qu[k] = pre[j];
                     }, qp);
+      r.src_hi = U;
+      while (r.src_hi > 0 && pp[r.src_hi] == pp[r.src_hi - 1]) --r.src_hi;
+      r.src_lo = 0;
+      while (r.src_lo < r.src_hi && pp[r.src_lo + 1] == pp[r.src_lo]) ++r.src_lo;
       r.max_post = 0;
       for (size_t v = 0; v + 1 < qp.size(); ++v) r.max_post = std::max(r.max_post, qp[v + 1] - qp[v]);
       if ((rc = dalloc(&r.d_ev_pre_ptr, (size_t)U + 1))) return rc;
@@ -2806,7 +2863,7 @@ int spk_step_group(spk_network* n, float t, int flags) {
   if (n->generated && !(flags & SPK_RUN_FORCE_LAUNCHES) && n->G == n->Gprep) {
     if (int rc = check_time(n, t)) return rc;
     spk::FusedArgs a;
-    if (int rc = fill_fused_args(n, rules_mode(n, (flags & SPK_RUN_PLASTICITY) != 0), a)) return rc;
+    if (int rc = fill_fused_args(n, rules_mode(n, (flags & SPK_RUN_PLASTICITY) != 0, event_run_ok(n, t, 1)), a)) return rc;
     return launch_fused(n, a, t, 0, 1);
   }
   if (int rc = check_listed(n)) return rc;
