@@ -124,18 +124,19 @@ struct FusedArgs {
   const uint32_t* wc;       // 16-bit weights (wfmt 1 bfloat16, 2 binary16) in the low halves, instead of the records'
   int wfmt;
   const float* scale;       // nullptr: uniform scale0
-  // compact form (no plasticity, one label, uniform scale): every synapse of a source
-  // u < src_split has weight w_lo, every other one w_hi, all have delay src_delay, and the
-  // records are the 16-bit local targets alone (null: the full records above)
+  // compact form (no plasticity, one label, uniform scale): every synapse of a source u in
+  // [src_split, src_split + src_nhi) has weight w_hi (the inhibitory neurons), every other one
+  // w_lo (the excitatory ones, inputs), all have delay src_delay, and the records are the
+  // 16-bit local targets alone (null: the full records above)
   const uint16_t* syn16;
   float w_lo, w_hi;
-  int src_split, src_delay;
+  int src_split, src_nhi, src_delay;
   // compact form with the partition's delivery table in LDS (copied from seg and syn16 when
   // the group loop starts): 16-bit local starts of the lseg_U source units' segments (and
   // the end), at most lrec targets per partition; 0: off
   int lseg_U, lrec;
   // compact form with a count ring: each LDS ring word holds the step's count of
-  // deliveries from sources below src_split (low 16 bits) and from the others (high 16
+  // deliveries from sources of weight w_lo (low 16 bits) and of weight w_hi (high 16
   // bits); the reading neuron rebuilds the exact fixed-point sum from the counts.  The
   // global int64 ring then only carries the inputs pending when the launch starts (read
   // for steps below the launch's first step + BL) and receives the pending ones at its end.
@@ -601,14 +602,18 @@ __device__ __forceinline__ void deliver_quad(const FusedArgs& a, const uint32_t*
   }
 }
 
+// Whether a source of the compact form weighs w_hi.
+__device__ __forceinline__ bool compact_hi(const FusedArgs& a, uint32_t id) {
+  return id - (uint32_t)a.src_split < (uint32_t)a.src_nhi;
+}
+
 // Compact form of deliver_quad: 2-byte records, the fixed-point weight and the slot are
-// those of the spike's source (q_lo below src_split, q_hi from it on), computed once per
+// those of the spike's source (q_lo or q_hi: compact_hi), computed once per
 // spike with the same expression as the full form.  The targets are read eight at a time:
 // a spike's segment [s0, s1) of syn16 is covered by the 16-byte aligned chunks it touches
 // (the array is padded to whole chunks), lane q of the quad takes chunks q, q + 4, ... and
 // adds the chunk's targets that lie inside the segment; the first chunk of every spike is
-// loaded before any is used.  With the count ring the increment is 1 (sources below
-// src_split) or 1 << 16.
+// loaded before any is used.  With the count ring the increment is 1 (weight w_lo) or 1 << 16.
 template <bool CR>
 __device__ __forceinline__ void deliver_quad_compact(const FusedArgs& a, const uint32_t* ents, int n, int q,
                                                      int p, int slot0, int B, int nown, int64_t* sring,
@@ -628,7 +633,8 @@ __device__ __forceinline__ void deliver_quad_compact(const FusedArgs& a, const u
       const size_t sb = (size_t)id * (a.P + 1) + p;
       s0[r] = a.seg[sb];
       s1[r] = a.seg[sb + 1];
-      qv[r] = CR ? ((int)id < a.src_split ? 1 : 0x10000) : ((int)id < a.src_split ? q_lo : q_hi);
+      const bool hi = compact_hi(a, id);
+      qv[r] = CR ? (hi ? 0x10000 : 1) : (hi ? q_hi : q_lo);
       int sl = slot0 + (int)(e >> 24) + a.src_delay;
       while (sl >= B) sl -= B;
       slot[r] = sl;
@@ -700,11 +706,11 @@ __device__ __forceinline__ void deliver_quad_lds(const FusedArgs& a, const uint3
     while (sl >= B) sl -= B;
     if (q == 0) st_del += (unsigned long long)(s1 - s0);
     if (CR) {
-      const uint32_t inc = (int)id < a.src_split ? 1u : 0x10000u;
+      const uint32_t inc = compact_hi(a, id) ? 0x10000u : 1u;
       uint32_t* row = (uint32_t*)sring + (size_t)sl * nown;
       for (uint32_t k = s0 + (uint32_t)q; k < s1; k += kQuad) atomicAdd(&row[slrec[k]], inc);
     } else {
-      const unsigned long long qv = (unsigned long long)((int)id < a.src_split ? q_lo : q_hi);
+      const unsigned long long qv = (unsigned long long)(compact_hi(a, id) ? q_hi : q_lo);
       unsigned long long* row = (unsigned long long*)(sring + (size_t)sl * nown);
       for (uint32_t k = s0 + (uint32_t)q; k < s1; k += kQuad) atomicAdd(&row[slrec[k]], qv);
     }
@@ -722,7 +728,7 @@ __device__ __forceinline__ void deliver_lane_lds(const FusedArgs& a, uint32_t e,
   int sl = slot0 + (int)(e >> 24) + a.src_delay;
   while (sl >= B) sl -= B;
   st_del += (unsigned long long)(s1 - s0);
-  const bool lo = (int)id < a.src_split;
+  const bool lo = !compact_hi(a, id);
   uint32_t* crow = (uint32_t*)sring + (size_t)sl * nown;
   unsigned long long* row = (unsigned long long*)(sring + (size_t)sl * nown);
   const uint32_t inc = lo ? 1u : 0x10000u;
