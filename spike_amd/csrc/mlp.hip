@@ -22,10 +22,12 @@
 // the hardware orders the 32 reduction indices within one instruction.
 //
 // Tensors that a later kernel reads as MFMA operands are stored in "fragment order" FL:
-// for a matrix X[m][c] (m = batch row, c = column; M rows in all)
-//   FL(m, c) = ((c / 16) (M / 32) + m / 32) * 512 + ((c % 16) + 16 ((m % 32) / 8)) * 8 + m % 8
+// for a matrix X[m][c] (m = batch row, c = column; C columns in all)
+//   FL(m, c) = ((m / 32) (C / 16) + c / 16) * 512 + ((c % 16) + 16 ((m % 32) / 8)) * 8 + m % 8
 // so that one 16-byte load per lane fetches an operand fragment with the reduction running
-// over rows -- what the weight gradient needs for both dZ and A.
+// over rows -- what the weight gradient needs for both dZ and A.  The fragments of 32 rows lie
+// in a row: with all rows of 16 columns together, the fragments that are read at one time were
+// a power of two apart, on the same memory channels.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -55,10 +57,13 @@ constexpr int DIN = SPK_MLP_INPUTS;
 constexpr int DOUT = SPK_MLP_OUTPUTS;
 constexpr int K1 = 32;     // first-layer reduction: features hi (0..4), lo (5..9), zeros
 constexpr int NO = 16;     // output layer padded to one 16-column block
-constexpr int MT = SPK_MLP_ROW_TILE;  // rows per workgroup
+constexpr int MT = SPK_MLP_ROW_TILE;  // rows per workgroup at most (a batch is a multiple of it)
 constexpr int NT = 256;    // threads per workgroup (4 waves; wave w owns columns 64w..64w+63)
+constexpr int NW = NT / 64;
+constexpr int CW = H / NW, NB = CW / 16;   // columns of a wave, in blocks of 16
 constexpr int LS = H + 8;  // LDS row stride in bf16 (16-byte pad: conflict-free operand reads)
-constexpr int LDS_BYTES = MT * LS * 2 + 64;
+constexpr int NLOSS = 64;  // rows per partial loss (those of the smaller tile)
+constexpr size_t lds_bytes(int mt) { return (size_t)mt * LS * 2 + 4 * H * sizeof(float); }   // tile, biases
 constexpr uint32_t kStreamBatch = 4;
 
 // FP32 master layout (per member)
@@ -70,13 +75,21 @@ constexpr int oW5 = ob4 + H, ob5 = oW5 + DOUT * H;
 constexpr int P = ob5 + DOUT;
 static_assert(P == SPK_MLP_PARAMS, "parameter count");
 
-// BF16 working copies (per member)
+// BF16 working copies (per member), every matrix in operand order (wf_index): a wavefront's
+// load of one fragment is 1 KB in a row.  From [row][column] matrices the same load touched
+// half of 16 lines.
 constexpr int bW1 = 0;               // [256][32]: W1 in columns 0..4 and again in 5..9
 constexpr int bW = bW1 + H * K1;     // layers 2..4, [256][256] each, W[out][in]
 constexpr int bWT = bW + 3 * H * H;  // layers 2..4 transposed, WT[in][out]
 constexpr int bW5 = bWT + 3 * H * H; // [16][256]: rows 0..2 = W5
 constexpr int bW5T = bW5 + NO * H;   // [256][32]: W5T[k][o] = W5[o][k], o < 3
 constexpr int BF = bW5T + H * 32;
+
+// Place of W[n][k] of a matrix of K columns in operand order: fragment (n / 16, k / 32), in it
+// lane n % 16 + 16 (k % 32 / 8), element k % 8.
+__host__ __device__ constexpr int wf_index(int n, int k, int K) {
+  return ((n >> 4) * (K >> 5) + (k >> 5)) * 512 + ((n & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
 
 constexpr int oW[5] = {oW1, oW2, oW3, oW4, oW5};
 constexpr int ob[5] = {ob1, ob2, ob3, ob4, ob5};
@@ -108,63 +121,77 @@ __device__ __forceinline__ f32x4 mfma(u16x8 a, u16x8 b, f32x4 c) {
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-__device__ __forceinline__ size_t fl_index(int M, int m, int c) {
-  return ((size_t)(c >> 4) * (size_t)(M >> 5) + (size_t)(m >> 5)) * 512 +
+__device__ __forceinline__ size_t fl_index(int C, int m, int c) {
+  return ((size_t)(m >> 5) * (size_t)(C >> 4) + (size_t)(c >> 4)) * 512 +
          (size_t)(((c & 15) + 16 * ((m & 31) >> 3)) * 8 + (m & 7));
 }
 
-// Columns [0, C) of the LDS tile (rows 0..MT-1 = batch rows m0..) into fragment order.
-__device__ __forceinline__ void store_fl(const uint16_t* lds, int C, uint16_t* dst, int M, int m0,
-                                         int w, int lane) {
-  const int nmb = MT / 32;
+// Columns [0, C) of the LDS tile (rows 0..TILE-1 = batch rows m0..) into fragment order.
+template <int TILE>
+__device__ __forceinline__ void store_fl(const uint16_t* lds, int C, uint16_t* dst, int m0, int w, int lane) {
+  const int nmb = TILE / 32;
   const int nblk = (C / 16) * nmb;
-  for (int b = w; b < nblk; b += 4) {
-    const int cb = b / nmb, mb = b - cb * nmb;
+  for (int b = w; b < nblk; b += NW) {
+    const int mb = b / (C / 16), cb = b - mb * (C / 16);
     const int c = cb * 16 + (lane & 15), r = mb * 32 + (lane >> 4) * 8;
     u16x8 v;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = lds[(r + j) * LS + c];
-    *(u16x8*)(dst + fl_index(M, m0 + r, c)) = v;
+    *(u16x8*)(dst + fl_index(C, m0 + r, c)) = v;
   }
 }
 
-// Transposed tile product: acc[nb][mb] += W[64 w + 16 nb.., k] . lds[16 mb.., k] over KS steps
+// Transposed tile product: acc[nb][mb] += W[32 w + 16 nb.., k] . lds[16 mb.., k] over KS steps
 // of 32 (K = 32 KS), i.e. Z^T = W A^T.  Result element r of acc[nb][mb] belongs to batch
-// row m = 16 mb + lane % 16 and output n = 64 w + 16 nb + 4 (lane / 16) + r: every lane
+// row m = 16 mb + lane % 16 and output n = 32 w + 16 nb + 4 (lane / 16) + r: every lane
 // holds four consecutive outputs of one row, which it writes back as one 8-byte LDS store.
+// `wf` holds the weight fragments of the first step (load_w, issued before the previous
+// layer's epilogue); those of step ks + 1, and the activations of the next half step, are in
+// flight while this one multiplies.
 template <int KS>
+__device__ __forceinline__ void load_w(const uint16_t* __restrict__ W, int w, int lane, int ks, u16x8 (&wf)[NB]) {
+  const uint16_t* wp = W + ((size_t)(CW / 16 * w) * KS + ks) * 512 + lane * 8;
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) wf[nb] = *(const u16x8*)(wp + (size_t)nb * KS * 512);
+}
+
+template <int KS, int MB>
 __device__ __forceinline__ void mm_tile(const uint16_t* lds, const uint16_t* __restrict__ W, int w, int lane,
-                                        f32x4 (&acc)[4][8]) {
-  constexpr int K = 32 * KS;
-  const int r16 = lane & 15, kg = (lane >> 4) * 8;
-  const uint16_t* wp = W + (size_t)(64 * w + r16) * K + kg;
-  // weight fragments of step ks + 1 are in flight while step ks multiplies
-  u16x8 wf[4], wn[4];
+                                        u16x8 (&wf)[NB], f32x4 (&acc)[NB][MB]) {
+  const uint16_t* ap = lds + (lane & 15) * LS + (lane >> 4) * 8;
+  u16x8 wn[NB], af[2][MB / 2];
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) wf[nb] = *(const u16x8*)(wp + (size_t)16 * nb * K);
-#pragma unroll 2
+  for (int i = 0; i < MB / 2; ++i) af[0][i] = *(const u16x8*)(ap + 16 * i * LS);
+#pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
-    if (ks + 1 < KS) {
+    if (ks + 1 < KS) load_w<KS>(W, w, lane, ks + 1, wn);
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) wn[nb] = *(const u16x8*)(wp + (size_t)16 * nb * K + (ks + 1) * 32);
+    for (int h = 0; h < 2; ++h) {
+      const int mn = h == 0 ? MB / 2 : 0, kn = h == 0 ? ks : ks + 1;
+      if (kn < KS) {
+#pragma unroll
+        for (int i = 0; i < MB / 2; ++i) af[h ^ 1][i] = *(const u16x8*)(ap + 16 * (mn + i) * LS + kn * 32);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < MB / 2; ++i)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          acc[nb][h * (MB / 2) + i] = mfma(wf[nb], af[h][i], acc[nb][h * (MB / 2) + i]);
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int mb = 0; mb < 8; ++mb) {
-      const u16x8 af = *(const u16x8*)(lds + (16 * mb + r16) * LS + ks * 32 + kg);
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) acc[nb][mb] = mfma(wf[nb], af, acc[nb][mb]);
-    }
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) wf[nb] = wn[nb];
+    for (int nb = 0; nb < NB; ++nb) wf[nb] = wn[nb];
   }
 }
 
+template <int MB>
 __device__ __forceinline__ size_t slope_index(int tile, int w, int nb, int mb, int lane) {
-  return ((((size_t)tile * 4 + w) * 4 + nb) * 8 + mb) * 256 + (size_t)lane * 4;
+  return ((((size_t)tile * NW + w) * NB + nb) * MB + mb) * 256 + (size_t)lane * 4;
 }
 
 __device__ __forceinline__ uint16_t* lds_quad(uint16_t* lds, int w, int nb, int mb, int lane) {
-  return lds + (16 * mb + (lane & 15)) * LS + 64 * w + 16 * nb + 4 * (lane >> 4);
+  return lds + (16 * mb + (lane & 15)) * LS + CW * w + 16 * nb + 4 * (lane >> 4);
 }
 
 struct FwdArgs {
@@ -182,18 +209,23 @@ struct FwdArgs {
   uint16_t* slopes;      // [E][4][H*M] SiLU slopes in result-fragment order
 };
 
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_mlp_forward(FwdArgs a) {
+template <bool TRAIN, int TILE>
+__global__ __launch_bounds__(NT, TILE == MT ? 2 : 3) void k_mlp_forward(FwdArgs a) {
+  constexpr int MB = TILE / 16;
   extern __shared__ __align__(16) uint16_t lds[];
+  float* lbias = (float*)(lds + TILE * LS);   // biases of layers 1..4
   const int tile = blockIdx.x, e = blockIdx.y;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int m0 = tile * MT;
+  const int m0 = tile * TILE;
   const int M = a.M;
   const uint16_t* wb = a.wb + (size_t)e * BF;
   const float* mst = a.master + (size_t)e * P;
-  const bool train = a.acts != nullptr;
 
+#pragma unroll
+  for (int l = 0; l < 4; ++l) lbias[l * H + tid] = mst[ob[l] + tid];
+  static_assert(NT == H, "a bias per thread and layer");
   // features -> hi/lo bf16 pairs in LDS columns 0..9, zeros up to 31
-  if (tid < MT) {
+  if (tid < TILE) {
     const int r = m0 + tid;
     int64_t i;
     if (a.mode == 1) {
@@ -215,69 +247,72 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
     for (int j = 2 * DIN; j < K1; ++j) row[j] = 0;
   }
   __syncthreads();
-  if (train) store_fl(lds, K1, a.acts + ((size_t)e * 5 + 0) * H * M, M, m0, w, lane);
+  if constexpr (TRAIN) store_fl<TILE>(lds, K1, a.acts + ((size_t)e * 5 + 0) * H * M, m0, w, lane);
 
-  const int ng = 4 * (lane >> 4);
+  // a layer's first weights, loaded before the epilogue of the layer before
+  u16x8 wf[NB];
+  load_w<1>(wb + bW1, w, lane, 0, wf);
   for (int l = 1; l <= 4; ++l) {
-    f32x4 acc[4][8];
-    const float* bias = mst + ob[l - 1] + 64 * w + ng;
+    f32x4 acc[NB][MB];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const float* bq = bias + 16 * nb;  // member stride P is odd: four scalar loads
-      const f32x4 bv = {bq[0], bq[1], bq[2], bq[3]};
+    for (int nb = 0; nb < NB; ++nb) {
+      const f32x4 bv = *(const f32x4*)(lbias + (l - 1) * H + CW * w + 16 * nb + 4 * (lane >> 4));
 #pragma unroll
-      for (int mb = 0; mb < 8; ++mb) acc[nb][mb] = bv;
+      for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = bv;
     }
     if (l == 1)
-      mm_tile<1>(lds, wb + bW1, w, lane, acc);
+      mm_tile<1, MB>(lds, wb + bW1, w, lane, wf, acc);
     else
-      mm_tile<8>(lds, wb + bW + (size_t)(l - 2) * H * H, w, lane, acc);
+      mm_tile<8, MB>(lds, wb + bW + (size_t)(l - 2) * H * H, w, lane, wf, acc);
+    if (l < 4) load_w<8>(wb + bW + (size_t)(l - 1) * H * H, w, lane, 0, wf);
     __syncthreads();  // every wave has read the layer input
-    uint16_t* sl = train ? a.slopes + ((size_t)e * 4 + (l - 1)) * H * M : nullptr;
+    uint16_t* sl = TRAIN ? a.slopes + ((size_t)e * 4 + (l - 1)) * H * M : nullptr;
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int mb = 0; mb < 8; ++mb) {
+      for (int mb = 0; mb < MB; ++mb) {
         const f32x4 z = acc[nb][mb];
         const f32x4 sg = {sigmoid(z[0]), sigmoid(z[1]), sigmoid(z[2]), sigmoid(z[3])};
         *(u16x4*)lds_quad(lds, w, nb, mb, lane) = pack4(z[0] * sg[0], z[1] * sg[1], z[2] * sg[2], z[3] * sg[3]);
-        if (train)
-          *(u16x4*)(sl + slope_index(tile, w, nb, mb, lane)) =
+        if constexpr (TRAIN)
+          *(u16x4*)(sl + slope_index<MB>(tile, w, nb, mb, lane)) =
               pack4(sg[0] * (1.0f + z[0] * (1.0f - sg[0])), sg[1] * (1.0f + z[1] * (1.0f - sg[1])),
                     sg[2] * (1.0f + z[2] * (1.0f - sg[2])), sg[3] * (1.0f + z[3] * (1.0f - sg[3])));
       }
     __syncthreads();
-    if (train) store_fl(lds, H, a.acts + ((size_t)e * 5 + l) * H * M, M, m0, w, lane);
+    if constexpr (TRAIN) store_fl<TILE>(lds, H, a.acts + ((size_t)e * 5 + l) * H * M, m0, w, lane);
   }
 
-  // output layer, transposed: Y^T = W5 A4^T; wave w takes row blocks 2w, 2w+1; lanes 0..15
-  // hold outputs 0..3 (3 used) of row 16 mb + lane
+  // output layer, transposed: Y^T = W5 A4^T; wave w takes row block w; lanes 0..15 hold
+  // outputs 0..3 (3 used) of row 16 w + lane
   {
     const int r16 = lane & 15, kg = (lane >> 4) * 8;
-    f32x4 o0 = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (lane < 16) o0 = f32x4{mst[ob5], mst[ob5 + 1], mst[ob5 + 2], 0.0f};
-    f32x4 o1 = o0;
-    const uint16_t* wp = wb + bW5 + (size_t)r16 * H + kg;
+    const uint16_t* wp = wb + bW5 + lane * 8;
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-      const u16x8 wf = *(const u16x8*)(wp + ks * 32);
-      const u16x8 a0 = *(const u16x8*)(lds + (32 * w + r16) * LS + ks * 32 + kg);
-      const u16x8 a1 = *(const u16x8*)(lds + (32 * w + 16 + r16) * LS + ks * 32 + kg);
-      o0 = mfma(wf, a0, o0);
-      o1 = mfma(wf, a1, o1);
-    }
-    if (lane < 16) {
-      const int ra = m0 + 32 * w + lane, rb2 = ra + 16;
-      if (ra < M) {
-        float* yp = a.y + ((size_t)e * M + ra) * DOUT;
-        yp[0] = o0[0]; yp[1] = o0[1]; yp[2] = o0[2];
-      }
-      if (rb2 < M) {
-        float* yp = a.y + ((size_t)e * M + rb2) * DOUT;
-        yp[0] = o1[0]; yp[1] = o1[1]; yp[2] = o1[2];
+    for (int rb = 0; rb < MB; rb += NW) {
+      const int row = 16 * (rb + w);
+      f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+      if (lane < 16) o = f32x4{mst[ob5], mst[ob5 + 1], mst[ob5 + 2], 0.0f};
+#pragma unroll
+      for (int ks = 0; ks < 8; ++ks)
+        o = mfma(*(const u16x8*)(wp + ks * 512), *(const u16x8*)(lds + (row + r16) * LS + ks * 32 + kg), o);
+      const int r = m0 + row + lane;
+      if (lane < 16 && r < M) {
+        float* yp = a.y + ((size_t)e * M + r) * DOUT;
+        yp[0] = o[0]; yp[1] = o[1]; yp[2] = o[2];
       }
     }
   }
+}
+
+// What all parameters of an Adam step share, computed by the thread that counts the step (per
+// parameter: two powf and a cosf each).
+constexpr float kBeta1 = 0.9f, kBeta2 = 0.999f;
+__device__ __forceinline__ void adam_uniform(int t, float lr0, float lr_min, int total, float* uni) {
+  const float u = (float)min(max(t - 1, 0), total) / (float)max(total, 1);
+  uni[0] = lr_min + 0.5f * (lr0 - lr_min) * (1.0f + cosf(3.14159265358979f * u));
+  uni[1] = 1.0f - powf(kBeta1, (float)t);
+  uni[2] = 1.0f - powf(kBeta2, (float)t);
 }
 
 struct BwdArgs {
@@ -289,25 +324,32 @@ struct BwdArgs {
   float scale;            // 2 / M
   const uint16_t* slopes; // [E][4][H*M]
   uint16_t* grads;        // [E][5][H*M]: FL(dZ_1..dZ_4) in slots 0..3, FL(dY) (16 columns) in 4
-  float* loss_part;       // [E][tiles]
-  int* step;              // incremented once when tick != 0
+  float* loss_part;       // [E][M / NLOSS]
+  int* step;              // incremented once when tick != 0, which also sets uni (adam_uniform)
   int tick;
+  float lr0, lr_min;
+  int total;
+  float* uni;
   int M;
 };
 
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_mlp_backward(BwdArgs a) {
+template <int TILE>
+__global__ __launch_bounds__(NT, TILE == MT ? 2 : 3) void k_mlp_backward(BwdArgs a) {
+  constexpr int MB = TILE / 16;
   extern __shared__ __align__(16) uint16_t lds[];
-  float* red = (float*)(lds + MT * LS);
-  const int tile = blockIdx.x, e = blockIdx.y, tiles = gridDim.x;
+  const int tile = blockIdx.x, e = blockIdx.y;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int m0 = tile * MT, M = a.M;
+  const int m0 = tile * TILE, M = a.M;
   const uint16_t* wb = a.wb + (size_t)e * BF;
 
-  if (a.tick && tile == 0 && e == 0 && tid == 0) *a.step += 1;
+  if (a.tick && tile == 0 && e == 0 && tid == 0) {
+    *a.step += 1;
+    adam_uniform(*a.step, a.lr0, a.lr_min, a.total, a.uni);
+  }
 
   // output gradient dy = bf16(2 w_o (y - t) / M) in LDS columns 0..2, zeros up to 31
   float lsum = 0.0f;
-  if (tid < MT) {
+  if (tid < TILE) {
     const int r = m0 + tid;
     const int64_t i = a.idx ? a.idx[(size_t)e * M + r] : r;
     const float wo[3] = {a.w0, a.w1, a.w2};
@@ -321,38 +363,41 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
 #pragma unroll
     for (int j = DOUT; j < K1; ++j) row[j] = 0;
   }
-  // per-tile loss, summed in a fixed order
+  // loss of every NLOSS rows, summed in a fixed order
+  static_assert(NLOSS == 64, "rows of a wavefront");
 #pragma unroll
   for (int s = 32; s > 0; s >>= 1) lsum += __shfl_xor(lsum, s);
-  if (lane == 0) red[w] = lsum;
+  if (lane == 0 && w < TILE / NLOSS) a.loss_part[(size_t)e * (M / NLOSS) + m0 / NLOSS + w] = lsum;
   __syncthreads();
-  if (tid == 0) a.loss_part[(size_t)e * tiles + tile] = (red[0] + red[1]) + (red[2] + red[3]);
-  store_fl(lds, NO, a.grads + ((size_t)e * 5 + 4) * H * M, M, m0, w, lane);
+  store_fl<TILE>(lds, NO, a.grads + ((size_t)e * 5 + 4) * H * M, m0, w, lane);
 
+  u16x8 wf[NB];
+  load_w<1>(wb + bW5T, w, lane, 0, wf);
   for (int l = 4; l >= 1; --l) {
     // dA_l^T = W_(l+1)^T dZ_(l+1)^T  (for l = 4: W5^T dY^T)
-    f32x4 acc[4][8];
+    f32x4 acc[NB][MB];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int mb = 0; mb < 8; ++mb) acc[nb][mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     if (l == 4)
-      mm_tile<1>(lds, wb + bW5T, w, lane, acc);
+      mm_tile<1, MB>(lds, wb + bW5T, w, lane, wf, acc);
     else
-      mm_tile<8>(lds, wb + bWT + (size_t)(l - 1) * H * H, w, lane, acc);
+      mm_tile<8, MB>(lds, wb + bWT + (size_t)(l - 1) * H * H, w, lane, wf, acc);
+    if (l > 1) load_w<8>(wb + bWT + (size_t)(l - 2) * H * H, w, lane, 0, wf);
     __syncthreads();
     const uint16_t* sl = a.slopes + ((size_t)e * 4 + (l - 1)) * H * M;
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-      for (int mb = 0; mb < 8; ++mb) {
-        const u16x4 sv = *(const u16x4*)(sl + slope_index(tile, w, nb, mb, lane));
+      for (int mb = 0; mb < MB; ++mb) {
+        const u16x4 sv = *(const u16x4*)(sl + slope_index<MB>(tile, w, nb, mb, lane));
         const f32x4 d = acc[nb][mb];
         *(u16x4*)lds_quad(lds, w, nb, mb, lane) =
             pack4(d[0] * from_bf16(sv[0]), d[1] * from_bf16(sv[1]), d[2] * from_bf16(sv[2]), d[3] * from_bf16(sv[3]));
       }
     __syncthreads();
-    store_fl(lds, H, a.grads + ((size_t)e * 5 + (l - 1)) * H * M, M, m0, w, lane);
+    store_fl<TILE>(lds, H, a.grads + ((size_t)e * 5 + (l - 1)) * H * M, m0, w, lane);
   }
 }
 
@@ -361,27 +406,40 @@ struct WgradArgs {
   const uint16_t* grads;  // [E][5][H*M]
   float* part;            // [E][S][P]
   int M, chunk;           // rows, rows per split
+  int S, models;
 };
+
+// Workgroups of layers 2..4 for `se` splits of members: four for each, in groups of 8 XCDs.
+__host__ __device__ constexpr int wgrad_big_blocks(int se) { return (3 * se + 7) / 8 * 32; }
 
 // 56 wave jobs per member and split: dW1 (4 row tiles of 64 x 32 columns), dW2..dW4
 // (16 tiles of 64 x 64 each), dW5 (4 tiles of 16 rows x 64 columns); the first column
-// tile of each layer also sums the bias gradient.
+// tile of each layer also sums the bias gradient.  A workgroup takes the four tiles of one
+// row of a layer, which share their dZ; the four workgroups of a layer share its A and follow
+// each other at a distance of 8 in the grid, on one XCD, whose L2 then reads A once.  Layers 2
+// to 4 of every member and split come first, then the two small layers.
 __global__ __launch_bounds__(NT) void k_mlp_wgrad(WgradArgs a) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int job = blockIdx.x * 4 + w, s = blockIdx.y, e = blockIdx.z;
-  const int S = gridDim.y, M = a.M;
-  int layer, n0, k0, nrb, ncb;
-  if (job < 4) {
-    layer = 1; n0 = 64 * job; k0 = 0; nrb = 4; ncb = 2;
-  } else if (job < 52) {
-    const int q = job - 4;
-    layer = 2 + q / 16; n0 = 64 * ((q % 16) / 4); k0 = 64 * (q % 4); nrb = 4; ncb = 4;
+  const int S = a.S, M = a.M, SE = S * a.models, big = wgrad_big_blocks(SE);
+  int layer, n0, k0, nrb, ncb, se;
+  if ((int)blockIdx.x < big) {
+    const int g = ((int)blockIdx.x / 32) * 8 + (int)blockIdx.x % 8;   // layer, split and member
+    if (g >= 3 * SE) return;
+    layer = 2 + g / SE; se = g % SE;
+    n0 = 64 * (((int)blockIdx.x / 8) % 4); k0 = 64 * w; nrb = 4; ncb = 4;
   } else {
-    layer = 5; n0 = 0; k0 = 64 * (job - 52); nrb = 1; ncb = 4;
+    const int q = (int)blockIdx.x - big;
+    se = q % SE;
+    if (q < SE) {
+      layer = 1; n0 = 64 * w; k0 = 0; nrb = 4; ncb = 2;
+    } else {
+      layer = 5; n0 = 0; k0 = 64 * w; nrb = 1; ncb = 4;
+    }
   }
+  const int s = se % S, e = se / S;
   const uint16_t* dz = a.grads + ((size_t)e * 5 + (layer - 1)) * H * M;  // layer 5: dY
   const uint16_t* ac = a.acts + ((size_t)e * 5 + (layer - 1)) * H * M;
-  const int nmb = M >> 5;
+  const int dcb = layer == 5 ? 1 : H / 16, acb = layer == 1 ? K1 / 16 : H / 16;   // column blocks of dZ and A
   const int mb0 = (s * a.chunk) >> 5, mb1 = mb0 + (a.chunk >> 5);
   f32x4 acc[4][4];
   float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -390,24 +448,38 @@ __global__ __launch_bounds__(NT) void k_mlp_wgrad(WgradArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   const bool bias = k0 == 0;
-  for (int mb = mb0; mb < mb1; ++mb) {
-    u16x8 bv[4], av[4];
+  // fragments of the next 96 rows are in flight while 32 multiply
+  u16x8 bv[4][4], av[4][4];
+  auto load = [&](int mb, int k) {
 #pragma unroll
     for (int cb = 0; cb < 4; ++cb)
-      if (cb < ncb) bv[cb] = *(const u16x8*)(ac + ((size_t)((k0 >> 4) + cb) * nmb + mb) * 512 + lane * 8);
+      if (cb < ncb) bv[k][cb] = *(const u16x8*)(ac + ((size_t)mb * acb + (k0 >> 4) + cb) * 512 + lane * 8);
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
-      if (rb < nrb) av[rb] = *(const u16x8*)(dz + ((size_t)((n0 >> 4) + rb) * nmb + mb) * 512 + lane * 8);
+      if (rb < nrb) av[k][rb] = *(const u16x8*)(dz + ((size_t)mb * dcb + (n0 >> 4) + rb) * 512 + lane * 8);
+  };
+  auto mul = [&](int k) {
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb) {
       if (rb >= nrb) continue;
       if (bias) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) rs[rb] += from_bf16(av[rb][j]);
+        for (int j = 0; j < 8; ++j) rs[rb] += from_bf16(av[k][rb][j]);
       }
 #pragma unroll
       for (int cb = 0; cb < 4; ++cb)
-        if (cb < ncb) acc[rb][cb] = mfma(av[rb], bv[cb], acc[rb][cb]);
+        if (cb < ncb) acc[rb][cb] = mfma(av[k][rb], bv[k][cb], acc[rb][cb]);
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < 3; ++k) load(mb0 + k, k);
+  for (int mb = mb0; mb < mb1; mb += 4) {   // (chunks are multiples of 128 rows)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (mb + k + 3 < mb1) load(mb + k + 3, (k + 3) & 3);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(k);
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
   float* out = a.part + ((size_t)e * S + s) * P;
@@ -448,8 +520,7 @@ struct AdamArgs {
   const float* part; int S;   // partial gradients [E][S][P] (or)
   const float* gin;           // caller gradients [E][P]
   float* gout;                // gradients [E][P] (optional)
-  const int* step;
-  float lr0, lr_min; int total;
+  const float* uni;           // learning rate and bias corrections of the step (adam_uniform)
   int apply;                  // 0: gradients only; 1: Adam step; 2: write the BF16 copies only
 };
 
@@ -457,8 +528,8 @@ __device__ __forceinline__ void write_copies(uint16_t* wb, int p, float v) {
   const uint16_t h = to_bf16(v);
   if (p < ob1) {
     const int n = p / DIN, k = p - n * DIN;
-    wb[bW1 + n * K1 + k] = h;
-    wb[bW1 + n * K1 + DIN + k] = h;
+    wb[bW1 + wf_index(n, k, K1)] = h;
+    wb[bW1 + wf_index(n, DIN + k, K1)] = h;
   } else if (p >= oW2 && p < oW5) {
     int L = -1, q = 0;
     if (p < ob2) {
@@ -470,19 +541,37 @@ __device__ __forceinline__ void write_copies(uint16_t* wb, int p, float v) {
     }
     if (L >= 0) {  // biases of layers 2..4 have no working copy
       const int n = q >> 8, k = q & 255;
-      wb[bW + L * H * H + n * H + k] = h;
-      wb[bWT + L * H * H + k * H + n] = h;
+      wb[bW + L * H * H + wf_index(n, k, H)] = h;
+      wb[bWT + L * H * H + wf_index(k, n, H)] = h;
     }
   } else if (p >= oW5 && p < ob5) {
     const int o = (p - oW5) >> 8, k = (p - oW5) & 255;
-    wb[bW5 + o * H + k] = h;
-    wb[bW5T + k * 32 + o] = h;
+    wb[bW5 + wf_index(o, k, H)] = h;
+    wb[bW5T + wf_index(k, o, 32)] = h;
   }
 }
 
+// The parameter of a thread: tiles of 8 outputs x 32 inputs of the big matrices (a wavefront
+// 8 x 8, whose working copies W and W^T are runs of 128 bytes each), then the other parameters
+// in order; -1: none.  In plain order the copies W^T went out two bytes at a time into lines
+// that eight XCDs shared.
+constexpr int kAdamBig = 3 * H * H / 256, kAdamBlocks = kAdamBig + (P - 3 * H * H + 255) / 256;
+__device__ __forceinline__ int adam_param(int block, int tid) {
+  if (block < kAdamBig) {
+    const int l = block / (H * H / 256), q = block % (H * H / 256);
+    const int n = q / (H / 32) * 8 + (tid & 7), k = q % (H / 32) * 32 + (tid >> 3);
+    return (l == 0 ? oW2 : l == 1 ? oW3 : oW4) + n * H + k;
+  }
+  const int r = (block - kAdamBig) * 256 + tid;   // W1, b1 | b2 | b3 | b4, W5, b5
+  if (r < oW2) return r;
+  if (r < oW2 + H) return ob2 + r - oW2;
+  if (r < oW2 + 2 * H) return ob3 + r - oW2 - H;
+  return r < P - 3 * H * H ? ob4 + r - oW2 - 2 * H : -1;
+}
+
 __global__ __launch_bounds__(256) void k_mlp_adam(AdamArgs a) {
-  const int p = blockIdx.x * 256 + threadIdx.x, e = blockIdx.y;
-  if (p >= P) return;
+  const int p = adam_param(blockIdx.x, threadIdx.x), e = blockIdx.y;
+  if (p < 0) return;
   const size_t ep = (size_t)e * P + p;
   float* mst = a.master + ep;
   uint16_t* wb = a.wb + (size_t)e * BF;
@@ -500,22 +589,22 @@ __global__ __launch_bounds__(256) void k_mlp_adam(AdamArgs a) {
   }
   if (a.gout) a.gout[ep] = g;
   if (!a.apply) return;
-  const int t = *a.step;
-  const float u = (float)min(max(t - 1, 0), a.total) / (float)max(a.total, 1);
-  const float lr = a.lr_min + 0.5f * (a.lr0 - a.lr_min) * (1.0f + cosf(3.14159265358979f * u));
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  const float b1 = kBeta1, b2 = kBeta2, eps = 1e-8f;
+  const float lr = a.uni[0], c1 = a.uni[1], c2 = a.uni[2];
   const float m = b1 * a.mom[ep] + (1.0f - b1) * g;
   const float v = b2 * a.vel[ep] + (1.0f - b2) * g * g;
   a.mom[ep] = m;
   a.vel[ep] = v;
-  const float c1 = 1.0f - powf(b1, (float)t), c2 = 1.0f - powf(b2, (float)t);
   const float val = *mst - lr * (m / c1) / (sqrtf(v / c2) + eps);
   *mst = val;
   write_copies(wb, p, val);
 }
 
-__global__ void k_mlp_tick(int* step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
+__global__ void k_mlp_tick(int* step, float lr, float* uni) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    *step += 1;
+    adam_uniform(*step, lr, lr, 1, uni);
+  }
 }
 
 }  // namespace
@@ -534,6 +623,7 @@ struct spk_mlp {
   uint16_t *acts = nullptr, *slopes = nullptr, *grads = nullptr;
   float *part = nullptr, *loss_part = nullptr, *gbuf = nullptr, *gin = nullptr;
   int* step = nullptr;
+  float* uni = nullptr;
   float *px = nullptr, *py = nullptr;
   int64_t pcap = 0;
   float* scratch = nullptr;  // this device's copy of the file-scope staging array
@@ -612,10 +702,30 @@ void free_d(T*& p) {
 int lds_attributes() {
   static int done = 0;
   if (done) return SPK_OK;
-  MLP_HIP(hipFuncSetAttribute((const void*)k_mlp_forward, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
-  MLP_HIP(hipFuncSetAttribute((const void*)k_mlp_backward, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_BYTES));
+  for (const void* fn : {(const void*)k_mlp_forward<false, MT>, (const void*)k_mlp_forward<true, MT>,
+                         (const void*)k_mlp_backward<MT>})
+    MLP_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes(MT)));
   done = 1;
   return SPK_OK;
+}
+
+// Row tile of the passes over `rows` rows of `models` members.
+bool half_tiles(int64_t rows, int models) { return (rows + MT - 1) / MT * models <= 512; }
+
+template <bool TRAIN>
+void launch_forward(const FwdArgs& f, int models, hipStream_t st) {
+  if (half_tiles(f.M, models))
+    hipLaunchKernelGGL((k_mlp_forward<TRAIN, MT / 2>), dim3((unsigned)(((int64_t)f.M + MT / 2 - 1) / (MT / 2)), models), dim3(NT),
+                       lds_bytes(MT / 2), st, f);
+  else
+    hipLaunchKernelGGL((k_mlp_forward<TRAIN, MT>), dim3((unsigned)(((int64_t)f.M + MT - 1) / MT), models), dim3(NT), lds_bytes(MT), st, f);
+}
+
+void launch_backward(const BwdArgs& b, int models, hipStream_t st) {
+  if (half_tiles(b.M, models))
+    hipLaunchKernelGGL(k_mlp_backward<MT / 2>, dim3(b.M / (MT / 2), models), dim3(NT), lds_bytes(MT / 2), st, b);
+  else
+    hipLaunchKernelGGL(k_mlp_backward<MT>, dim3(b.M / MT, models), dim3(NT), lds_bytes(MT), st, b);
 }
 
 // Row chunks of the weight gradient: chunks of about 1024 rows (8 tiles), at most
@@ -632,32 +742,32 @@ int splits(int batch) {
 // one training step (forward, backward, weight gradient, Adam) on the surrogate's stream
 int enqueue_step(spk_mlp* m, int batch, int mode, uint64_t seed, int apply, float lr0, float lr_min, int total,
                  float* gout, float* loss_part, bool timed) {
-  const int tiles = batch / MT;
   FwdArgs f{};
   f.wb = m->wb; f.master = m->master; f.x = m->x; f.n = m->n; f.M = batch; f.mode = mode; f.seed = seed;
   f.step = m->step; f.idx = m->idx; f.y = m->y; f.acts = m->acts; f.slopes = m->slopes;
   if (timed) MLP_HIP(hipEventRecord(m->ev[0], m->stream));
-  hipLaunchKernelGGL(k_mlp_forward, dim3(tiles, m->E), dim3(NT), LDS_BYTES, m->stream, f);
+  launch_forward<true>(f, m->E, m->stream);
   if (timed) MLP_HIP(hipEventRecord(m->ev[1], m->stream));
   BwdArgs b{};
   b.wb = m->wb; b.y = m->y; b.t = m->t; b.idx = mode == 1 ? m->idx : nullptr;
   b.w0 = m->wout[0]; b.w1 = m->wout[1]; b.w2 = m->wout[2];
   b.scale = 2.0f / (float)batch;
   b.slopes = m->slopes; b.grads = m->grads; b.loss_part = loss_part; b.step = m->step; b.tick = apply == 1;
+  b.lr0 = lr0; b.lr_min = lr_min; b.total = total; b.uni = m->uni;
   b.M = batch;
-  hipLaunchKernelGGL(k_mlp_backward, dim3(tiles, m->E), dim3(NT), LDS_BYTES, m->stream, b);
+  launch_backward(b, m->E, m->stream);
   if (timed) MLP_HIP(hipEventRecord(m->ev[2], m->stream));
   const int S = splits(batch);
   const int chunk = batch / S;
   WgradArgs g{};
-  g.acts = m->acts; g.grads = m->grads; g.part = m->part; g.M = batch; g.chunk = chunk;
-  hipLaunchKernelGGL(k_mlp_wgrad, dim3(14, S, m->E), dim3(NT), 0, m->stream, g);
+  g.acts = m->acts; g.grads = m->grads; g.part = m->part; g.M = batch; g.chunk = chunk; g.S = S; g.models = m->E;
+  hipLaunchKernelGGL(k_mlp_wgrad, dim3(wgrad_big_blocks(S * m->E) + 2 * S * m->E), dim3(NT), 0, m->stream, g);
   if (timed) MLP_HIP(hipEventRecord(m->ev[3], m->stream));
   AdamArgs ad{};
   ad.master = m->master; ad.mom = m->mom; ad.vel = m->vel; ad.wb = m->wb; ad.part = m->part; ad.S = S;
-  ad.gin = nullptr; ad.gout = gout; ad.step = m->step; ad.lr0 = lr0; ad.lr_min = lr_min; ad.total = total;
+  ad.gin = nullptr; ad.gout = gout; ad.uni = m->uni;
   ad.apply = apply;
-  hipLaunchKernelGGL(k_mlp_adam, dim3((P + 255) / 256, m->E), dim3(256), 0, m->stream, ad);
+  hipLaunchKernelGGL(k_mlp_adam, dim3(kAdamBlocks, m->E), dim3(256), 0, m->stream, ad);
   if (timed) MLP_HIP(hipEventRecord(m->ev[4], m->stream));
   MLP_HIP(hipGetLastError());
   return SPK_OK;
@@ -719,9 +829,10 @@ int spk_mlp_create(int models, int max_batch, spk_mlp** out) {
   MLP_ALLOC(m->slopes, E * 4 * H * Mx);
   MLP_ALLOC(m->grads, E * 5 * H * Mx);
   MLP_ALLOC(m->part, E * S * P);
-  MLP_ALLOC(m->loss_part, E * (Mx / MT));
+  MLP_ALLOC(m->loss_part, E * (Mx / NLOSS));
   MLP_ALLOC(m->gbuf, E * P);
   MLP_ALLOC(m->step, 1);
+  MLP_ALLOC(m->uni, 3);
 #undef MLP_ALLOC
   hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
   if (e != hipSuccess) return bail(mfail(SPK_ERR_HIP, "hipStreamCreate failed"));
@@ -742,7 +853,7 @@ int spk_mlp_destroy(spk_mlp* m) {
   free_d(m->master); free_d(m->mom); free_d(m->vel); free_d(m->wb);
   free_d(m->x); free_d(m->t); free_d(m->idx); free_d(m->y);
   free_d(m->acts); free_d(m->slopes); free_d(m->grads);
-  free_d(m->part); free_d(m->loss_part); free_d(m->gbuf); free_d(m->gin); free_d(m->step);
+  free_d(m->part); free_d(m->loss_part); free_d(m->gbuf); free_d(m->gin); free_d(m->step); free_d(m->uni);
   free_d(m->px); free_d(m->py);
   for (auto& ev : m->ev)
     if (ev) (void)hipEventDestroy(ev);
@@ -768,7 +879,7 @@ int spk_mlp_set_params(spk_mlp* m, const float* params) {
   // padding entries of the working copies stay zero from creation; every used entry is rewritten
   AdamArgs ad{};
   ad.master = m->master; ad.wb = m->wb; ad.apply = 2;
-  hipLaunchKernelGGL(k_mlp_adam, dim3((P + 255) / 256, m->E), dim3(256), 0, m->stream, ad);
+  hipLaunchKernelGGL(k_mlp_adam, dim3(kAdamBlocks, m->E), dim3(256), 0, m->stream, ad);
   MLP_HIP(hipGetLastError());
   return spk_mlp_reset_optimizer(m);
 }
@@ -820,7 +931,7 @@ int spk_mlp_gradients(spk_mlp* m, int rows, float* grads, float* loss) {
   MLP_HIP(hipStreamSynchronize(m->stream));
   if (grads) MLP_HIP(hipMemcpy(grads, m->gbuf, (size_t)m->E * P * sizeof(float), hipMemcpyDeviceToHost));
   if (loss) {
-    const int tiles = rows / MT;
+    const int tiles = rows / NLOSS;
     std::vector<float> lp((size_t)m->E * tiles);
     MLP_HIP(hipMemcpy(lp.data(), m->loss_part, lp.size() * sizeof(float), hipMemcpyDeviceToHost));
     for (int e = 0; e < m->E; ++e) {
@@ -840,11 +951,10 @@ int spk_mlp_apply_gradients(spk_mlp* m, const float* grads, float lr) {
   int rc;
   if (!m->gin && (rc = malloc_d(&m->gin, (size_t)m->E * P))) return rc;
   MLP_HIP(hipMemcpyAsync(m->gin, grads, (size_t)m->E * P * sizeof(float), hipMemcpyHostToDevice, m->stream));
-  hipLaunchKernelGGL(k_mlp_tick, dim3(1), dim3(64), 0, m->stream, m->step);
+  hipLaunchKernelGGL(k_mlp_tick, dim3(1), dim3(64), 0, m->stream, m->step, lr, m->uni);
   AdamArgs ad{};
-  ad.master = m->master; ad.mom = m->mom; ad.vel = m->vel; ad.wb = m->wb; ad.gin = m->gin; ad.step = m->step;
-  ad.lr0 = lr; ad.lr_min = lr; ad.total = 1; ad.apply = 1;
-  hipLaunchKernelGGL(k_mlp_adam, dim3((P + 255) / 256, m->E), dim3(256), 0, m->stream, ad);
+  ad.master = m->master; ad.mom = m->mom; ad.vel = m->vel; ad.wb = m->wb; ad.gin = m->gin; ad.uni = m->uni; ad.apply = 1;
+  hipLaunchKernelGGL(k_mlp_adam, dim3(kAdamBlocks, m->E), dim3(256), 0, m->stream, ad);
   MLP_HIP(hipGetLastError());
   MLP_HIP(hipStreamSynchronize(m->stream));
   return SPK_OK;
@@ -861,7 +971,7 @@ int spk_mlp_train(spk_mlp* m, int steps, int batch, int mode, uint64_t seed, flo
     return mfail(SPK_ERR_STATE, "training set missing or smaller than the batch");
   if (!(lr0 >= 0.0f) || !(lr_min >= 0.0f) || !std::isfinite(lr0) || !std::isfinite(lr_min))
     return mfail(SPK_ERR_ARG, "bad learning rate");
-  const int tiles = batch / MT;
+  const int tiles = batch / NLOSS;
   float* lhist = nullptr;
   if (loss_per_step && steps > 0 && (rc = malloc_d(&lhist, (size_t)steps * m->E * tiles))) return rc;
   MLP_HIP(hipEventRecord(m->ev[5], m->stream));
@@ -929,9 +1039,8 @@ int spk_mlp_predict(spk_mlp* m, const float* features, int64_t n, float* out) {
   FwdArgs f{};
   f.wb = m->wb; f.master = m->master; f.x = m->px; f.n = n; f.M = (int)n; f.mode = 0;
   f.y = m->py;
-  const int tiles = (int)((n + MT - 1) / MT);
   MLP_HIP(hipEventRecord(m->ev[0], m->stream));
-  hipLaunchKernelGGL(k_mlp_forward, dim3(tiles, m->E), dim3(NT), LDS_BYTES, m->stream, f);
+  launch_forward<false>(f, m->E, m->stream);
   MLP_HIP(hipEventRecord(m->ev[1], m->stream));
   MLP_HIP(hipGetLastError());
   MLP_HIP(hipMemcpyAsync(out, m->py, (size_t)m->E * n * DOUT * sizeof(float), hipMemcpyDeviceToHost, m->stream));
@@ -956,9 +1065,8 @@ int spk_mlp_predict_noalloc(spk_mlp* m, const float* features, int64_t n, float*
   FwdArgs f{};
   f.wb = m->wb; f.master = m->master; f.x = px; f.n = n; f.M = (int)n; f.mode = 0;
   f.y = py;
-  const int tiles = (int)((n + MT - 1) / MT);
   MLP_HIP(hipEventRecord(m->ev[0], m->stream));
-  hipLaunchKernelGGL(k_mlp_forward, dim3(tiles, m->E), dim3(NT), LDS_BYTES, m->stream, f);
+  launch_forward<false>(f, m->E, m->stream);
   MLP_HIP(hipEventRecord(m->ev[1], m->stream));
   MLP_HIP(hipGetLastError());
   MLP_HIP(hipMemcpyAsync(out, py, (size_t)m->E * n * DOUT * sizeof(float), hipMemcpyDeviceToHost, m->stream));
