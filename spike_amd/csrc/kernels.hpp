@@ -402,6 +402,9 @@ __device__ __forceinline__ float lif_unit(const LifArgs& a, int i, const uint32_
   }
   const int bits = a.W * 32;
   int hpos = a.b0, slot = a.slot0;
+  // groups of one step: the history word beside the other loads, not behind the ring's clear
+  uint32_t* hw = a.hist + (size_t)(hpos >> 5) * a.N + ii;
+  const uint32_t h0 = CH == 1 ? *hw : 0u;
   for (int g0 = 0; g0 < a.G; g0 += CH) {
     const int gn = CH == 1 ? 1 : min(CH, a.G - g0);
     // external per-neuron Poisson drive, joined to label 0 of each step's input: counts of the
@@ -496,7 +499,12 @@ __device__ __forceinline__ float lif_unit(const LifArgs& a, int i, const uint32_
         if (step >= a.st.t0 && step < a.st.t0 + a.st.nsteps) atomicAdd(a.st.hist + (step - a.st.t0) / a.st.bin, 1u);
       }
     }
-    if (active) hist_update(a.hist, a.N, i, bits, hpos, gn, mask);
+    if (CH == 1) {
+      const uint32_t h1 = (h0 & ~(1u << (hpos & 31))) | (mask << (hpos & 31));
+      if (active && h1 != h0) *hw = h1;
+    } else if (active) {
+      hist_update(a.hist, a.N, i, bits, hpos, gn, mask);
+    }
     hpos += gn;
     if (hpos >= bits) hpos -= bits;
     wave_append_steps(mask, g0, gn, (uint32_t)i, i, a.lists, a.counts, a.cap, a.spike_stat, a.mon, a.n_mons, a.t, a.dt);
@@ -865,15 +873,16 @@ __device__ __forceinline__ void wave_push(bool pred, uint32_t id, uint32_t* __re
   if (pred && p < cap) list[p] = id;
 }
 
-// Per-neuron traces of unit u as a presynaptic source (l: its last spike time); lists it
-// (when `push`) if it spiked in the group and has rule synapses.  Wavefront-uniform call.
-__device__ __forceinline__ void wd_pre_unit(const WdEventArgs& a, int u, bool active, float l, bool push) {
-  const int G = a.G;
-  const float* Ep = a.tab + 5 + (G + 1);
+// Per-neuron traces of unit u as a presynaptic source (l: its last spike time, x0: its stored
+// trace, tab: a.tab or a copy); lists it (when `push`) if it spiked in the group and has rule
+// synapses.  Wavefront-uniform call.
+__device__ __forceinline__ void wd_pre_unit(const WdEventArgs& a, const float* tab, int G, int u, bool active, float l,
+                                            float x0, bool push) {
+  const float* Ep = tab + 5 + (G + 1);
   bool listed = false;
   if (active) {
     const int pg = wd_pre_step(l, a.t, a.dt, G);
-    const float x = wd_trace(tload(a.trn, 0, u), pg, a.tab[1], Ep, G, a.nearest);
+    const float x = wd_trace(x0, pg, tab[1], Ep, G, a.nearest);
     a.xa[u] = x;
     tstore(a.trn, 0, u, x);
     listed = pg >= 0 && a.pre_ptr[u + 1] > a.pre_ptr[u];
@@ -881,29 +890,30 @@ __device__ __forceinline__ void wd_pre_unit(const WdEventArgs& a, int u, bool ac
   if (push) wave_push(listed, (uint32_t)u, a.act, a.cnt + 2 * a.par, a.N + a.Nin);
 }
 
-// The same for neuron v as a postsynaptic target (l: its last spike time).
-__device__ __forceinline__ void wd_post_unit(const WdEventArgs& a, int v, bool active, float l) {
-  const int G = a.G;
-  const float* Em = a.tab + 5;
+// The same for neuron v as a postsynaptic target.
+__device__ __forceinline__ void wd_post_unit(const WdEventArgs& a, const float* tab, int G, int v, bool active, float l,
+                                             float x0, bool push) {
+  const float* Em = tab + 5;
   bool listed = false;
   if (active) {
     const int qg = wd_post_step(l, a.t, a.dt, G);
-    const float x = wd_trace(tload(a.trn, 1, v), qg, a.tab[0], Em, G, a.nearest);
+    const float x = wd_trace(x0, qg, tab[0], Em, G, a.nearest);
     a.xb[v] = x;
     tstore(a.trn, 1, v, x);
     listed = qg >= 0 && a.post_ptr[v + 1] > a.post_ptr[v];
   }
-  wave_push(listed, (uint32_t)v, a.act + a.N + a.Nin, a.cnt + 2 * a.par + 1, a.N);
+  if (push) wave_push(listed, (uint32_t)v, a.act + a.N + a.Nin, a.cnt + 2 * a.par + 1, a.N);
 }
 
 static __global__ __launch_bounds__(256) void k_wd_neurons(WdEventArgs a) {
   const int U = a.N + a.Nin;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool pre = i < U;
-  wd_pre_unit(a, i, pre, pre ? (i < a.N ? a.last_n[i] : a.last_in[i - a.N]) : 0.0f, true);
+  wd_pre_unit(a, a.tab, a.G, i, pre, pre ? (i < a.N ? a.last_n[i] : a.last_in[i - a.N]) : 0.0f,
+              pre ? tload(a.trn, 0, i) : 0.0f, true);
   const int v = i - U;
   const bool post = v >= 0 && v < a.N;
-  wd_post_unit(a, v, post, post ? a.last_n[v] : 0.0f);
+  wd_post_unit(a, a.tab, a.G, v, post, post ? a.last_n[v] : 0.0f, post ? tload(a.trn, 1, v) : 0.0f, true);
 }
 
 static __global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
@@ -953,17 +963,21 @@ static __global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
 // One group of the per-phase path in two launches, for networks with Poisson (or no) inputs:
 //   k_units   LIF neurons and Poisson inputs (one lane each), the spike monitors' records, and
 //             for a weight-dependent rule in its spike-driven form (G = 1) the rule's
-//             per-neuron traces and its list of spiking targets; clears the spike counts of
+//             per-neuron traces; clears the spike counts of
 //             the next group's list slot (so no separate group-start launch is needed);
 //   k_deliver propagation of this group's spikes and, with that rule, both its sides:
 //             - source side: each spiking unit's row is walked once; a synapse the rule
 //               lists (bit of `mask`) is updated first and delivered with its new weight
 //               (the reference applies plasticity before propagation, SpikingModel.cpp:228-233);
-//             - target side: the rule synapses onto each listed spiking neuron whose source
-//               did not spike in the group (those the source side does not reach).
+//             - target side: the rule synapses onto each spiking neuron of the same list whose
+//               source did not spike in the group (those the source side does not reach).
 //             The two sides touch disjoint synapses, and propagation reads only the rows of
 //             this group's spikers, so all of it runs in one launch.
-// Other rules run between the two launches.  Results equal those of the separate kernels
+// Other rules run between the two launches.  5e5 neurons with 1000 synapses each, 3.2e8 of them
+// plastic: k_units 12.9 us a step, bound by the latency of a unit's loads and of the list's
+// atomics (14.4 us with the traces, the rule's table and the history word loaded after the
+// neuron's stores and a second list of targets); k_deliver 31 us, bound by random accesses (per
+// synapse a ring atomic, the target's trace and last spike).  Results equal those of the separate kernels
 // (k_begin_group, k_lif, k_poisson, k_wd_neurons, k_wd_events, k_propagate, k_collect) bit for
 // bit.
 
@@ -987,19 +1001,29 @@ __global__ __launch_bounds__(256) void k_units(UnitsArgs a) {
       a.slot_tidx[a.slot] = a.lif.tidx;
     }
   }
+  // a folded rule (groups of one step): its table and the unit's traces are loaded beside the
+  // unit's state
+  float tab[9];
+  if (WD) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) tab[k] = a.wd.tab[k];
+  }
   if ((int)blockIdx.x < a.nb_neurons) {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    const bool on = i < a.lif.N;
+    const float xa = WD && on ? tload(a.wd.trn, 0, i) : 0.0f, xb = WD && on ? tload(a.wd.trn, 1, i) : 0.0f;
     load_ext_table(a.lif, scdf);
     const float last = lif_unit<KIND, CH>(a.lif, i, scdf);
     if (WD) {
-      const bool on = i < a.lif.N;
-      wd_pre_unit(a.wd, i, on, last, false);
-      wd_post_unit(a.wd, i, on, last);
+      wd_pre_unit(a.wd, tab, 1, i, on, last, xa, false);
+      wd_post_unit(a.wd, tab, 1, i, on, last, xb, false);
     }
   } else {
     const int i = (int)((blockIdx.x - a.nb_neurons) * blockDim.x + threadIdx.x);
+    const bool on = i < a.in.Nin;
+    const float xa = WD && on ? tload(a.wd.trn, 0, a.in.N + i) : 0.0f;
     const float last = poisson_unit<CH>(a.in, i);
-    if (WD) wd_pre_unit(a.wd, a.in.N + i, i < a.in.Nin, last, false);
+    if (WD) wd_pre_unit(a.wd, tab, 1, a.in.N + i, on, last, xa, false);
   }
 }
 
@@ -1019,12 +1043,6 @@ __global__ __launch_bounds__(256) void k_deliver(DeliverArgs a) {
   const PropArgs& p = a.p;
   const WdEventArgs& r = a.wd;
   const size_t NL = (size_t)p.N * p.L;
-  int npost = 0;
-  if (WD) {
-    npost = min(r.cnt[2 * r.par + 1], r.N);
-    // the other buffer is next group's: clear it (nothing reads it in this group)
-    if (blockIdx.x == 0 && threadIdx.x < 2) r.cnt[2 * (r.par ^ 1) + threadIdx.x] = 0;
-  }
   unsigned long long ev = 0;
   // source side: tasks (sub-step, spike, wavefront of its row), the sub-steps 64 at a time --
   // lane x holds the tasks up to and including sub-step g0 + x
@@ -1076,11 +1094,14 @@ __global__ __launch_bounds__(256) void k_deliver(DeliverArgs a) {
       }
     }
     if (WD) {
-      // target side (G = 1): the wavefronts after those of the source side
+      // target side (G = 1, the same list's neurons): the wavefronts after those of the source
+      // side
+      const int npost = min(p.counts[0], p.cap);
       for (int w = wave + (wave < tasks ? (tasks - wave + nwaves - 1) / nwaves * nwaves : 0) - tasks;
            w < npost * a.post_waves; w += nwaves) {
         const int k = w / a.post_waves, c = w - k * a.post_waves;
-        const int v = (int)r.act[r.N + r.Nin + k];
+        const int v = (int)p.lists[k];
+        if (v >= r.N) continue;
         const int qg = wd_post_step(r.last_n[v], r.t, r.dt, r.G);
         const float xpost = r.xb[v];
         const int64_t e1 = r.post_ptr[v + 1];

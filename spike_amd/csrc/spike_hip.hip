@@ -1087,7 +1087,6 @@ int launch_group_fast(spk_network* n, float t, bool plastic) {
     d.mask = n->d_wd_mask;
     d.post_waves = (int)std::min<int64_t>(64, std::max<int64_t>(1, (r->max_post + spk::kWave - 1) / spk::kWave));
     hipLaunchKernelGGL(spk::k_deliver<true>, dim3(db), dim3(256), 0, n->stream, d);
-    r->par ^= 1;
     r->syn_tr = false;
   } else {
     d.post_waves = 1;
