@@ -3,8 +3,8 @@
 // One lane per neuron for the neuron phases; for delivery, each spiking unit's row is
 // shared by several 64-lane wavefronts.  State is structure-of-arrays FP32; the input ring
 // is int64 fixed point (exact, order-independent sums); spike lists are compacted with a
-// wavefront ballot + popcount prefix and one atomic per wavefront.  Networks with G = 1 run
-// a group as two launches (k_units, k_deliver) built from the same per-unit functions.
+// wavefront ballot + popcount prefix and one atomic per wavefront.  Groups of any length run
+// as two launches (k_units, k_deliver) built from the same per-unit functions.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -819,15 +819,16 @@ void launch_forward(FwdArgs f, int models, hipStream_t st) {
 
 // Outputs of every member for n rows of features on the device, into `y` and from there to
 // the host (`out`); ev[0], ev[1] around the kernels.  Few rows (at most one 16-row tile per CU)
-// take the kernel made for latency.  Many rows are cut into pieces, and the copy of a piece
-// runs on a second stream while the next one computes.
-int infer(spk_mlp* m, const float* x, int64_t n, float* y, float* out) {
+// take the kernel made for latency.  Many rows are cut into pieces (`pieces`: not for callers
+// that may not allocate, as the first such call makes a stream), and the copy of a piece runs
+// on a second stream while the next one computes.
+int infer(spk_mlp* m, const float* x, int64_t n, float* y, float* out, bool pieces_ok) {
   FwdArgs f{};
   f.wb = m->wb; f.master = m->master; f.x = x; f.n = n; f.M = (int)n; f.mode = 0; f.y = y;
   const size_t row = DOUT * sizeof(float);
   const int64_t small = (n + TS - 1) / TS * m->E, blocks = (n + MT - 1) / MT * m->E;
   MLP_HIP(hipEventRecord(m->ev[0], m->stream));
-  if (small > kSmallTiles && blocks >= 2 * kPieceTiles) {
+  if (pieces_ok && small > kSmallTiles && blocks >= 2 * kPieceTiles) {
     if (!m->copy) MLP_HIP(hipStreamCreateWithFlags(&m->copy, hipStreamNonBlocking));
     f.tiles = (int)((n + MT - 1) / MT);
     const int pieces = (int)std::min<int64_t>(kMaxPieces, blocks / kPieceTiles);
@@ -1196,7 +1197,7 @@ int spk_mlp_predict(spk_mlp* m, const float* features, int64_t n, float* out) {
     m->pcap = n;
   }
   MLP_HIP(hipMemcpyAsync(m->px, features, (size_t)n * DIN * sizeof(float), hipMemcpyHostToDevice, m->stream));
-  if (int rc = infer(m, m->px, n, m->py, out)) return rc;
+  if (int rc = infer(m, m->px, n, m->py, out, true)) return rc;
   const float ms = elapsed(m->ev[0], m->ev[1]);
   m->timing = spk_mlp_timing{ms, ms, 0, 0, 0, 0, n};
   return SPK_OK;
@@ -1214,7 +1215,7 @@ int spk_mlp_predict_noalloc(spk_mlp* m, const float* features, int64_t n, float*
   float* px = m->scratch;
   float* py = m->scratch + xfl;
   MLP_HIP(hipMemcpyAsync(px, features, (size_t)n * DIN * sizeof(float), hipMemcpyHostToDevice, m->stream));
-  if (int rc = infer(m, px, n, py, out)) return rc;
+  if (int rc = infer(m, px, n, py, out, false)) return rc;
   const float ms = elapsed(m->ev[0], m->ev[1]);
   m->timing = spk_mlp_timing{ms, ms, 0, 0, 0, 0, n};
   return SPK_OK;
