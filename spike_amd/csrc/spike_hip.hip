@@ -40,11 +40,33 @@ int fail(int code, const std::string& msg) {
       return fail(SPK_ERR_HIP, std::string(#expr) + " failed: " + hipGetErrorString(e_)); \
   } while (0)
 
+// Device memory of closed generated networks, kept for the next ones: in a process that has used
+// much of the memory before, the driver clears what it hands out again, and 48 networks of 2.4 GB
+// in all took 136 ms longer to generate (38 ms while it hands out clear memory).  At most
+// kIdleSlabBytes per device, the oldest given back first, all of it when an allocation fails; a
+// slab is kept only after the device has been waited for (as hipFree does) and is cleared on the
+// next owner's stream.
+constexpr size_t kIdleSlabBytes = (size_t)4 << 30;
+struct IdleSlab { char* p; size_t bytes; };
+std::mutex g_slab_mu;
+std::map<int, std::vector<IdleSlab>> g_idle_slabs;   // oldest first
+
+void trim_slabs() {
+  std::lock_guard<std::mutex> lock(g_slab_mu);
+  for (auto& d : g_idle_slabs)
+    for (auto& s : d.second) (void)hipFree(s.p);
+  g_idle_slabs.clear();
+}
+
 template <typename T>
 int dalloc(T** p, size_t n) {
   *p = nullptr;
   if (n == 0) n = 1;
   hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+  if (e == hipErrorOutOfMemory) {
+    trim_slabs();
+    e = hipMalloc((void**)p, n * sizeof(T));
+  }
   if (e != hipSuccess) return fail(SPK_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   return SPK_OK;
 }
@@ -55,11 +77,61 @@ void dfree(T*& p) {
   p = nullptr;
 }
 
+// A slab of at least `bytes` for work on `st`: the smallest idle one at most a quarter larger, or
+// a new one.
+int take_slab(size_t& bytes, int& dev, char** p, hipStream_t st) {
+  *p = nullptr;
+  SPK_HIP(hipGetDevice(&dev));
+  {
+    std::lock_guard<std::mutex> lock(g_slab_mu);
+    auto& idle = g_idle_slabs[dev];
+    size_t best = idle.size();
+    for (size_t k = 0; k < idle.size(); ++k)
+      if (idle[k].bytes >= bytes && idle[k].bytes - bytes <= bytes / 4 + (1u << 20) &&
+          (best == idle.size() || idle[k].bytes < idle[best].bytes))
+        best = k;
+    if (best < idle.size()) {
+      *p = idle[best].p;
+      bytes = idle[best].bytes;
+      idle.erase(idle.begin() + (long)best);
+    }
+  }
+  if (!*p) return dalloc(p, bytes);
+  const hipError_t e = hipMemsetAsync(*p, 0, bytes, st);
+  if (e == hipSuccess) return SPK_OK;
+  (void)hipFree(*p);
+  *p = nullptr;
+  return fail(SPK_ERR_HIP, std::string("hipMemsetAsync: ") + hipGetErrorString(e));
+}
+
+void give_slab(char* p, size_t bytes, int dev) {
+  if (!p) return;
+  int cur = -1;
+  std::vector<char*> old;
+  if (bytes <= kIdleSlabBytes && hipGetDevice(&cur) == hipSuccess && cur == dev && hipDeviceSynchronize() == hipSuccess) {
+    std::lock_guard<std::mutex> lock(g_slab_mu);
+    auto& idle = g_idle_slabs[dev];
+    size_t total = bytes;
+    for (auto& s : idle) total += s.bytes;
+    size_t drop = 0;
+    for (; total > kIdleSlabBytes; ++drop) {
+      total -= idle[drop].bytes;
+      old.push_back(idle[drop].p);
+    }
+    idle.erase(idle.begin(), idle.begin() + (long)drop);
+    idle.push_back({p, bytes});
+  } else {
+    old.push_back(p);
+  }
+  for (char* q : old) (void)hipFree(q);
+}
+
 // One allocation cut into arrays (each on a 256-byte boundary): a generated network's device
 // memory.  hipFree takes 28 us and hipMalloc 4 us a call, and such a network has 25 arrays.
 struct Slab {
   char* base = nullptr;
   size_t bytes = 0;
+  int dev = 0;
   struct Want { void** p; size_t bytes; };
   std::vector<Want> wants;
   template <typename T>
@@ -67,10 +139,10 @@ struct Slab {
     *p = nullptr;
     wants.push_back({(void**)p, (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256});
   }
-  int allocate() {
+  int allocate(hipStream_t st) {
     size_t total = 0;
     for (auto& w : wants) total += w.bytes;
-    if (int rc = dalloc(&base, total)) return rc;
+    if (int rc = take_slab(total, dev, &base, st)) return rc;
     bytes = total;
     size_t o = 0;
     for (auto& w : wants) {
@@ -82,7 +154,8 @@ struct Slab {
   }
   bool owns(const void* p) const { return base && (const char*)p >= base && (const char*)p < base + bytes; }
   void release() {
-    dfree(base);
+    give_slab(base, bytes, dev);
+    base = nullptr;
     bytes = 0;
   }
 };
@@ -2917,7 +2990,7 @@ int spk_stats_begin(spk_network* n, int bin_steps, int64_t max_steps) {
     n->st_slab.want(&n->d_st_s1, N);
     n->st_slab.want(&n->d_st_s2, N);
     n->st_slab.want(&n->d_st_out, 1);
-    if (int rc = n->st_slab.allocate()) return rc;
+    if (int rc = n->st_slab.allocate(n->stream)) return rc;
   }
   if (nb > n->st_nbins) {
     dfree(n->d_st_hist);
@@ -3260,7 +3333,7 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   ALLOC(n->d_xlist, (size_t)2 * 2 * P * spk::fused_xstride(n->xcap));   // 64-bit words
   ALLOC(n->d_bar, (size_t)(spk::kBarGroups + 2) * spk::kBarStride); ALLOC(n->d_err, 1);
 #undef ALLOC
-  if ((rc = n->slab.allocate())) return bail(rc);
+  if ((rc = n->slab.allocate(n->stream))) return bail(rc);
   // tiles: about 512 workgroups for the largest LDS form, whole partitions otherwise
   spk::BrunelGenArgs ga{};
   ga.seed = n->seed; ga.N = N; ga.ne = p->n_exc; ga.ni = p->n_inh; ga.ce = p->ce; ga.ci = p->ci; ga.P = P;
@@ -3270,9 +3343,11 @@ int spk_create_brunel(const spk_brunel_params* p, int partitions, spk_network** 
   ga.tq = (n->nown_max + ga.ts - 1) / ga.ts;
   const int tiles = P * ga.tq;
   unsigned int* d_cnt = nullptr;
-  if ((rc = dalloc(&d_cnt, ((size_t)tiles + 1) * NN))) return bail(rc);
+  Slab tables;
+  tables.want(&d_cnt, ((size_t)tiles + 1) * NN);
+  if ((rc = tables.allocate(n->stream))) return bail(rc);
   hipStream_t st = n->stream;
-  auto cleanup = [&]() { dfree(d_cnt); };
+  auto cleanup = [&]() { tables.release(); };
 #define GEN_HIP(expr)                                                                                  \
   do {                                                                                                 \
     hipError_t e_ = (expr);                                                                            \

@@ -28,3 +28,31 @@ def test_generated_equals_replay(n, partitions, eps):
     assert spikes == o["spikes_neurons"] > 0 and events == o["external_events"]
     assert np.array_equal(net.membrane().astype(np.float64), ora.membrane())
     assert np.array_equal(net.ring(), ora.ring())
+
+
+def _run(p):
+    net = sweep.build(p, 0)
+    net.stats_begin(10, 600)
+    net.run(0.0, 20, plasticity=False)
+    v, ring, rate = net.membrane().astype(np.float64), net.ring(), net.stats().rate_hz
+    net.close()
+    return v, ring, rate
+
+
+def test_memory_of_closed_networks():
+    """Networks that take the memory of closed ones: a little smaller, the same size, another
+    in-degree, and from two threads at a time -- each as the oracle's replay."""
+    from concurrent.futures import ThreadPoolExecutor
+    points = [sweep.SweepPoint(n, 5.0, 2.5, 1e-4, 12, seed, eps=eps)
+              for seed, (n, eps) in enumerate([(3000, 0.1), (2900, 0.1), (3000, 0.1), (2950, 0.09), (1500, 0.1)])]
+    want = []
+    for p in points:
+        ora = oracle_py.OracleNetwork(replay_desc(p), precision=32)
+        ora.run(0.0, 20)
+        want.append((ora.membrane(), ora.ring()))
+    one = [_run(p) for p in points]
+    with ThreadPoolExecutor(2) as pool:
+        two = list(pool.map(_run, points * 2))
+    for k, (v, ring, rate) in enumerate(one + two):
+        assert np.array_equal(v, want[k % 5][0]) and np.array_equal(ring, want[k % 5][1]), k
+        assert rate == one[k % 5][2]
