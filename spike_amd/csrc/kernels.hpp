@@ -979,7 +979,8 @@ static __global__ __launch_bounds__(256) void k_wd_events(WdEventArgs a) {
 // neuron's stores and a second list of targets); k_deliver 31 us, bound by random accesses (per
 // synapse a ring atomic, the target's trace and last spike).  Results equal those of the separate kernels
 // (k_begin_group, k_lif, k_poisson, k_wd_neurons, k_wd_events, k_propagate, k_collect) bit for
-// bit.
+// bit.  A rule is folded in only where the units whose spikes count in the group are those of its
+// list (wd_group_resolved on the host); k_wd_neurons lists them by their times instead.
 
 struct UnitsArgs {
   LifArgs lif;

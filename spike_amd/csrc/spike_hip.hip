@@ -367,6 +367,8 @@ struct MonitorHost {
 
 }  // namespace
 
+constexpr float kNoSpike = -1000.0f;   // last spike time of a unit that has not spiked
+
 struct spk_network {
   int N = 0, Nin = 0, kind = 0, L = 1;
   float dt = 1e-4f;
@@ -506,6 +508,7 @@ struct spk_network {
   // (SpikingModel::run continues from the current time), so last-spike times never lie
   // ahead of a group, which the plasticity tables rely on
   float t_hi = -INFINITY;
+  float spike_hi = kNoSpike;     // latest time a spike so far can have (group_end)
   // rate monitors: one spike counter per neuron / input (shared by the monitors of a
   // population; each monitor keeps the counts at its last reset as a baseline)
   uint32_t* d_rate[2] = {nullptr, nullptr};
@@ -816,6 +819,21 @@ int build_wd_mask(spk_network* n) {
   return SPK_OK;
 }
 
+// Time of the last sub-step of the group at t, as the kernels compute it.
+float group_end(const spk_network* n, float t) { return t + (float)(n->G - 1) * n->dt; }
+
+// Whether a launch that walks the group's spikes applies the weight-dependent rule as the
+// per-synapse form does.  That form reads the step of a unit's spike from its last spike time:
+//   - a spike before the group (at most at `before`) must lie more than half a step in front of
+//     it, else it counts in this group, too, and its unit is not among the group's spikes.  Not so
+//     where float32 no longer resolves a step (dt = 0.1 ms: from 1024 s on) and where a group
+//     begins on the last one's time again;
+//   - no unit spikes twice in the group (the refractory test over its whole length).
+bool wd_group_resolved(const spk_network* n, float before, float t) {
+  if (!(roundf((before - t) / n->dt) < 0.0f)) return false;
+  return n->G == 1 || !((group_end(n, t) - t) - n->tref > 0.5f * n->dt);
+}
+
 int check_time(spk_network* n, float t) {
   if (!(t >= n->t_hi - 0.5f * n->dt))
     return fail(SPK_ERR_ARG, "group start time precedes the latest group simulated "
@@ -826,6 +844,7 @@ int check_time(spk_network* n, float t) {
 
 int begin_group(spk_network* n, float t, bool force = false) {
   if (int rc = check_time(n, t)) return rc;
+  n->spike_hi = std::max(n->spike_hi, group_end(n, t));
   const int tidx = (int)roundf(t / n->dt);
   if (tidx == n->cur_tidx && !force) return SPK_OK;
   n->cur_tidx = tidx;
@@ -1073,11 +1092,13 @@ bool fast_group_ok(const spk_network* n) {
   return !n->gen && n->N > 0 && n->S > 0 && n->slots >= 2;
 }
 
-// A weight-dependent rule that k_units and k_deliver apply themselves (in its spike-driven form).
-bool rule_folds(const spk_network* n, bool plastic) {
+// A weight-dependent rule that k_units and k_deliver apply themselves in the group at t (in its
+// spike-driven form).
+bool rule_folds(const spk_network* n, bool plastic, float t) {
   if (!plastic || n->rules.size() != 1 || n->G != 1 || n->Gprep != 1) return false;
   const RuleHost& r = n->rules[0];
-  return r.kind == 0 && r.ev_ok && r.cnt > 0 && !r.dense_next && n->d_wd_mask != nullptr;
+  return r.kind == 0 && r.ev_ok && r.cnt > 0 && !r.dense_next && n->d_wd_mask != nullptr &&
+         wd_group_resolved(n, n->spike_hi, t);
 }
 
 // Workgroups of a delivery launch: two units' rows per workgroup keep the chip full for the
@@ -1101,16 +1122,17 @@ int launch_collect(spk_network* n, int mid, int slot0, int nslots);
 // clears them.
 int launch_group_fast(spk_network* n, float t, bool plastic) {
   const int tidx = (int)roundf(t / n->dt);
+  const bool wd = rule_folds(n, plastic, t);   // (by the spikes before this group)
   if (n->cleared_tidx != tidx) {
     if (int rc = begin_group(n, t, true)) return rc;
   } else {
     if (int rc = check_time(n, t)) return rc;
+    n->spike_hi = std::max(n->spike_hi, group_end(n, t));
     n->cur_tidx = tidx;
     n->cur_slot = (tidx / n->G) % n->slots;
   }
   const int slot = n->cur_slot;
   const int next = (tidx / n->G + 1) % n->slots;
-  const bool wd = rule_folds(n, plastic);
   RuleHost* r = wd ? &n->rules[0] : nullptr;
   spk::UnitsArgs u{};
   if (wd) {
@@ -1491,18 +1513,27 @@ int plan_event_rule(spk_network* n, bool input_sources) {
   return SPK_OK;
 }
 
-// Time step of group `g` of a run from `start`, as the kernels compute it.
+// Start time and time step of group `g` of a run from `start`, as the kernels compute them.
+float group_start(const spk_network* n, float start, int64_t g) { return start + (float)(g * n->G) * n->dt; }
 int64_t group_step(const spk_network* n, float start, int64_t g) {
-  return (int64_t)roundf((start + (float)(g * n->G) * n->dt) / n->dt);
+  return (int64_t)roundf(group_start(n, start, g) / n->dt);
 }
 
-// Whether a run of `ngroups` groups may apply the rule by spikes.  A delayed rule then takes the
-// spikes of one group for the arrivals of the next: all its delays equal the group's length, and
-// the groups' steps follow each other without a gap or an overlap (not so where float32 times
-// no longer resolve the step).
+// Whether a run of `ngroups` groups may apply the rule by spikes: the weight-dependent rule where
+// every group is resolved (wd_group_resolved).  A delayed rule takes the spikes of one group for
+// the arrivals of the next: all its delays equal the group's length, and the groups' steps follow
+// each other without a gap or an overlap (not so where float32 times no longer resolve the step).
 bool event_run_ok(const spk_network* n, float start, int64_t ngroups) {
   if (!n->ev_fused) return false;
-  if (event_mode(n) == spk::kRulesEvents) return true;
+  if (event_mode(n) == spk::kRulesEvents) {
+    float before = n->spike_hi;
+    for (int64_t g = 0; g < ngroups; ++g) {
+      const float t = group_start(n, start, g);
+      if (!wd_group_resolved(n, before, t)) return false;
+      before = std::max(before, group_end(n, t));
+    }
+    return true;
+  }
   if (n->rules[0].delay != n->G) return false;
   for (int64_t g = 1; g < ngroups; ++g)
     if (group_step(n, start, g) != group_step(n, start, g - 1) + n->G) return false;
@@ -1642,6 +1673,7 @@ int stage_fused(spk_network* n, spk::FusedArgs& a, float start, int64_t group0, 
   a.arm_step = n->Nin > 0 ? n->arm_step : -1;
   a.st = stats_args(n, start);
   stats_advance(n, (int64_t)roundf(start / n->dt), group0 + ng);
+  if (ng > 0) n->spike_hi = std::max(n->spike_hi, group_end(n, group_start(n, start, group0 + ng - 1)));
   if (ng > 0 && !n->mons.empty()) {
     note_steps(n, group_step(n, start, group0), 0);
     note_steps(n, group_step(n, start, group0 + ng - 1), n->G);
@@ -2858,6 +2890,7 @@ int spk_reset_state(spk_network* n) {
   }
   n->cur_tidx = n->cleared_tidx = -1;
   n->t_hi = -INFINITY;
+  n->spike_hi = kNoSpike;
   return launch_reset(n, true);
 }
 

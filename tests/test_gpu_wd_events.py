@@ -74,3 +74,46 @@ def test_synapse_kinds(kind, labels):
 def test_networks_that_stay_per_synapse(case):
     d = _net(dmin=3, dmax=6) if case.startswith("inputs") else _net(dmin=8, dmax=9, inputs_in_rule=False, tref=4e-4)
     _pieces(d, 3, False)
+
+
+@pytest.mark.parametrize("form", ["persistent", "launches", "steps"])
+@pytest.mark.parametrize("dmin", [1, 3])
+@pytest.mark.parametrize("start", ["late", "again", "half a step back"])
+def test_spikes_that_count_in_two_groups(start, dmin, form):
+    """Groups whose float32 start is not clear of the group before: beyond 1024 s, where times no
+    longer resolve a step, and runs that begin on the last group's time again or half a step
+    before it.  The rule reads a spike's step from its time, so the earlier group's spikes count
+    in these groups, too, and their units have to be walked although they did not spike.  The
+    persistent kernel keeps its input ring by steps that follow each other and is compared with
+    its own per-synapse form (a second rule, which changes nothing, takes the network there)."""
+    def net():
+        d = _net(dmin=dmin, dmax=dmin + 5, inputs_in_rule=dmin == 1)
+        d.monitors = []   # (records of one time in several groups come in the order of the drains)
+        return d
+
+    d = net()
+    gpu = abi.Network(d, partitions=3)
+    if form == "persistent":
+        e = net()
+        other = np.setdiff1d(np.arange(e.n_synapses), e.rules[0].synapses)[:1]
+        e.rules.append(Rule(RULE_WD, other, builders.wd_params(lam=0.0)))
+        ref = abi.Network(e, partitions=3)
+        assert ref.info().fused == 1
+    else:
+        ref = oracle_py.OracleNetwork(d, precision=32)
+
+    def both(t, ng):
+        ref.run(t, ng)
+        if form == "steps":
+            for s in range(ng):
+                gpu.step_group(d.group_time(t, s))
+        else:
+            gpu.run(t, ng, force_launches=form == "launches")
+
+    both(0.0, 50)
+    last = np.float32(d.group_time(0.0, 49))
+    t = {"late": np.float32(1500.0), "again": last, "half a step back": last - np.float32(0.45) * np.float32(d.dt)}[start]
+    if start == "late" and dmin == 1:
+        assert any(d.group_time(t, s) == d.group_time(t, s + 1) for s in range(60))
+    both(float(t), 60)
+    _compare(gpu, ref, d, f"{start} {form}")
