@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -17,6 +18,7 @@
 #include <vector>
 
 #include "../../include/spike_hip.h"
+#include "alloc.hpp"
 #include "kernels.hpp"
 #include "fused.hpp"
 #include "fused_table.hpp"
@@ -58,15 +60,25 @@ void trim_slabs() {
   g_idle_slabs.clear();
 }
 
+// Requests still to pass and then to refuse (spk_refuse_allocations).
+std::atomic<int> g_pass{0}, g_refuse{0};
+
+hipError_t malloc_once(void** p, size_t bytes) {
+  // a refused request asks for more than any device has, so that the runtime itself fails it
+  if (g_refuse.load(std::memory_order_relaxed) > 0 && g_pass.fetch_sub(1) <= 0 && g_refuse.fetch_sub(1) > 0)
+    bytes = (size_t)1 << 60;
+  const hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  *p = nullptr;
+  (void)hipGetLastError();
+  return e;
+}
+
 template <typename T>
 int dalloc(T** p, size_t n) {
   *p = nullptr;
   if (n == 0) n = 1;
-  hipError_t e = hipMalloc((void**)p, n * sizeof(T));
-  if (e == hipErrorOutOfMemory) {
-    trim_slabs();
-    e = hipMalloc((void**)p, n * sizeof(T));
-  }
+  const hipError_t e = spk::device_malloc((void**)p, n * sizeof(T));
   if (e != hipSuccess) return fail(SPK_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   return SPK_OK;
 }
@@ -1797,9 +1809,21 @@ int run_fused(spk_network* n, float start, int64_t ngroups, int flags) {
 }  // namespace
 
 namespace spk {
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = malloc_once(p, bytes);
+  if (e != hipErrorOutOfMemory) return e;
+  trim_slabs();
+  return malloc_once(p, bytes);
+}
+
 // error message of the calling thread, shared with the surrogate's entry points (mlp.hip)
 void set_last_error(const std::string& msg) { g_error = msg; }
 }  // namespace spk
+
+extern "C" void spk_refuse_allocations(int pass, int count) {
+  g_pass = pass;
+  g_refuse = count;
+}
 
 // =====================================================================================
 extern "C" {

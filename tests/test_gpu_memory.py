@@ -1,0 +1,57 @@
+"""What the library does when device memory runs out: calls that found the memory without the
+idle memory of closed networks still find it, a refused request leaves no error for a later call
+to report, and an object whose buffers could not grow stays usable.  The library refuses requests
+itself (spk_refuse_allocations: `pass` requests are served, then `count` refused; a request that is
+tried again after the idle memory went back counts twice)."""
+import contextlib
+
+import numpy as np
+import pytest
+
+import oracle_py
+from spike_amd import abi, builders, sweep
+from sweep_replay import replay_desc
+
+pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def _refused(count, after=0):
+    lib = abi.load()
+    lib.spk_refuse_allocations(after, count)
+    try:
+        yield
+    finally:
+        lib.spk_refuse_allocations(0, 0)
+
+
+def _generated(n, seed):
+    return sweep.SweepPoint(n, 5.0, 2.5, 1e-4, 12, seed)
+
+
+def _equals_replay(p, net):
+    ora = oracle_py.OracleNetwork(replay_desc(p), precision=32)
+    net.run(0.0, 20, plasticity=False)
+    ora.run(0.0, 20)
+    assert np.array_equal(net.membrane().astype(np.float64), ora.membrane())
+    assert np.array_equal(net.ring(), ora.ring())
+
+
+def test_request_that_succeeds_after_idle_memory_went_back():
+    sweep.build(_generated(3000, 1), 0).close()      # leaves idle memory
+    p = _generated(7001, 2)
+    with _refused(1):
+        net = sweep.build(p, 0)
+    _equals_replay(p, net)
+
+
+def test_refused_request_leaves_no_error_behind():
+    d = builders.random_net(seed=2, input_rate=400.0, whi=4e-3)
+    with _refused(2):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            abi.Network(d)
+    gpu = abi.Network(d)
+    ora = oracle_py.OracleNetwork(d, precision=32)
+    gpu.run(0.0, 20)
+    ora.run(0.0, 20)
+    assert np.array_equal(gpu.membrane().astype(np.float64), ora.membrane())
