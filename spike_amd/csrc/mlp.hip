@@ -39,6 +39,7 @@
 
 #include "../../include/spike_hip.h"
 #include "../../include/spike_mlp.h"
+#include "alloc.hpp"
 #include "philox.hpp"
 
 namespace spk {
@@ -774,7 +775,7 @@ int mfail(int code, const std::string& msg) {
 template <typename T>
 int malloc_d(T** p, size_t n) {
   *p = nullptr;
-  hipError_t e = hipMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T));
+  const hipError_t e = spk::device_malloc((void**)p, std::max<size_t>(n, 1) * sizeof(T));
   if (e != hipSuccess) return mfail(SPK_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   return SPK_OK;
 }

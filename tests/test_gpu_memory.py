@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import oracle_py
-from spike_amd import abi, builders, sweep
+from spike_amd import abi, builders, mlp, sweep
 from sweep_replay import replay_desc
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +55,19 @@ def test_refused_request_leaves_no_error_behind():
     gpu.run(0.0, 20)
     ora.run(0.0, 20)
     assert np.array_equal(gpu.membrane().astype(np.float64), ora.membrane())
+
+
+def test_surrogate_takes_what_idle_memory_gives_back():
+    p = mlp.init_params(5, 2)
+    x = np.random.default_rng(6).uniform(-1.0, 1.0, (300, mlp.INPUTS)).astype(np.float32)
+    ref = mlp.Mlp(2, 256)
+    ref.set_params(p)
+    want = ref.predict(x)
+    with _refused(2):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            mlp.Mlp(2, 256)
+    sweep.build(_generated(3000, 1), 0).close()
+    with _refused(1):
+        net = mlp.Mlp(2, 256)
+    net.set_params(p)
+    assert np.array_equal(net.predict(x), want)
