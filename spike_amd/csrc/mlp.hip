@@ -1025,19 +1025,26 @@ int spk_mlp_reset_optimizer(spk_mlp* m) {
 int spk_mlp_set_params(spk_mlp* m, const float* params) {
   if (!m || !params) return mfail(SPK_ERR_ARG, "null argument");
   // checked on the device before they take the place of the current ones (a pass over the
-  // 1.6e6 parameters of 8 members takes 1 ms on the host)
-  int rc;
+  // 1.6e6 parameters of 8 members takes 1 ms on the host, where they are checked without memory
+  // for a copy)
   const size_t cnt = (size_t)m->E * P;
-  if (!m->gin && (rc = malloc_d(&m->gin, cnt))) return rc;
-  MLP_HIP(hipMemcpyAsync(m->gin, params, cnt * sizeof(float), hipMemcpyHostToDevice, m->stream));
-  MLP_HIP(hipMemsetAsync(m->bad, 0xFF, sizeof(unsigned int), m->stream));
-  hipLaunchKernelGGL(k_mlp_check, dim3(512), dim3(256), 0, m->stream, m->gin, (unsigned int)cnt, m->bad);
-  MLP_HIP(hipGetLastError());
-  unsigned int bad = 0;
-  MLP_HIP(hipMemcpyAsync(&bad, m->bad, sizeof(bad), hipMemcpyDeviceToHost, m->stream));
-  MLP_HIP(hipStreamSynchronize(m->stream));
+  size_t bad = cnt;
+  if (m->gin || malloc_d(&m->gin, cnt) == SPK_OK) {
+    MLP_HIP(hipMemcpyAsync(m->gin, params, cnt * sizeof(float), hipMemcpyHostToDevice, m->stream));
+    MLP_HIP(hipMemsetAsync(m->bad, 0xFF, sizeof(unsigned int), m->stream));
+    hipLaunchKernelGGL(k_mlp_check, dim3(512), dim3(256), 0, m->stream, m->gin, (unsigned int)cnt, m->bad);
+    MLP_HIP(hipGetLastError());
+    unsigned int first = 0;
+    MLP_HIP(hipMemcpyAsync(&first, m->bad, sizeof(first), hipMemcpyDeviceToHost, m->stream));
+    MLP_HIP(hipStreamSynchronize(m->stream));
+    bad = std::min<size_t>(first, cnt);
+  } else {
+    for (size_t i = cnt; i-- > 0;)
+      if (!std::isfinite(params[i])) bad = i;
+  }
   if (bad < cnt) return mfail(SPK_ERR_ARG, "non-finite parameter at " + std::to_string(bad));
-  MLP_HIP(hipMemcpyAsync(m->master, m->gin, cnt * sizeof(float), hipMemcpyDeviceToDevice, m->stream));
+  if (m->gin) MLP_HIP(hipMemcpyAsync(m->master, m->gin, cnt * sizeof(float), hipMemcpyDeviceToDevice, m->stream));
+  else MLP_HIP(hipMemcpyAsync(m->master, params, cnt * sizeof(float), hipMemcpyHostToDevice, m->stream));
   // padding entries of the working copies stay zero from creation; every used entry is rewritten
   AdamArgs ad{};
   ad.master = m->master; ad.wb = m->wb; ad.apply = 2;

@@ -71,3 +71,20 @@ def test_surrogate_takes_what_idle_memory_gives_back():
         net = mlp.Mlp(2, 256)
     net.set_params(p)
     assert np.array_equal(net.predict(x), want)
+
+
+def test_parameters_without_memory_for_a_copy():
+    p = mlp.init_params(7, 3)
+    bad = p.copy()
+    bad[1, 17] = np.nan
+    bad[2, 5] = np.inf
+    x = np.random.default_rng(8).uniform(-1.0, 1.0, (40, mlp.INPUTS)).astype(np.float32)
+    net = mlp.Mlp(3, 128)
+    with _refused(100):
+        net.set_params(p)
+        with pytest.raises(abi.SpikeError, match=f"non-finite parameter at {mlp.PARAMS + 17}$"):
+            net.set_params(bad)
+    y = net.predict(x)
+    assert np.array_equal(net.params(), p)
+    net.set_params(p)
+    assert np.array_equal(net.predict(x), y)
