@@ -1069,8 +1069,12 @@ int spk_mlp_set_data(spk_mlp* m, const float* features, const float* targets, in
     MLP_HIP(hipStreamSynchronize(m->stream));
     free_d(m->x);
     free_d(m->t);
+    m->cap = m->n = 0;   // no training set while there is no memory for one
     int rc;
-    if ((rc = malloc_d(&m->x, (size_t)n * DIN)) || (rc = malloc_d(&m->t, (size_t)n * DOUT))) return rc;
+    if ((rc = malloc_d(&m->x, (size_t)n * DIN)) || (rc = malloc_d(&m->t, (size_t)n * DOUT))) {
+      free_d(m->x);
+      return rc;
+    }
     m->cap = n;
   }
   MLP_HIP(hipMemcpyAsync(m->x, features, (size_t)n * DIN * sizeof(float), hipMemcpyHostToDevice, m->stream));
@@ -1200,8 +1204,12 @@ int spk_mlp_predict(spk_mlp* m, const float* features, int64_t n, float* out) {
     MLP_HIP(hipStreamSynchronize(m->stream));
     free_d(m->px);
     free_d(m->py);
+    m->pcap = 0;
     int rc;
-    if ((rc = malloc_d(&m->px, (size_t)n * DIN)) || (rc = malloc_d(&m->py, (size_t)m->E * n * DOUT))) return rc;
+    if ((rc = malloc_d(&m->px, (size_t)n * DIN)) || (rc = malloc_d(&m->py, (size_t)m->E * n * DOUT))) {
+      free_d(m->px);
+      return rc;
+    }
     m->pcap = n;
   }
   MLP_HIP(hipMemcpyAsync(m->px, features, (size_t)n * DIN * sizeof(float), hipMemcpyHostToDevice, m->stream));

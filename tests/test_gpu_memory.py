@@ -88,3 +88,29 @@ def test_parameters_without_memory_for_a_copy():
     assert np.array_equal(net.params(), p)
     net.set_params(p)
     assert np.array_equal(net.predict(x), y)
+
+
+@pytest.mark.parametrize("served", [0, 1])
+def test_surrogate_buffers_that_could_not_grow(served):
+    """Rows and results of a prediction, and a training set, after a larger one was refused: the
+    sizes that were there before are not taken for memory that is."""
+    rng = np.random.default_rng(9)
+    x = rng.uniform(-1.0, 1.0, (5000, mlp.INPUTS)).astype(np.float32)
+    t = rng.standard_normal((5000, mlp.OUTPUTS)).astype(np.float32)
+    net = mlp.Mlp(2, 128)
+    net.set_params(mlp.init_params(9, 2))
+    y = net.predict(x[:300])
+    net.set_data(x[:256], t[:256])
+    loss, grads = net.gradients(128)
+    with _refused(2, served):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            net.predict(x)
+    with _refused(2, served):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            net.set_data(x, t)
+    assert np.array_equal(net.predict(x[:300]), y)
+    with pytest.raises(abi.SpikeError, match="training set"):
+        net.gradients(128)
+    net.set_data(x[:256], t[:256])
+    loss1, grads1 = net.gradients(128)
+    assert np.array_equal(loss1, loss) and np.array_equal(grads1, grads)
