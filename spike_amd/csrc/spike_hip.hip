@@ -152,16 +152,17 @@ struct Slab {
     wants.push_back({(void**)p, (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256});
   }
   int allocate(hipStream_t st) {
+    std::vector<Want> list;   // (a refused list is not asked for again beside the caller's next one)
+    list.swap(wants);
     size_t total = 0;
-    for (auto& w : wants) total += w.bytes;
+    for (auto& w : list) total += w.bytes;
     if (int rc = take_slab(total, dev, &base, st)) return rc;
     bytes = total;
     size_t o = 0;
-    for (auto& w : wants) {
+    for (auto& w : list) {
       *w.p = base + o;
       o += w.bytes;
     }
-    wants.clear();
     return SPK_OK;
   }
   bool owns(const void* p) const { return base && (const char*)p >= base && (const char*)p < base + bytes; }

@@ -7,6 +7,7 @@ import contextlib
 
 import numpy as np
 import pytest
+import torch
 
 import oracle_py
 from spike_amd import abi, builders, mlp, sweep
@@ -114,3 +115,16 @@ def test_surrogate_buffers_that_could_not_grow(served):
     net.set_data(x[:256], t[:256])
     loss1, grads1 = net.gradients(128)
     assert np.array_equal(loss1, loss) and np.array_equal(grads1, grads)
+
+
+def test_refused_statistics_are_not_asked_for_twice():
+    n = 400_000                                  # 28 bytes a neuron: 11 MB
+    gpu = abi.Network(builders.large_plastic(n=n, out_degree=2, input_out_degree=2, generated=True))
+    with _refused(100):                          # (idle memory of this size may serve it)
+        with contextlib.suppress(abi.SpikeError):
+            gpu.stats_begin(1, 10)
+    free = torch.cuda.mem_get_info()[0]
+    gpu.stats_begin(1, 10)
+    assert free - torch.cuda.mem_get_info()[0] <= 28 * n + (6 << 20)
+    gpu.run(0.0, 10)
+    assert gpu.stats().steps == 10
