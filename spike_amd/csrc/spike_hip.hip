@@ -3052,6 +3052,8 @@ int spk_stats_begin(spk_network* n, int bin_steps, int64_t max_steps) {
   }
   if (nb > n->st_nbins) {
     dfree(n->d_st_hist);
+    n->st_nbins = 0;
+    n->st_on = false;   // no window while there is no memory for its histogram
     if (int rc = dalloc(&n->d_st_hist, (size_t)nb)) return rc;
     n->st_nbins = nb;
   }
@@ -3073,7 +3075,7 @@ int spk_stats_begin(spk_network* n, int bin_steps, int64_t max_steps) {
 int spk_stats_get(spk_network* n, spk_stats* out) {
   if (int rc = check_prepared(n)) return rc;
   if (!out) return fail(SPK_ERR_ARG, "null output");
-  if (!n->d_st_cnt) return fail(SPK_ERR_STATE, "statistics were never started");
+  if (!n->d_st_cnt || !n->d_st_hist) return fail(SPK_ERR_STATE, "statistics were never started");
   spk::StatsArgs st{};
   st.count = n->d_st_cnt; st.nisi = n->d_st_nisi; st.prev = n->d_st_prev;
   st.s1 = n->d_st_s1; st.s2 = n->d_st_s2; st.hist = n->d_st_hist;

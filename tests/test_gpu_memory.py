@@ -128,3 +128,26 @@ def test_refused_statistics_are_not_asked_for_twice():
     assert free - torch.cuda.mem_get_info()[0] <= 28 * n + (6 << 20)
     gpu.run(0.0, 10)
     assert gpu.stats().steps == 10
+
+
+def test_statistics_window_that_could_not_grow():
+    d = builders.random_net(seed=2, input_rate=400.0, whi=4e-3, dmin=2, dmax=6)
+    gpu, ref = abi.Network(d), abi.Network(d)
+    gpu.stats_begin(10, 200)
+    gpu.run(0.0, 50)
+    assert gpu.stats().spikes > 0
+    with _refused(2):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            gpu.stats_begin(1, 100_000)
+    with pytest.raises(abi.SpikeError, match="never started"):
+        gpu.stats()
+    t = float(d.group_time(0.0, 50))
+    gpu.run(t, 50)                               # no window
+    ref.run(0.0, 50)
+    ref.run(t, 50)
+    t = float(d.group_time(0.0, 100))
+    for net in (gpu, ref):
+        net.stats_begin(10, 200)
+        net.run(t, 60)
+    a, b = gpu.stats(), ref.stats()
+    assert (a.spikes, a.isi_cv, a.synchrony, a.steps) == (b.spikes, b.isi_cv, b.synchrony, b.steps)
