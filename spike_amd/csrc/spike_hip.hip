@@ -1407,25 +1407,33 @@ int drain_monitor(spk_network* n, MonitorHost& m, std::vector<int32_t>& ids,
   return SPK_OK;
 }
 
-int ensure_monitor_capacity(spk_network* n, MonitorHost& m, int64_t need) {
+// A monitor's store of `cap` records, or none.
+int alloc_store(MonitorHost& m, int64_t cap) {
+  m.capacity = 0;
+  if (int rc = dalloc(&m.d_ids, (size_t)cap)) return rc;
+  if (int rc = dalloc(&m.d_times, (size_t)cap)) {
+    dfree(m.d_ids);
+    return rc;
+  }
+  m.capacity = cap;
+  return SPK_OK;
+}
+
+// Room for `need` records; where there is no memory for them, for `least`.
+int ensure_monitor_capacity(spk_network* n, MonitorHost& m, int64_t need, int64_t least) {
   if (m.capacity >= need && m.d_ids) return SPK_OK;
   // keep what is on the device
-  std::vector<int32_t> ids;
-  std::vector<float> times;
   if (m.d_ids) {
-    int rc = drain_monitor(n, m, m.h_ids, m.h_times);
-    if (rc) return rc;
+    if (int rc = drain_monitor(n, m, m.h_ids, m.h_times)) return rc;
   }
+  const int64_t had = m.capacity;
   dfree(m.d_ids);
   dfree(m.d_times);
-  m.capacity = need;
-  int rc = dalloc(&m.d_ids, (size_t)need);
-  if (rc) return rc;
-  rc = dalloc(&m.d_times, (size_t)need);
+  int rc = alloc_store(m, need);
+  if (rc && least < need) rc = alloc_store(m, std::max(least, had));
   if (rc) return rc;
   if (!m.d_count) {
-    rc = dalloc(&m.d_count, 1);
-    if (rc) return rc;
+    if ((rc = dalloc(&m.d_count, 1))) return rc;
   }
   SPK_HIP(hipMemsetAsync(m.d_count, 0, sizeof(unsigned long long), n->stream));
   return SPK_OK;
@@ -1747,13 +1755,14 @@ int run_fused(spk_network* n, float start, int64_t ngroups, int flags) {
   const int G = n->G;
   int64_t chunk = 1000;  // bounds the length of one launch
   // every monitor store holds the records of a whole launch (each unit spikes at most once
-  // per sub-step); larger stores allow longer launches
+  // per sub-step); larger stores allow longer launches (1000 neurons, groups of one step: one
+  // launch of 1000 groups instead of four), where there is memory for them
   for (auto& m : n->mons) {
     const int64_t pop = std::max<int64_t>(1, m.pop == SPK_POP_NEURONS ? n->N : n->Nin);
     const int64_t per_group = pop * G;
-    const int64_t want = std::max<int64_t>(m.capacity, std::max(std::min<int64_t>(per_group * 256, (int64_t)1 << 27),
-                                                                std::min<int64_t>(per_group * chunk, (int64_t)1 << 24)));
-    if (int rc = ensure_monitor_capacity(n, m, std::max<int64_t>(want, per_group))) return rc;
+    const int64_t least = std::max(per_group, std::max<int64_t>(m.capacity, std::min<int64_t>(per_group * 256, (int64_t)1 << 27)));
+    const int64_t want = std::max(least, std::min<int64_t>(per_group * chunk, (int64_t)1 << 24));
+    if (int rc = ensure_monitor_capacity(n, m, want, least)) return rc;
     chunk = std::max<int64_t>(1, std::min<int64_t>(chunk, m.capacity / per_group));
   }
   spk::FusedArgs a;
@@ -2967,7 +2976,7 @@ int spk_run(spk_network* n, float start, int64_t ngroups, int flags) {
     // each monitor store must hold 64 groups of its population
     for (auto& m : n->mons) {
       const int64_t pop = m.pop == SPK_POP_NEURONS ? n->N : n->Nin;
-      if (int rc = ensure_monitor_capacity(n, m, std::max<int64_t>(m.capacity, pop * n->G * 64))) return rc;
+      if (int rc = ensure_monitor_capacity(n, m, pop * n->G * 64, pop * n->G * 64)) return rc;
     }
     const bool plastic = (flags & SPK_RUN_PLASTICITY) != 0;
     int since_drain = 0;

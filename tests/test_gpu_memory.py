@@ -151,3 +151,24 @@ def test_statistics_window_that_could_not_grow():
         net.run(t, 60)
     a, b = gpu.stats(), ref.stats()
     assert (a.spikes, a.isi_cv, a.synchrony, a.steps) == (b.spikes, b.isi_cv, b.synchrony, b.steps)
+
+
+def _monitored():
+    d = builders.random_net(n_neurons=700, n_inputs=900, p=0.02, seed=11, input_rate=300.0, whi=4e-3, monitors=(0, 1))
+    return d, abi.Network(d), oracle_py.OracleNetwork(d, precision=32)
+
+
+def _same_rasters(gpu, ora):
+    for m in (0, 1):
+        for a, b in zip(gpu.take_spikes(m), ora.take_spikes(m)):
+            assert len(a) > 0 and np.array_equal(a, b)
+
+
+def test_monitor_stores_smaller_than_a_whole_run():
+    d, gpu, ora = _monitored()
+    assert d.timestep_grouping() == 1
+    with _refused(2):                            # the store of the first monitor for 1000 groups
+        tm = gpu.run(0.0, 600)
+    assert tm.kernel_launches == 3               # 256 groups at a time
+    ora.run(0.0, 600)
+    _same_rasters(gpu, ora)
