@@ -1419,7 +1419,8 @@ int alloc_store(MonitorHost& m, int64_t cap) {
   return SPK_OK;
 }
 
-// Room for `need` records; where there is no memory for them, for `least`.
+// Room for `need` records; where there is no memory for them, for `least`.  A store that cannot
+// grow to that keeps its size.
 int ensure_monitor_capacity(spk_network* n, MonitorHost& m, int64_t need, int64_t least) {
   if (m.capacity >= need && m.d_ids) return SPK_OK;
   // keep what is on the device
@@ -1431,7 +1432,10 @@ int ensure_monitor_capacity(spk_network* n, MonitorHost& m, int64_t need, int64_
   dfree(m.d_times);
   int rc = alloc_store(m, need);
   if (rc && least < need) rc = alloc_store(m, std::max(least, had));
-  if (rc) return rc;
+  if (rc) {
+    if (had > 0) (void)alloc_store(m, had);
+    return rc;
+  }
   if (!m.d_count) {
     if ((rc = dalloc(&m.d_count, 1))) return rc;
   }

@@ -172,3 +172,30 @@ def test_monitor_stores_smaller_than_a_whole_run():
     assert tm.kernel_launches == 3               # 256 groups at a time
     ora.run(0.0, 600)
     _same_rasters(gpu, ora)
+
+
+@pytest.mark.parametrize("refused", [4, 100])
+def test_monitor_store_that_could_not_grow(refused):
+    """The store of before stays (or, where even that is not to be had, none), and the records of
+    the next groups go nowhere else."""
+    d, gpu, ora = _monitored()
+    with _refused(refused):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            gpu.run(0.0, 600)
+    gpu.reset_state()
+    for s in range(40):
+        gpu.step_group(d.group_time(0.0, s))
+    ora.run(0.0, 40)
+    if refused == 4:
+        _same_rasters(gpu, ora)
+    else:
+        with pytest.raises(abi.SpikeError, match="error 5"):
+            gpu.take_spikes(0)
+        gpu.lib.spk_monitor_reset(gpu.h, gpu.monitor_ids[0])
+        ora.take_spikes(0)
+        ora.take_spikes(1)
+    gpu.take_spikes(1)
+    t = float(d.group_time(0.0, 40))
+    gpu.run(t, 100)
+    ora.run(t, 100)
+    _same_rasters(gpu, ora)
