@@ -1284,29 +1284,35 @@ int order_on_device(spk_network* n, const MonitorHost& m, int64_t cnt, std::vect
   const int64_t wpr = ((m.pop == SPK_POP_NEURONS ? n->N : n->Nin) + 31) / 32;
   const int64_t words = nrows * wpr;
   if (words > kRasterMaxWords) return SPK_OK;
-  int rc;
-  if (!n->d_ras_flag && (rc = dalloc(&n->d_ras_flag, 2))) return rc;
+  // without memory for the buffers the records are ordered on the host
+  if (!n->d_ras_flag && dalloc(&n->d_ras_flag, 2)) return SPK_OK;
   const int64_t tiles = (words + spk::kRasterTile - 1) / spk::kRasterTile;
   if (words > n->ras_words) {
     const int64_t cap = std::min(kRasterMaxWords, words + words / 2);
     dfree(n->d_ras_bits); dfree(n->d_ras_tile);
     n->ras_words = 0;
-    if ((rc = dalloc(&n->d_ras_bits, (size_t)cap))) return rc;
-    if ((rc = dalloc(&n->d_ras_tile, (size_t)(cap + spk::kRasterTile - 1) / spk::kRasterTile))) return rc;
+    if (dalloc(&n->d_ras_bits, (size_t)cap)) return SPK_OK;
+    if (dalloc(&n->d_ras_tile, (size_t)(cap + spk::kRasterTile - 1) / spk::kRasterTile)) {
+      dfree(n->d_ras_bits);
+      return SPK_OK;
+    }
     n->ras_words = cap;
     SPK_HIP(hipMemsetAsync(n->d_ras_bits, 0, sizeof(uint32_t) * cap, n->stream));   // k_raster_emit keeps it zero
   }
   if (nrows > n->ras_rows) {
     dfree(n->d_ras_time);
     n->ras_rows = 0;
-    if ((rc = dalloc(&n->d_ras_time, (size_t)(nrows + nrows / 2)))) return rc;
+    if (dalloc(&n->d_ras_time, (size_t)(nrows + nrows / 2))) return SPK_OK;
     n->ras_rows = nrows + nrows / 2;
   }
   if (cnt > n->ras_n) {
     dfree(n->d_ras_ids); dfree(n->d_ras_times);
     n->ras_n = 0;
-    if ((rc = dalloc(&n->d_ras_ids, (size_t)(cnt + cnt / 2)))) return rc;
-    if ((rc = dalloc(&n->d_ras_times, (size_t)(cnt + cnt / 2)))) return rc;
+    if (dalloc(&n->d_ras_ids, (size_t)(cnt + cnt / 2))) return SPK_OK;
+    if (dalloc(&n->d_ras_times, (size_t)(cnt + cnt / 2))) {
+      dfree(n->d_ras_ids);
+      return SPK_OK;
+    }
     n->ras_n = cnt + cnt / 2;
   }
   spk::RasterArgs a{};

@@ -199,3 +199,19 @@ def test_monitor_store_that_could_not_grow(refused):
     gpu.run(t, 100)
     ora.run(t, 100)
     _same_rasters(gpu, ora)
+
+
+@pytest.mark.parametrize("served", [0, 1, 2, 3, 4, 5, 6])
+def test_raster_without_memory_to_order_it_on_the_device(served):
+    d, gpu, ora = _monitored()
+
+    def steps(t):
+        for s in range(150):
+            gpu.step_group(d.group_time(t, s))
+        ora.run(t, 150)
+
+    steps(0.0)
+    with _refused(100, served):
+        _same_rasters(gpu, ora)
+    steps(float(d.group_time(0.0, 150)))
+    _same_rasters(gpu, ora)
