@@ -456,12 +456,14 @@ struct spk_network {
   uint32_t* d_wc = nullptr;   // per synapse: 16-bit weight | compensation << 16
   float cw_lo = 0.0f, cw_hi = 0.0f;
   int csplit = 0, cnhi = 0, cdelay = 0;
-  // CSR position of each caller synapse (none for generated synapses: the same order);
-  // 64-bit from 2^32 synapses on
-  uint32_t* d_pos = nullptr;
-  int64_t* d_pos64 = nullptr;
-  float* d_wstage = nullptr;  // caller weights on their way in or out, wstage_n at a time
+  // buffers of spk_get_weights / spk_set_weights, made by the first of them: caller weights on
+  // their way in or out, wstage_n at a time; the CSR position of each caller synapse (none for
+  // generated synapses: the same order; 64-bit from 2^32 synapses on) or, where there is no memory
+  // for all of them, of the piece's synapses
+  float* d_wstage = nullptr;
   int64_t wstage_n = 0;
+  uint32_t* d_pos = nullptr;
+  int64_t *d_pos64 = nullptr, *d_piece_pos = nullptr;
   float* d_scale = nullptr;
   uint16_t* d_delay = nullptr;
   uint8_t* d_label = nullptr;
@@ -614,7 +616,7 @@ void free_device(spk_network* n) {
     dfree(m.d_ids); dfree(m.d_times); dfree(m.d_count);
   }
   dfree(n->d_ras_bits); dfree(n->d_ras_time); dfree(n->d_ras_tile); dfree(n->d_ras_ids); dfree(n->d_ras_times);
-  dfree(n->d_ras_flag); dfree(n->d_pos); dfree(n->d_pos64); dfree(n->d_wstage);
+  dfree(n->d_ras_flag); dfree(n->d_pos); dfree(n->d_pos64); dfree(n->d_piece_pos); dfree(n->d_wstage);
   n->slab.release();
   n->st_slab.release();
 }
@@ -1238,14 +1240,41 @@ int launch_group_phases(spk_network* n, float t, bool plastic) {
   return SPK_OK;
 }
 
-// Staging buffer of spk_get_weights / spk_set_weights (64 MB at most).
-constexpr int64_t kWeightPiece = (int64_t)1 << 24;
+// The buffers of spk_get_weights / spk_set_weights: 64 MB at most beside the positions (4 bytes
+// a synapse; uploaded once, as reading them again in every call would cost as much as the
+// weights).  Where memory is short the pieces get smaller, down to 16 KB, and the positions
+// travel with them.
+constexpr int64_t kWeightPiece = (int64_t)1 << 24, kWeightPieceMin = 4096;
 int weight_staging(spk_network* n) {
   if (n->d_wstage) return SPK_OK;
-  const int64_t cnt = std::min<int64_t>(n->S, kWeightPiece);
-  if (int rc = dalloc(&n->d_wstage, (size_t)cnt)) return rc;
-  n->wstage_n = cnt;
-  return SPK_OK;
+  int rc = SPK_OK;
+  if (!n->od && !n->d_pos && !n->d_pos64) {
+    const int64_t S = n->S;
+    if (S >= ((int64_t)1 << 32)) {
+      if (dalloc(&n->d_pos64, (size_t)S) == SPK_OK && (rc = upload(n->d_pos64, n->perm.data(), (size_t)S, n->stream))) {
+        dfree(n->d_pos64);
+        return rc;
+      }
+    } else if (dalloc(&n->d_pos, (size_t)S) == SPK_OK) {
+      hvec<uint32_t> pos(S);
+      host_chunks(S, host_threads(), [&](int, int64_t a, int64_t b) {
+        for (int64_t k = a; k < b; ++k) pos[k] = (uint32_t)n->perm[k];
+      });
+      rc = upload(n->d_pos, pos.data(), (size_t)S, n->stream);
+      const hipError_t e = hipStreamSynchronize(n->stream);   // (the host array ends here)
+      if (rc || e != hipSuccess) {
+        dfree(n->d_pos);
+        return rc ? rc : fail(SPK_ERR_HIP, std::string("uploading synapse positions: ") + hipGetErrorString(e));
+      }
+    }
+  }
+  const bool piece_pos = !n->od && !n->d_pos && !n->d_pos64;
+  for (int64_t cnt = std::min<int64_t>(n->S, kWeightPiece);; cnt = (cnt + 3) / 4) {
+    rc = dalloc(&n->d_wstage, (size_t)cnt);
+    if (!rc && piece_pos && (rc = dalloc(&n->d_piece_pos, (size_t)cnt))) dfree(n->d_wstage);
+    n->wstage_n = cnt;
+    if (!rc || cnt <= kWeightPieceMin) return rc;
+  }
 }
 
 // Caller synapses [s0, s0 + cnt) from the CSR into the staging buffer (`out`) or back.
@@ -1256,7 +1285,9 @@ int launch_weights(spk_network* n, int64_t s0, int64_t cnt, bool out) {
     if (w.wc) w.wc += s0;
   }
   const uint32_t* p32 = n->d_pos ? n->d_pos + s0 : nullptr;
-  const int64_t* p64 = n->d_pos64 ? n->d_pos64 + s0 : nullptr;
+  const int64_t* p64 = n->d_pos64 ? n->d_pos64 + s0 : n->d_piece_pos;
+  if (n->d_piece_pos)
+    SPK_HIP(hipMemcpyAsync(n->d_piece_pos, n->perm.data() + s0, cnt * sizeof(int64_t), hipMemcpyHostToDevice, n->stream));
   const dim3 grid((int)std::min<int64_t>(4096, (cnt + 255) / 256)), block(256);
   if (out && p64) hipLaunchKernelGGL(spk::k_weights_out<int64_t>, grid, block, 0, n->stream, w, p64, cnt, n->d_wstage);
   else if (out) hipLaunchKernelGGL(spk::k_weights_out<uint32_t>, grid, block, 0, n->stream, w, p32, cnt, n->d_wstage);
@@ -2685,17 +2716,6 @@ int spk_prepare(spk_network* n, int G) {
       }
     });
     if ((rc = upload(n->d_syn, rec.data(), S, st))) return rc;
-  }
-  if (S >= ((int64_t)1 << 32)) {
-    if ((rc = dalloc(&n->d_pos64, S))) return rc;
-    if ((rc = upload(n->d_pos64, n->perm.data(), S, st))) return rc;
-  } else {
-    hvec<uint32_t> pos(S);
-    host_chunks(S, T, [&](int, int64_t a, int64_t b) {
-      for (int64_t k = a; k < b; ++k) pos[k] = (uint32_t)n->perm[k];
-    });
-    if ((rc = dalloc(&n->d_pos, S))) return rc;
-    if ((rc = upload(n->d_pos, pos.data(), S, st))) return rc;
   }
   if (n->wfmt != SPK_WEIGHTS_FP32) {
     // 16-bit weights of the records' weights, compensations zero

@@ -215,3 +215,54 @@ def test_raster_without_memory_to_order_it_on_the_device(served):
         _same_rasters(gpu, ora)
     steps(float(d.group_time(0.0, 150)))
     _same_rasters(gpu, ora)
+
+
+def _weights_name_synapses(gpu, S, fmt):
+    """Weights that name their synapse (in two passes of 256 values, exact in every format), set
+    and read, whole and every piece's first and last."""
+    k = np.arange(S)
+    for part in (k % 256, k // 256 % 256, k // 65536):
+        w = part.astype(np.float32)
+        gpu.set_weights(w)
+        assert np.array_equal(gpu.weights(), w), fmt
+
+
+# (requests refused, after how many served): positions for all synapses first, then the piece,
+# each tried twice; a refused piece is tried at a quarter of its size
+@pytest.mark.parametrize("refused,served", [(0, 0), (2, 0), (4, 0), (4, 1), (6, 0), (6, 1), (2, 2)])
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+def test_weights_in_pieces(fmt, refused, served):
+    """Weights of a listed network (synapses in shuffled order) with pieces of S, S / 4 and S / 16
+    synapses (rounded up: the last one ragged), positions kept or travelling with the piece."""
+    d = builders.random_net(n_neurons=331, n_inputs=77, p=0.53, seed=3, whi=1.0, monitors=())
+    o = np.random.default_rng(5).permutation(d.n_synapses)
+    d.pre, d.post, d.weight, d.delay = d.pre[o], d.post[o], d.weight[o], d.delay[o]
+    d.weight_format = fmt
+    d.grouping = 1
+    assert d.n_synapses > 16 * 4096
+    gpu = abi.Network(d)
+    with _refused(refused, served):
+        w = gpu.weights()
+    assert np.array_equal(w, d.weight) if fmt == 0 else np.abs(w - d.weight).max() <= 0.004
+    _weights_name_synapses(gpu, d.n_synapses, fmt)
+
+
+@pytest.mark.parametrize("refused", [0, 2, 4])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_weights_of_generated_synapses_in_pieces(fmt, refused):
+    d = builders.large_plastic(n=3000, out_degree=30, input_out_degree=31, generated=True)
+    d.weight_format = fmt
+    gpu, ref = abi.Network(d), abi.Network(d)
+    with _refused(refused):
+        w = gpu.weights()
+    assert np.array_equal(w, ref.weights())
+    _weights_name_synapses(gpu, d.n_synapses, fmt)
+
+
+def test_weights_without_memory_for_any_piece():
+    d = builders.random_net(seed=2)
+    gpu = abi.Network(d)
+    with _refused(1000):
+        with pytest.raises(abi.SpikeError, match="error 4"):
+            gpu.weights()
+    assert np.array_equal(gpu.weights(), d.weight)
