@@ -2811,18 +2811,12 @@ int spk_prepare(spk_network* n, int G) {
       while (r.src_lo < r.src_hi && pp[r.src_lo + 1] == pp[r.src_lo]) ++r.src_lo;
       r.max_post = 0;
       for (size_t v = 0; v + 1 < qp.size(); ++v) r.max_post = std::max(r.max_post, qp[v + 1] - qp[v]);
-      if ((rc = dalloc(&r.d_ev_pre_ptr, (size_t)U + 1))) return rc;
       if ((rc = dalloc(&r.d_ev_post_ptr, (size_t)n->N + 1))) return rc;
       if ((rc = dalloc(&r.d_ev_post_pos, P))) return rc;
       if ((rc = dalloc(&r.d_ev_post_pre, P))) return rc;
-      if ((rc = upload(r.d_ev_pre_ptr, pp.data(), pp.size(), st))) return rc;
       if ((rc = upload(r.d_ev_post_ptr, qp.data(), qp.size(), st))) return rc;
       if ((rc = upload(r.d_ev_post_pos, qs.data(), P, st))) return rc;
       if ((rc = upload(r.d_ev_post_pre, qu.data(), P, st))) return rc;
-      if (!grouped) {
-        if ((rc = dalloc(&r.d_ev_pre_idx, P))) return rc;
-        if ((rc = upload(r.d_ev_pre_idx, pi.data(), P, st))) return rc;
-      }
       if (n->wfmt != SPK_WEIGHTS_FP32) {
         if ((rc = dalloc(&r.d_xn_a16, (size_t)U))) return rc;
         if ((rc = dalloc(&r.d_xn_b16, (size_t)n->N))) return rc;
@@ -2830,10 +2824,18 @@ int spk_prepare(spk_network* n, int G) {
         if ((rc = dalloc(&r.d_xn_a, (size_t)U))) return rc;
         if ((rc = dalloc(&r.d_xn_b, (size_t)n->N))) return rc;
       }
-      if ((rc = dalloc(&r.d_xcur_a, (size_t)U))) return rc;
-      if ((rc = dalloc(&r.d_xcur_b, (size_t)n->N))) return rc;
-      if ((rc = dalloc(&r.d_act, (size_t)U + n->N))) return rc;
-      if ((rc = dalloc(&r.d_act_cnt, 4))) return rc;
+      if (r.kind == 0) {   // what the per-phase kernels (k_wd_*) read besides
+        if ((rc = dalloc(&r.d_ev_pre_ptr, (size_t)U + 1))) return rc;
+        if ((rc = upload(r.d_ev_pre_ptr, pp.data(), pp.size(), st))) return rc;
+        if (!grouped) {
+          if ((rc = dalloc(&r.d_ev_pre_idx, P))) return rc;
+          if ((rc = upload(r.d_ev_pre_idx, pi.data(), P, st))) return rc;
+        }
+        if ((rc = dalloc(&r.d_xcur_a, (size_t)U))) return rc;
+        if ((rc = dalloc(&r.d_xcur_b, (size_t)n->N))) return rc;
+        if ((rc = dalloc(&r.d_act, (size_t)U + n->N))) return rc;
+        if ((rc = dalloc(&r.d_act_cnt, 4))) return rc;
+      }
       SPK_HIP(hipStreamSynchronize(st));   // the host index arrays end with this scope
     }
     if (r.kind == 4) {
@@ -2947,7 +2949,7 @@ int spk_reset_state(spk_network* n) {
       if (r.d_xn_b) SPK_HIP(hipMemsetAsync(r.d_xn_b, 0, sizeof(float) * N, st));
       if (r.d_xn_a16) SPK_HIP(hipMemsetAsync(r.d_xn_a16, 0, sizeof(uint16_t) * U, st));
       if (r.d_xn_b16) SPK_HIP(hipMemsetAsync(r.d_xn_b16, 0, sizeof(uint16_t) * N, st));
-      SPK_HIP(hipMemsetAsync(r.d_act_cnt, 0, sizeof(int) * 4, st));
+      if (r.d_act_cnt) SPK_HIP(hipMemsetAsync(r.d_act_cnt, 0, sizeof(int) * 4, st));
       r.par = 0;
     }
     r.syn_tr = r.neu_tr = true;

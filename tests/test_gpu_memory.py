@@ -11,6 +11,7 @@ import torch
 
 import oracle_py
 from spike_amd import abi, builders, mlp, sweep
+from spike_amd.netdesc import Rule, RULE_VOGELS
 from sweep_replay import replay_desc
 
 pytestmark = pytest.mark.gpu
@@ -266,3 +267,26 @@ def test_weights_without_memory_for_any_piece():
         with pytest.raises(abi.SpikeError, match="error 4"):
             gpu.weights()
     assert np.array_equal(gpu.weights(), d.weight)
+
+
+def test_delayed_rule_keeps_what_its_kernels_read():
+    """Beside what the per-synapse form has, a Vogels rule that runs by spikes keeps the synapses
+    of each target (8 bytes each), a bit per synapse and arrays of a few bytes per unit."""
+    n = 2000
+    syn = np.arange(n * n, dtype=np.int64)
+
+    def memory(delay_of_one):
+        d = builders.random_net(n_neurons=n, n_inputs=0, p=1.0, seed=1, dmin=4, dmax=4, monitors=())
+        assert d.n_synapses == n * n
+        d.delay[7] = delay_of_one
+        d.rules.append(Rule(RULE_VOGELS, syn, builders.vogels_params(lr=1e-5)))
+        free = torch.cuda.mem_get_info()[0]
+        gpu = abi.Network(d)
+        assert gpu.info().fused == 1
+        used = free - torch.cuda.mem_get_info()[0]
+        gpu.close()
+        return used
+
+    memory(4)
+    by_spikes, per_synapse = memory(4), memory(5)
+    assert 8 * n * n <= by_spikes - per_synapse <= 8 * n * n + n * n // 8 + (6 << 20)
