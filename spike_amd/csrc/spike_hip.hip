@@ -825,7 +825,7 @@ int build_wd_mask(spk_network* n) {
   dfree(n->d_wd_mask);
   if (n->rules.size() != 1 || !n->rules[0].ev_ok || n->rules[0].cnt == 0) return SPK_OK;
   const size_t words = (size_t)(n->S + 31) / 32;
-  if (int rc = dalloc(&n->d_wd_mask, words)) return rc;
+  if (int rc = dalloc(&n->d_wd_mask, words)) return n->rules[0].kind == 0 ? rc : SPK_OK;   // (delayed rules: per synapse)
   SPK_HIP(hipMemsetAsync(n->d_wd_mask, 0, sizeof(uint32_t) * words, n->stream));
   const int64_t P = n->rules[0].cnt;
   const int grid = (int)std::min<int64_t>(16384, (P + 255) / 256);
@@ -2811,31 +2811,43 @@ int spk_prepare(spk_network* n, int G) {
       while (r.src_lo < r.src_hi && pp[r.src_lo + 1] == pp[r.src_lo]) ++r.src_lo;
       r.max_post = 0;
       for (size_t v = 0; v + 1 < qp.size(); ++v) r.max_post = std::max(r.max_post, qp[v + 1] - qp[v]);
-      if ((rc = dalloc(&r.d_ev_post_ptr, (size_t)n->N + 1))) return rc;
-      if ((rc = dalloc(&r.d_ev_post_pos, P))) return rc;
-      if ((rc = dalloc(&r.d_ev_post_pre, P))) return rc;
-      if ((rc = upload(r.d_ev_post_ptr, qp.data(), qp.size(), st))) return rc;
-      if ((rc = upload(r.d_ev_post_pos, qs.data(), P, st))) return rc;
-      if ((rc = upload(r.d_ev_post_pre, qu.data(), P, st))) return rc;
-      if (n->wfmt != SPK_WEIGHTS_FP32) {
-        if ((rc = dalloc(&r.d_xn_a16, (size_t)U))) return rc;
-        if ((rc = dalloc(&r.d_xn_b16, (size_t)n->N))) return rc;
-      } else {
-        if ((rc = dalloc(&r.d_xn_a, (size_t)U))) return rc;
-        if ((rc = dalloc(&r.d_xn_b, (size_t)n->N))) return rc;
-      }
-      if (r.kind == 0) {   // what the per-phase kernels (k_wd_*) read besides
-        if ((rc = dalloc(&r.d_ev_pre_ptr, (size_t)U + 1))) return rc;
-        if ((rc = upload(r.d_ev_pre_ptr, pp.data(), pp.size(), st))) return rc;
-        if (!grouped) {
-          if ((rc = dalloc(&r.d_ev_pre_idx, P))) return rc;
-          if ((rc = upload(r.d_ev_pre_idx, pi.data(), P, st))) return rc;
+      auto event_arrays = [&]() -> int {
+        if (int rc_ = dalloc(&r.d_ev_post_ptr, (size_t)n->N + 1)) return rc_;
+        if (int rc_ = dalloc(&r.d_ev_post_pos, P)) return rc_;
+        if (int rc_ = dalloc(&r.d_ev_post_pre, P)) return rc_;
+        if (int rc_ = upload(r.d_ev_post_ptr, qp.data(), qp.size(), st)) return rc_;
+        if (int rc_ = upload(r.d_ev_post_pos, qs.data(), P, st)) return rc_;
+        if (int rc_ = upload(r.d_ev_post_pre, qu.data(), P, st)) return rc_;
+        if (n->wfmt != SPK_WEIGHTS_FP32) {
+          if (int rc_ = dalloc(&r.d_xn_a16, (size_t)U)) return rc_;
+          if (int rc_ = dalloc(&r.d_xn_b16, (size_t)n->N)) return rc_;
+        } else {
+          if (int rc_ = dalloc(&r.d_xn_a, (size_t)U)) return rc_;
+          if (int rc_ = dalloc(&r.d_xn_b, (size_t)n->N)) return rc_;
         }
-        if ((rc = dalloc(&r.d_xcur_a, (size_t)U))) return rc;
-        if ((rc = dalloc(&r.d_xcur_b, (size_t)n->N))) return rc;
-        if ((rc = dalloc(&r.d_act, (size_t)U + n->N))) return rc;
-        if ((rc = dalloc(&r.d_act_cnt, 4))) return rc;
+        if (r.kind == 0) {   // what the per-phase kernels (k_wd_*) read besides
+          if (int rc_ = dalloc(&r.d_ev_pre_ptr, (size_t)U + 1)) return rc_;
+          if (int rc_ = upload(r.d_ev_pre_ptr, pp.data(), pp.size(), st)) return rc_;
+          if (!grouped) {
+            if (int rc_ = dalloc(&r.d_ev_pre_idx, P)) return rc_;
+            if (int rc_ = upload(r.d_ev_pre_idx, pi.data(), P, st)) return rc_;
+          }
+          if (int rc_ = dalloc(&r.d_xcur_a, (size_t)U)) return rc_;
+          if (int rc_ = dalloc(&r.d_xcur_b, (size_t)n->N)) return rc_;
+          if (int rc_ = dalloc(&r.d_act, (size_t)U + n->N)) return rc_;
+          if (int rc_ = dalloc(&r.d_act_cnt, 4)) return rc_;
+        }
+        return SPK_OK;
+      };
+      rc = event_arrays();
+      if (rc == SPK_ERR_NOMEM && r.kind != 0) {
+        // a delayed rule runs per synapse where there is no memory for its spike-driven form
+        dfree(r.d_ev_post_ptr); dfree(r.d_ev_post_pos); dfree(r.d_ev_post_pre);
+        dfree(r.d_xn_a); dfree(r.d_xn_b); dfree(r.d_xn_a16); dfree(r.d_xn_b16);
+        r.ev_ok = false;
+        rc = SPK_OK;
       }
+      if (rc) return rc;
       SPK_HIP(hipStreamSynchronize(st));   // the host index arrays end with this scope
     }
     if (r.kind == 4) {

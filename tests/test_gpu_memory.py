@@ -290,3 +290,37 @@ def test_delayed_rule_keeps_what_its_kernels_read():
     memory(4)
     by_spikes, per_synapse = memory(4), memory(5)
     assert 8 * n * n <= by_spikes - per_synapse <= 8 * n * n + n * n // 8 + (6 << 20)
+
+
+@pytest.mark.parametrize("fmt", [0, 2])
+def test_delayed_rule_without_memory_for_its_spike_driven_form(fmt):
+    """Whichever request is refused: a network with a delayed rule that can run by spikes is
+    refused for as many as one whose rule cannot (it runs per synapse where its lists are not to
+    be had), and runs as the oracle does when it is not refused."""
+    def net(delay_of_one):
+        d = builders.random_net(n_neurons=60, n_inputs=20, p=0.2, seed=4, dmin=3, dmax=3, input_rate=500.0, whi=3e-3)
+        d.delay[7] = delay_of_one
+        d.rules.append(Rule(RULE_VOGELS, np.arange(d.n_synapses, dtype=np.int64), builders.vogels_params(lr=1e-5)))
+        d.weight_format = fmt
+        return d
+
+    def outcomes(d):
+        ora = oracle_py.OracleNetwork(d, precision=32)
+        ora.run(0.0, 30)
+        needed = forms = 0
+        for served in range(80):
+            with _refused(2, served):
+                try:
+                    gpu = abi.Network(d)
+                except abi.SpikeError as e:
+                    assert "error 4" in str(e)
+                    needed += 1
+                    continue
+            forms |= gpu.run(0.0, 30).kernel_launches
+            assert np.array_equal(gpu.weights().astype(np.float64), ora.weights())
+            assert np.array_equal(gpu.membrane().astype(np.float64), ora.membrane())
+        return needed, forms
+
+    by_spikes, per_synapse = outcomes(net(3)), outcomes(net(4))
+    assert by_spikes[0] == per_synapse[0] > 20
+    assert (by_spikes[1], per_synapse[1]) == (3, 1)   # launches of one run: per synapse 1, by spikes 2
