@@ -131,6 +131,10 @@ const char* spk_last_error(void);
 int spk_abi_version(void);
 /* Number of visible HIP devices; 0 when none. Does not fail. */
 int spk_device_count(void);
+/* Gives the device memory (at most 4 GiB per device) and the streams that the library keeps of
+ * closed networks back, for other users of the device in the process.  The library does so by
+ * itself only when one of its own allocations fails.  Waits for the device. */
+int spk_release_memory(void);
 
 /* ---------------------------------------------------------------------------- */
 /* network lifetime

@@ -126,6 +126,7 @@ SIGNATURES = {
     "spk_last_error": (C.c_char_p, []),
     "spk_abi_version": (C.c_int, []),
     "spk_device_count": (C.c_int, []),
+    "spk_release_memory": (C.c_int, []),
     "spk_create": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.c_float, C.POINTER(P)]),
     "spk_destroy": (C.c_int, [P]),
     "spk_set_stream": (C.c_int, [P, P]),
@@ -243,6 +244,11 @@ def check(rc: int):
     if rc != 0:
         msg = load().spk_last_error().decode(errors="replace")
         raise SpikeError(f"spike_hip error {rc}: {msg}")
+
+
+def release_memory():
+    """Give back the device memory and streams that the library keeps of closed networks."""
+    check(load().spk_release_memory())
 
 
 class Network:

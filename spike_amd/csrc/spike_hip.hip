@@ -251,6 +251,13 @@ void give_stream(int dev, hipStream_t s) {
   (void)hipStreamDestroy(s);
 }
 
+void trim_streams() {
+  std::lock_guard<std::mutex> lock(g_stream_mu);
+  for (auto& d : g_idle_streams)
+    for (hipStream_t s : d.second) (void)hipStreamDestroy(s);
+  g_idle_streams.clear();
+}
+
 // Bernoulli threshold of a Poisson input with rate r: floor((1 - exp(-r*dt)) * 2^32).
 uint32_t bernoulli_threshold(float rate, float dt) {
   double p = -std::expm1(-(double)rate * (double)dt);
@@ -1870,6 +1877,12 @@ hipError_t device_malloc(void** p, size_t bytes) {
 // error message of the calling thread, shared with the surrogate's entry points (mlp.hip)
 void set_last_error(const std::string& msg) { g_error = msg; }
 }  // namespace spk
+
+extern "C" int spk_release_memory(void) {
+  trim_slabs();
+  trim_streams();
+  return SPK_OK;
+}
 
 extern "C" void spk_refuse_allocations(int pass, int count) {
   g_pass = pass;

@@ -324,3 +324,14 @@ def test_delayed_rule_without_memory_for_its_spike_driven_form(fmt):
     by_spikes, per_synapse = outcomes(net(3)), outcomes(net(4))
     assert by_spikes[0] == per_synapse[0] > 20
     assert (by_spikes[1], per_synapse[1]) == (3, 1)   # launches of one run: per synapse 1, by spikes 2
+
+
+def test_memory_of_closed_networks_goes_back_on_request():
+    p = _generated(12000, 5)                     # 1200 synapses of 2 bytes a neuron: 29 MB
+    abi.release_memory()
+    sweep.build(p, 0).close()
+    kept = torch.cuda.mem_get_info()[0]
+    abi.release_memory()
+    assert torch.cuda.mem_get_info()[0] - kept >= 12000 * 1200 * 2
+    abi.release_memory()                         # nothing left
+    _equals_replay(_generated(1300, 6), sweep.build(_generated(1300, 6), 0))
