@@ -23,6 +23,7 @@
 #include "fused.hpp"
 #include "fused_table.hpp"
 #include "gen.hpp"
+#include "launch_split.hpp"
 
 #pragma clang fp contract(off)
 
@@ -1197,7 +1198,7 @@ int launch_group_fast(spk_network* n, float t, bool plastic) {
       if (int rc = launch_rule(n, q, t)) return rc;
   spk::DeliverArgs d{};
   fill_prop_args(n, t, slot, d.p);
-  d.row_waves = (int)std::min<int64_t>(64, std::max<int64_t>(1, (n->max_row + spk::kWave - 1) / spk::kWave));
+  d.row_waves = spk::deliver_row_waves(n->max_row, n->cap, n->G);
   const int db = deliver_blocks(n);
   if (wd) {
     d.wd = u.wd;
