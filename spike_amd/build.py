@@ -9,6 +9,8 @@ import os
 import subprocess
 from concurrent.futures import ThreadPoolExecutor
 
+from . import devcode
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB_DIR = os.path.join(HERE, "_lib")
@@ -52,6 +54,7 @@ def build_hip_library() -> str:
     out = os.path.join(LIB_DIR, "libspike_hip.so")
     tmp = out + ".tmp"
     run([HIPCC, *HIP_FLAGS, "-shared", "-o", tmp, *objs])
+    devcode.check(tmp)
     os.replace(tmp, out)
     return out
 

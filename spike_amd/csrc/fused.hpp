@@ -1554,9 +1554,12 @@ __device__ __forceinline__ void fused_body(const FusedArgs& a, const int p, cons
     unsigned long long* imask = simask + (size_t)dslot * a.iown_max;
     const int b0 = tidx % bits;
     const int slot0 = tidx % BL;
-    // the lane's LDS addresses are computed in every group: hoisted out of the group loop they
-    // would stay live across the delivery, which has no registers to spare (an empty asm, no
-    // instruction; the other kinds' label loops are faster with them kept: 7 %)
+    // the lane's LDS addresses are computed in every group (an empty asm, no instruction): hoisted
+    // out of the group loop they stay live across the delivery, which has no registers to spare,
+    // and the compiler then saved one of them at a join with part of the wavefront still inactive
+    // -- wrong inputs from k_fused<0, true, kRulesOff> for lists of more than seven entries.  The
+    // build checks every kernel for such a copy (devcode.py).  The other kinds' kernels hold
+    // none with the addresses kept, and their label loops are 7 % faster for it.
     int lt = tid;
     if constexpr (KIND == 0) asm volatile("" : "+v"(lt));
     // -- A. Poisson inputs: append this group's spikes, update histories ------------
