@@ -93,7 +93,7 @@ struct EventRule {
 };
 
 struct FusedArgs {
-  EventRule ev;            // kRulesEvents only
+  EventRule ev;            // kRulesEvents and kRulesDelayed
   // partitions: neurons [nlo[p], nlo[p+1]), inputs [ilo[p], ilo[p+1])
   const int* nlo;
   const int* ilo;
@@ -145,13 +145,13 @@ struct FusedArgs {
   const FusedRule* rules;
   int n_rules;
   // exchange blocks [2][P][xstride]: {count, entries (id | g << 24)...}; 32-bit words
-  // behind the grid barrier (plastic launches), 64-bit tagged words otherwise (xlist64, the
+  // behind the grid barrier (kRulesDense), 64-bit tagged words otherwise (xlist64, the
   // same memory): low half the count or entry, high half the tag of the group that wrote it
   uint32_t* xlist;
   unsigned long long* xlist64;
   unsigned int xtag_base;     // tag of group s of this launch: xtag_base + s + 1
   int xquad;                  // tagged delivery by quads per source (small partitions) or staged
-  int early;                  // with xquad and no plasticity: wavefront 0 publishes its list right
+  int early;                  // with xquad and no grid barrier: wavefront 0 publishes its list right
                               // after its LIF, the other wavefronts make the next group's draws
   int dahead;                 // groups whose random draws are made in one pass (LDS slots; 1)
   // two-level grid barrier: counters bar[g * kBarStride] (g < 8), bar[8 * kBarStride]
@@ -174,7 +174,7 @@ struct FusedArgs {
   int64_t group0;             // index of the first group of this launch within the run
   int N, Nin, L, G, B, W, P, xcap, xstride, nown_max, iown_max, ext_k, ngroups;
   int BL;                       // slots of the LDS ring: max(largest delay, G)
-  int plastic;
+  int plastic;                  // how the launch applies the rules: kRules*
   unsigned long long* prof;   // optional: wall-clock ticks per phase of workgroup 0
 };
 
@@ -288,7 +288,7 @@ __device__ __forceinline__ uint32_t load_coherent(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Tagged exchange words (launches without plasticity): every 64-bit word carries the tag of
+// Tagged exchange words (every launch but those of kRulesDense): every 64-bit word carries the tag of
 // the group that wrote it next to its payload, and a reader accepts a word only when the
 // tag is the group's own.  A word is written and read whole (naturally aligned 64-bit
 // accesses at agent scope), so no ordering between the words of a block is needed and the

@@ -143,9 +143,9 @@ __device__ __forceinline__ void store_fl(const uint16_t* lds, int C, uint16_t* d
   }
 }
 
-// Transposed tile product: acc[nb][mb] += W[32 w + 16 nb.., k] . lds[16 mb.., k] over KS steps
+// Transposed tile product: acc[nb][mb] += W[CW w + 16 nb.., k] . lds[16 mb.., k] over KS steps
 // of 32 (K = 32 KS), i.e. Z^T = W A^T.  Result element r of acc[nb][mb] belongs to batch
-// row m = 16 mb + lane % 16 and output n = 32 w + 16 nb + 4 (lane / 16) + r: every lane
+// row m = 16 mb + lane % 16 and output n = CW w + 16 nb + 4 (lane / 16) + r: every lane
 // holds four consecutive outputs of one row, which it writes back as one 8-byte LDS store.
 // `wf` holds the weight fragments of the first step (load_w, issued before the previous
 // layer's epilogue); those of step ks + 1, and the activations of the next half step, are in
@@ -797,16 +797,18 @@ int lds_attributes() {
 }
 
 // Inference: pieces have at least one round of the chip of 128-row tiles (8 members x 262147
-// rows, 25 MB of results to pageable memory: 2.51 ms in one piece, 2.05 in 2, 1.90 in 4, 1.78 in
-// 8; the kernels alone 0.94 and 1.03 ms); k_mlp_forward_small takes at most one 16-row tile per
+// rows, 25 MB of results to pageable memory, the same rows and results array in every call: 2.51
+// ms in one piece, 2.05 in 2, 1.90 in 4, 1.78 in 8; the kernels alone 0.94 and 1.03 ms); k_mlp_forward_small takes at most one 16-row tile per
 // CU (8 members x 500 rows 10.3 us, in 64-row tiles 13.3; x 1000 rows, two rounds, 17.6 and
 // 14.8; x 100 rows 10.8, 14.3).
 constexpr int64_t kPieceTiles = 512, kSmallTiles = 256;
 
 // Row tile of the passes over `rows` rows of `models` members: half tiles while whole ones give
-// at most one workgroup per CU.  At 256 whole tiles (8 members x 4096 rows) inference takes 26
-// us in whole and 22 in half tiles, a training step's two passes 54 + 43 and 49 + 37 us; at 512
-// tiles 37 and 37, 80 + 65 and 97 + 84 us (half tiles read the weights twice).
+// at most one workgroup for each of the 256 CUs of the MI355X.  A training step's two passes take,
+// in whole and in half tiles, 71 and 55 us at 128 whole tiles, 85 and 80 at 256, 98 and 99 at 288,
+// 115 and 112 at 320, 126 and 131 at 384, 144 and 174 at 512 (half tiles read the weights twice).
+// Inference follows the same line: 26 and 22 us at 256 tiles; it would gain beyond it, too (35 and
+// 27 at 288, 38 and 35 at 512, 53 and 48 at 768).
 bool half_tiles(int64_t rows, int models) { return (rows + MT - 1) / MT * models <= 256; }
 
 template <bool TRAIN>
