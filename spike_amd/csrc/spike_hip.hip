@@ -464,8 +464,8 @@ struct spk_network {
   uint32_t* d_wc = nullptr;   // per synapse: 16-bit weight | compensation << 16
   float cw_lo = 0.0f, cw_hi = 0.0f;
   int csplit = 0, cnhi = 0, cdelay = 0;
-  // buffers of spk_get_weights / spk_set_weights, made by the first of them: caller weights on
-  // their way in or out, wstage_n at a time; the CSR position of each caller synapse (none for
+  // buffers of spk_get_weights / spk_set_weights (weight_positions, weight_staging): caller weights
+  // on their way in or out, wstage_n at a time; the CSR position of each caller synapse (none for
   // generated synapses: the same order; 64-bit from 2^32 synapses on) or, where there is no memory
   // for all of them, of the piece's synapses
   float* d_wstage = nullptr;
@@ -1251,37 +1251,41 @@ int launch_group_phases(spk_network* n, float t, bool plastic) {
   return SPK_OK;
 }
 
-// The buffers of spk_get_weights / spk_set_weights: 64 MB at most beside the positions (4 bytes
-// a synapse; uploaded once, as reading them again in every call would cost as much as the
-// weights).  Where memory is short the pieces get smaller, down to 16 KB, and the positions
-// travel with them.
+// The CSR positions of the caller's synapses on the device (4 bytes each), for spk_get_weights and
+// spk_set_weights: made once, as reading them again in every call would cost as much as the
+// weights.  None where there is no memory for them.
+int weight_positions(spk_network* n) {
+  const int64_t S = n->S;
+  if (n->od || n->d_pos || n->d_pos64 || S == 0) return SPK_OK;
+  hvec<uint32_t> pos;
+  int rc = SPK_OK;
+  if (S >= ((int64_t)1 << 32)) {
+    if (dalloc(&n->d_pos64, (size_t)S)) return SPK_OK;
+    rc = upload(n->d_pos64, n->perm.data(), (size_t)S, n->stream);
+  } else {
+    if (dalloc(&n->d_pos, (size_t)S)) return SPK_OK;
+    pos.resize(S);
+    host_chunks(S, host_threads(), [&](int, int64_t a, int64_t b) {
+      for (int64_t k = a; k < b; ++k) pos[k] = (uint32_t)n->perm[k];
+    });
+    rc = upload(n->d_pos, pos.data(), (size_t)S, n->stream);
+  }
+  const hipError_t e = hipStreamSynchronize(n->stream);   // (the host array ends here)
+  if (rc == SPK_OK && e == hipSuccess) return SPK_OK;
+  dfree(n->d_pos);
+  dfree(n->d_pos64);
+  return rc ? rc : fail(SPK_ERR_HIP, std::string("uploading synapse positions: ") + hipGetErrorString(e));
+}
+
+// Their staging buffer, 64 MB at most.  Where memory is short the pieces get smaller, down to
+// 16 KB, and without the positions above a piece carries its own.
 constexpr int64_t kWeightPiece = (int64_t)1 << 24, kWeightPieceMin = 4096;
 int weight_staging(spk_network* n) {
   if (n->d_wstage) return SPK_OK;
-  int rc = SPK_OK;
-  if (!n->od && !n->d_pos && !n->d_pos64) {
-    const int64_t S = n->S;
-    if (S >= ((int64_t)1 << 32)) {
-      if (dalloc(&n->d_pos64, (size_t)S) == SPK_OK && (rc = upload(n->d_pos64, n->perm.data(), (size_t)S, n->stream))) {
-        dfree(n->d_pos64);
-        return rc;
-      }
-    } else if (dalloc(&n->d_pos, (size_t)S) == SPK_OK) {
-      hvec<uint32_t> pos(S);
-      host_chunks(S, host_threads(), [&](int, int64_t a, int64_t b) {
-        for (int64_t k = a; k < b; ++k) pos[k] = (uint32_t)n->perm[k];
-      });
-      rc = upload(n->d_pos, pos.data(), (size_t)S, n->stream);
-      const hipError_t e = hipStreamSynchronize(n->stream);   // (the host array ends here)
-      if (rc || e != hipSuccess) {
-        dfree(n->d_pos);
-        return rc ? rc : fail(SPK_ERR_HIP, std::string("uploading synapse positions: ") + hipGetErrorString(e));
-      }
-    }
-  }
+  if (int rc = weight_positions(n)) return rc;
   const bool piece_pos = !n->od && !n->d_pos && !n->d_pos64;
   for (int64_t cnt = std::min<int64_t>(n->S, kWeightPiece);; cnt = (cnt + 3) / 4) {
-    rc = dalloc(&n->d_wstage, (size_t)cnt);
+    int rc = dalloc(&n->d_wstage, (size_t)cnt);
     if (!rc && piece_pos && (rc = dalloc(&n->d_piece_pos, (size_t)cnt))) dfree(n->d_wstage);
     n->wstage_n = cnt;
     if (!rc || cnt <= kWeightPieceMin) return rc;
@@ -2910,6 +2914,9 @@ int spk_prepare(spk_network* n, int G) {
   if (n->rules.size() == 1)
     for (size_t j = 0; j < n->rules[0].syn.size() && !input_sources; ++j) input_sources = n->h_pre[n->rules[0].syn[j]] < 0;
   if ((rc = plan_event_rule(n, input_sources))) return rc;
+  // networks that learn: their weights are read after a trial, the first one, too (3.1e6 synapses:
+  // 1 ms of it); others make the positions when their weights are first asked for
+  if (!n->rules.empty() && (rc = weight_positions(n))) return rc;
   n->prepared = true;
   return spk_reset_state(n);
 }
