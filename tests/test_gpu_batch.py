@@ -227,3 +227,33 @@ def test_full_sweep_at_configured_size():
     for j, k in enumerate(idx):
         print(f"point {k} N={pts[k].n}: FP32 {r32[j].mean():.3f} Hz FP64 {m64[j]:.3f} Hz err {100 * err[j]:.2f} %")
     assert err.max() <= 0.02
+
+
+def test_batch_right_after_unwaited_resets_on_the_callers_streams():
+    """spk_reset_state only enqueues; a batch, which runs on a stream of its own, starts after the
+    resets, also where they were enqueued behind other work of the caller's streams."""
+    import torch
+    pts = small_points(4, seed=5)
+    nets = [sweep.build(p, 0) for p in pts]
+    streams = [torch.cuda.Stream() for _ in nets]
+    for n, s in zip(nets, streams):
+        abi.check(n.lib.spk_set_stream(n.h, s.cuda_stream))
+    batch = abi.Batch(nets)
+    groups = [40] * len(nets)
+    a = torch.rand(4096, 4096, device="cuda")
+    torch.cuda.synchronize()
+    first = None
+    for k in range(3):
+        for n, s in zip(nets, streams):
+            with torch.cuda.stream(s):
+                for _ in range(4 if k else 0):
+                    a @ a                        # the reset waits for these
+            n.reset_state()
+        batch.run(np.zeros(len(nets)), groups)
+        got = [(n.membrane(), n.ring(), n.last_spike(0)) for n in nets]
+        first = first or got
+        for x, y in zip(first, got):
+            assert all(np.array_equal(p, q) for p, q in zip(x, y))
+    batch.close()
+    for n in nets:
+        n.close()
