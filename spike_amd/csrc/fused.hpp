@@ -70,7 +70,7 @@ enum { kRulesOff = 0, kRulesDense = 1, kRulesEvents = 2, kRulesDelayed = 3 };
 // workgroup reads another's state and no grid barrier is needed.  A weight moves only when its
 // source or its target has a spike in the group; it is touched only by the workgroup that owns
 // its target.  Bound by the exchange's latency: weight-dependent rule, 6000 neurons x 500
-// synapses (3.1e6, delays from one step) 5.1 us per group; per synapse, with the barrier's cache
+// synapses (3.1e6, delays from one step) 6.1 us per group; per synapse, with the barrier's cache
 // write-backs, 51 us.
 //   kRulesEvents   the weight-dependent rule (the per-phase form of kernels.hpp, k_wd_neurons
 //                  and k_wd_events): this group's spikes of the sources, after the exchange;

@@ -797,10 +797,12 @@ int lds_attributes() {
 }
 
 // Inference: pieces have at least one round of the chip of 128-row tiles (8 members x 262147
-// rows, 25 MB of results to pageable memory, the same rows and results array in every call: 2.51
-// ms in one piece, 2.05 in 2, 1.90 in 4, 1.78 in 8; the kernels alone 0.94 and 1.03 ms); k_mlp_forward_small takes at most one 16-row tile per
-// CU (8 members x 500 rows 10.3 us, in 64-row tiles 13.3; x 1000 rows, two rounds, 17.6 and
-// 14.8; x 100 rows 10.8, 14.3).
+// rows, 25 MB of results to pageable memory, one handle called in a loop: 2.51 ms in one piece,
+// 2.05 in 2, 1.90 in 4, 1.78 in 8; the kernels alone 0.94 and 1.03 ms.  The copy's time hangs on
+// the caller's pages: 1.75 to 1.9 ms in such loops, 2.5 to 2.6 where calls of several handles with
+// other rows take turns); k_mlp_forward_small takes at most one 16-row tile per CU (8 members x
+// 500 rows 10.3 us, in 64-row tiles 13.3; x 1000 rows, two rounds, 17.6 and 14.8; x 100 rows 10.8,
+// 14.3).
 constexpr int64_t kPieceTiles = 512, kSmallTiles = 256;
 
 // Row tile of the passes over `rows` rows of `models` members: half tiles while whole ones give

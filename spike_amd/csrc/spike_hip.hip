@@ -1566,7 +1566,7 @@ int event_mode(const spk_network* n) { return n->rules[0].kind == 0 ? spk::kRule
 // weight-dependent rule also every unit of the rule spiking at most once per group (a source's
 // row is then walked, and its trace raised, once).  Otherwise the rules run per synapse behind
 // the grid barrier.  Weight-dependent rule, 6000 neurons with 500 synapses each, delays from one
-// step: 51 us per group per synapse, 5.1 us by spikes.  The spike-driven form has no size from
+// step: 51 us per group per synapse, 6.1 us by spikes.  The spike-driven form has no size from
 // which it is slower: its cost per group is one pass over the sources, that of the other one
 // pass over the rule's synapses, and a source has at least one.
 int plan_event_rule(spk_network* n, bool input_sources) {
