@@ -1313,8 +1313,11 @@ int launch_weights(spk_network* n, int64_t s0, int64_t cnt, bool out) {
 }
 
 // Records from which the device orders a drained monitor: below, sorting them on the host costs
-// no more than the launches and fills do (about 30 ns a record against 60 us).
-constexpr int64_t kRasterMin = 2048;
+// no more than the launches, fills and the third copy do.  A drain of 300 units' records takes, on
+// the device and on the host, 152 and 106 us at 1760 records, 191 and 157 at 5300, 207 and 187 at
+// 7040, 224 and 248 at 10700; of 5000 units' 152 and 126 at 1870, 190 and 197 at 4800, 211 and 252
+// at 7870; of 10000 units' over 300 steps 202 and 208 at 5900.
+constexpr int64_t kRasterMin = 6144;
 constexpr int64_t kRasterMaxWords = (int64_t)1 << 24;   // 64 MB of bits
 // Steps below which a record's step and its time determine each other: the float time of step
 // k is within 2^-22 k steps of k.

@@ -207,14 +207,14 @@ def test_raster_without_memory_to_order_it_on_the_device(served):
     d, gpu, ora = _monitored()
 
     def steps(t):
-        for s in range(150):
+        for s in range(300):
             gpu.step_group(d.group_time(t, s))
-        ora.run(t, 150)
+        ora.run(t, 300)
 
     steps(0.0)
     with _refused(100, served):
         _same_rasters(gpu, ora)
-    steps(float(d.group_time(0.0, 150)))
+    steps(float(d.group_time(0.0, 300)))
     _same_rasters(gpu, ora)
 
 

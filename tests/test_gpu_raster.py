@@ -80,3 +80,22 @@ def test_times_past_the_steps_they_name():
     ora.run(start, 100)
     oi, ot = ora.take_spikes(0)
     assert np.array_equal(gi, oi) and np.array_equal(gt, ot)
+
+
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_store_around_the_line_between_host_and_device(extra):
+    """Exactly 6144 + extra records of 192 inputs that fire at every step but the first."""
+    n = 192
+    steps = 33    # 32 firing steps x 192 inputs = 6144
+    d = _net(n, 1e9)
+    d.rates = np.full((1, n), np.float32(1e9), np.float32)
+    if extra < 0:
+        d.rates[0, 5] = 0.0
+    gpu = abi.Network(d)
+    ora = oracle_py.OracleNetwork(d, precision=32)
+    gpu.run(0.0, steps + (extra > 0))
+    ora.run(0.0, steps + (extra > 0))
+    gi, gt = gpu.take_spikes(0)
+    oi, ot = ora.take_spikes(0)
+    assert len(gi) == {-1: 6144 - 32, 0: 6144, 1: 6144 + 192}[extra]
+    assert np.array_equal(gi, oi) and np.array_equal(gt, ot)
