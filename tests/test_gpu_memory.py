@@ -261,7 +261,8 @@ def test_weights_of_generated_synapses_in_pieces(fmt, refused):
 
 
 def test_weights_without_memory_for_any_piece():
-    d = builders.random_net(seed=2)
+    d = builders.random_net(n_neurons=200, n_inputs=80, p=0.7, seed=2)
+    assert d.n_synapses > 20480
     gpu = abi.Network(d)
     with _refused(1000):
         with pytest.raises(abi.SpikeError, match="error 4"):
@@ -335,3 +336,18 @@ def test_memory_of_closed_networks_goes_back_on_request():
     assert torch.cuda.mem_get_info()[0] - kept >= 12000 * 1200 * 2
     abi.release_memory()                         # nothing left
     _equals_replay(_generated(1300, 6), sweep.build(_generated(1300, 6), 0))
+
+
+@pytest.mark.parametrize("fmt", [0, 1, 2])
+@pytest.mark.parametrize("synapses", [1, 20479, 20480, 20481])
+def test_weights_around_the_line_between_host_and_device(synapses, fmt):
+    d = builders.random_net(n_neurons=200, n_inputs=80, p=0.7, seed=3, whi=1.0, monitors=())
+    o = np.random.default_rng(5).permutation(d.n_synapses)[:synapses]
+    d.pre, d.post, d.weight, d.delay = d.pre[o], d.post[o], d.weight[o], d.delay[o]
+    d.weight_format = fmt
+    d.grouping = 1
+    gpu = abi.Network(d)
+    with _refused(1000 if synapses <= 20480 else 0):
+        w = gpu.weights()
+    assert np.array_equal(w, d.weight) if fmt == 0 else np.abs(w - d.weight).max() <= 0.004
+    _weights_name_synapses(gpu, synapses, fmt)
